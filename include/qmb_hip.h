@@ -248,7 +248,10 @@ int qmb_apply_prepared(const qmb_terms* terms, const qmb_targets* targets, const
  * by the qmb_targets the cores were built from, rows distinct). */
 
 /* Merged coefficients of the pair-excitation terms, dense over (annihilated pair, created pair):
- * coef[pair_slot(r0,r1) * n_pairs + pair_slot(c0,c1)] = sum over terms of (-1)^delta_t coef_t.
+ * coef[pair_slot(r0,r1) * n_pairs + pair_slot(c0,c1)] = sum over terms of (-1)^(delta_t + o) coef_t, with
+ * o = 1 + the sites of {r0, r1} in [c0, c1): the part of the parity the term's own sites decide (0 for
+ * hard-core bosons), so the element on a source config with core C = c minus {r0, r1} is
+ * (-1)^popcount(C & ([r0, r1) ^ [c0, c1))) times the coefficient.
  * pair_slot numbers the pairs (a<b) of the n_bits = 8*n_qubytes sites in three blocks by site
  * parity: even-even pairs (index (b/2)((b/2)-1)/2 + a/2), then odd-odd, then even-odd
  * (2 C(n_bits/2, 2) + (even site / 2) (n_bits / 2) + odd site / 2).  n_qubytes <= 16.
@@ -274,8 +277,9 @@ int qmb_pairs_build(int n_qubytes, int particle_cut, const int16_t* site, const 
 
 /* Merged coefficients of the single excitations (annihilate r, create p, conditioned on at most
  * one other site k): the element on a source config c holding r and not p is
- *   (-1)^(popcount(c & (L(r) ^ L(p)))) * (a[r * n_bits + p] + sum_{k in c, k != r} kd[(r * n_bits + p) * n_bits + k])
- * with L(s) = the sites below s.  n_qubytes <= 16. */
+ *   (-1)^(popcount(C & (L(r) ^ L(p)))) * (a[r * n_bits + p] + sum_{k in C} kd[(r * n_bits + p) * n_bits + k])
+ * with C = c without r and L(s) = the sites below s (r itself is counted in the tables' sign when
+ * r < p, except for hard-core bosons).  n_qubytes <= 16. */
 typedef struct qmb_singles {
     int32_t n_qubytes, particle_cut, n_bits;
     int32_t real;      /* 1: the kernels read a_re / kd_re (set by qmb_singles_set_real) */
@@ -312,9 +316,8 @@ int qmb_terms_build_residual(int n_qubytes, int particle_cut, const int16_t* sit
  * (cores of single excitations) -- radix-sorted by a 32-bit key of the core (its class, order 2:
  * even sites of the core mod 3, order 1: 0, and a hash of it), stable within a group of equal keys;
  * and the start of every group.  Different cores with equal keys share a group: the build compares
- * the cores of neighbouring entries exactly and flags such a mixed group in bit 31 of its start,
- * and the apply calls compare cores per pair only there (elsewhere every row of a group has the
- * first entry's core).  capacity must be below 2^31.  max_occupied must bound the number of
+ * the cores of neighbouring entries exactly, flags such a mixed group in bit 31 of its start, and
+ * splits it by core for the apply calls.  capacity must be below 2^31.  max_occupied must bound the number of
  * occupied sites of every config (a row with more sets counts[2], and the apply calls then write
  * NaN into out[0] instead of a wrong result). */
 typedef struct qmb_cores {
@@ -330,6 +333,13 @@ typedef struct qmb_cores {
     uint64_t* vals;    /* [capacity] row << 16 | site1 << 8 | site0 of the removed sites (order 1: site0) */
     uint32_t* starts;  /* [capacity + 1] first entry of each group (bit 31: the group is mixed), then the end */
     int64_t* counts;   /* device: {entries, groups, overflow, 0} */
+    /* What the apply calls walk: the groups of two or more entries in bins by size. */
+    uint64_t* mvals;   /* their entries bin by bin: row | slot << 32 | sign << 63 (slot: pair_slot of the removed
+                          pair, order 1 the removed site; sign: parity of the core's sites in [site0, site1),
+                          order 1 below site0) */
+    uint64_t* glist;   /* groups of more than 32 entries and the groups of the mixed groups' cores, as two u32
+                          each: first entry in mvals, size (0: an unused slot) */
+    void* bins;        /* device table of the bins */
 } qmb_cores;
 
 int qmb_cores_workspace_size(int n_qubytes, int64_t n, int32_t max_occupied, int32_t order, size_t* bytes);
@@ -416,7 +426,7 @@ int qmb_apply_structured_dual(const qmb_pairs* pairs, const qmb_singles* singles
 /* ---------------- batched persistent launch (no reference counterpart) -------------------------
  * Many instances -- a term table and a config set each, of any sizes -- applied by two persistent
  * kernel launches for all of them: the diagonal, single- and pair-excitation work of every instance
- * is cut into units of 64 core groups or 64 rows; the first launch's waves take the pair units of
+ * is cut into units of a few passes over core groups of one size, or 64 rows; the first launch's waves take the pair units of
  * all instances round-robin, the second's the single and diagonal units.  For many small instances
  * this replaces a few kernels per instance by two launches that fill the GPU; both are capturable
  * in a hipGraph (no allocation, no sync).

@@ -5,8 +5,9 @@
 // of generating every (config, term) target and probing the index for it -- the reference's
 // scheme, qmb/_hamiltonian_cuda.cu:86-135, which for a molecular Hamiltonian spends ~90% of its
 // work on double-excitation targets that are not in the set -- every config emits one entry per
-// occupied pair (its cores), the entries are radix-sorted by core hash, and a wave walks each group
-// of equal cores, combining its rows pairwise with the merged coefficient table of qmb_pairs.
+// occupied pair (its cores), the entries are radix-sorted by core hash and dealt into bins by the size
+// of their group, and a wave walks the groups of equal cores, combining their rows pairwise with the
+// merged coefficient table of qmb_pairs.
 // Only connections whose target is in the set are visited; each output row sums in registers and
 // reaches HBM with one FP64 atomic per group it belongs to.
 #include <rocprim/device/device_radix_sort.hpp>
@@ -136,6 +137,15 @@ __device__ __forceinline__ void wave_count(int64_t* counter, bool add) {
     }
 }
 
+// The part of pair_parity that the excitation's own sites decide.  The source config is the core
+// with {r0, r1}, so popcount(c & ([r0, r1) ^ [c0, c1))) = popcount(core & [r0, r1)) + popcount(core &
+// [c0, c1)) + 1 (r0 in its own range) + the sites of {r0, r1} in [c0, c1).  The last two go into the
+// table; the first two are one sign per (core, pair), the entry's own, so the group kernels multiply
+// two entry signs in and compute no parity per pair.
+__device__ __forceinline__ int pair_own_parity(int r0, int r1, int c0, int c1) {
+    return 1 ^ static_cast<int>(r0 >= c0 && r0 < c1) ^ static_cast<int>(r1 >= c0 && r1 < c1);
+}
+
 // Launched with whole waves: threads past n_terms take part in the counts only.
 __global__ void pairs_fill_kernel(const int16_t* __restrict__ site, const uint8_t* __restrict__ kind,
                                   const double2* __restrict__ coef, int64_t n_terms, int particle_cut, int n_bits,
@@ -152,8 +162,9 @@ __global__ void pairs_fill_kernel(const int16_t* __restrict__ site, const uint8_
         } else if (c.status == kCompileOk && pair_excitation(c.rec, particle_cut, &e)) {
             const double2 v = coef[t];
             double2* dst = table + pair_slot(e.r0, e.r1, n_bits) * n_pairs + pair_slot(e.c0, e.c1, n_bits);
-            unsafeAtomicAdd(&dst->x, e.delta ? -v.x : v.x);
-            unsafeAtomicAdd(&dst->y, e.delta ? -v.y : v.y);
+            const int flip = e.delta ^ (particle_cut == 1 ? pair_own_parity(e.r0, e.r1, e.c0, e.c1) : 0);
+            unsafeAtomicAdd(&dst->x, flip ? -v.x : v.x);
+            unsafeAtomicAdd(&dst->y, flip ? -v.y : v.y);
             is_pair = true;
         }
     }
@@ -207,6 +218,34 @@ __device__ __forceinline__ Cfg<W> load_key(const uint64_t* __restrict__ keys, in
     return c;
 }
 
+// Sites in [a, b), a <= b: L(a) ^ L(b) with L(s) the sites below s.
+template <int W>
+__device__ __forceinline__ Cfg<W> range_mask(int a, int b) {
+    Cfg<W> m;
+    if (W == 1) {
+        m.w[0] = (1ull << b) - (1ull << a);  // sites of a one-word config are < 64
+    } else {
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const int lo = a - 64 * w, hi = b - 64 * w;
+            const uint64_t mh = hi <= 0 ? 0ull : (hi >= 64 ? ~0ull : (1ull << hi) - 1ull);
+            const uint64_t ml = lo <= 0 ? 0ull : (lo >= 64 ? ~0ull : (1ull << lo) - 1ull);
+            m.w[w] = mh & ~ml;
+        }
+    }
+    return m;
+}
+
+template <int W>
+__device__ __forceinline__ int masked_parity(const Cfg<W>& c, const Cfg<W>& m) {
+    int par = 0;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        par ^= __popcll(c.w[w] & m.w[w]);
+    }
+    return par & 1;
+}
+
 template <int W>
 __device__ __forceinline__ void flip_site(Cfg<W>& c, int s) {
 #pragma unroll
@@ -236,38 +275,15 @@ __device__ __forceinline__ uint32_t core_key(uint64_t h, uint32_t cls) {
 // among its row's pairs grows with its slot (ties where no core site lies between two slots), and
 // the stable sort leaves each group's entries close to ascending slots: the lanes of a wave then
 // read nearby columns of a coefficient table row.
-template <int W, int ORDER, bool PACKED>
-__global__ void core_emit_kernel(const uint64_t* __restrict__ keys, const uint64_t* __restrict__ cols, int64_t n, int n_bits,
-                                 int per_config, int sub_bits, uint32_t* __restrict__ okeys, void* __restrict__ ovals,
-                                 int64_t* __restrict__ counts) {
-    const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (i >= n) {
-        return;
-    }
+template <int W, int ORDER, typename Emit>
+__device__ __forceinline__ void emit_cores(const Cfg<W>& c, const uint64_t* __restrict__ cols, Emit&& emit) {
     constexpr uint64_t kEven = 0x5555555555555555ull;
-    const Cfg<W> c = load_key<W>(keys, i);
     const uint64_t h = hash_cfg<W>(c, cols);
     int even = 0;
 #pragma unroll
     for (int w = 0; w < W; ++w) {
         even += __popcll(c.w[w] & kEven);
     }
-    int64_t k = 0;
-    // the value: row << 16 | y << 8 | x, or packed into 32 bits as row << sub_bits | (pair slot of
-    // (x, y), or the site x); the packed value halves what the sort moves per value
-    auto emit = [&](uint64_t key, uint64_t val) {
-        if (k < per_config) {
-            if (PACKED) {
-                const uint32_t sub = ORDER == 2 ? static_cast<uint32_t>(pair_slot(static_cast<int>(val & 0xff), static_cast<int>(val >> 8), n_bits))
-                                                : static_cast<uint32_t>(val);
-                static_cast<uint64_t*>(ovals)[k * n + i] = (key << kPackedBits) | ((static_cast<uint32_t>(i) << sub_bits) | sub);
-            } else {
-                okeys[k * n + i] = static_cast<uint32_t>(key);
-                static_cast<uint64_t*>(ovals)[k * n + i] = (static_cast<uint64_t>(i) << 16) | val;
-            }
-        }
-        ++k;
-    };
     if (ORDER == 1) {
 #pragma unroll
         for (int wx = 0; wx < W; ++wx) {
@@ -275,7 +291,7 @@ __global__ void core_emit_kernel(const uint64_t* __restrict__ keys, const uint64
             while (mx) {
                 const int x = 64 * wx + __builtin_ctzll(mx);
                 mx &= mx - 1;
-                emit(core_key(h ^ cols[x], 0u), static_cast<uint64_t>(x));
+                emit(core_key(h ^ cols[x], 0u), static_cast<uint32_t>(x));
             }
         }
     } else {
@@ -299,7 +315,7 @@ __global__ void core_emit_kernel(const uint64_t* __restrict__ keys, const uint64
                         while (mx) {
                             const int x = 64 * wx + __builtin_ctzll(mx);
                             mx &= mx - 1;
-                            emit(core_key(hy ^ cols[x], cls), (static_cast<uint64_t>(y) << 8) | static_cast<uint64_t>(x));
+                            emit(core_key(hy ^ cols[x], cls), (static_cast<uint32_t>(y) << 8) | static_cast<uint32_t>(x));
                         }
                     }
                 }
@@ -322,12 +338,38 @@ __global__ void core_emit_kernel(const uint64_t* __restrict__ keys, const uint64
                         mo &= mo - 1;
                         const int x = ev < od ? ev : od;
                         const int y = ev < od ? od : ev;
-                        emit(core_key(he ^ cols[od], cls), (static_cast<uint64_t>(y) << 8) | static_cast<uint64_t>(x));
+                        emit(core_key(he ^ cols[od], cls), (static_cast<uint32_t>(y) << 8) | static_cast<uint32_t>(x));
                     }
                 }
             }
         }
     }
+}
+
+template <int W, int ORDER, bool PACKED>
+__global__ void core_emit_kernel(const uint64_t* __restrict__ keys, const uint64_t* __restrict__ cols, int64_t n, int n_bits,
+                                 int per_config, int sub_bits, uint32_t* __restrict__ okeys, void* __restrict__ ovals,
+                                 int64_t* __restrict__ counts) {
+    const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+    if (i >= n) {
+        return;
+    }
+    int64_t k = 0;
+    // the value: row << 16 | y << 8 | x, or packed into 32 bits as row << sub_bits | (pair slot of
+    // (x, y), or the site x); the packed value halves what the sort moves per value
+    emit_cores<W, ORDER>(load_key<W>(keys, i), cols, [&](uint32_t key, uint32_t sites) {
+        if (k < per_config) {
+            if (PACKED) {
+                const uint32_t sub =
+                    ORDER == 2 ? static_cast<uint32_t>(pair_slot(static_cast<int>(sites & 0xff), static_cast<int>(sites >> 8), n_bits)) : sites;
+                static_cast<uint64_t*>(ovals)[k * n + i] = (static_cast<uint64_t>(key) << kPackedBits) | ((static_cast<uint32_t>(i) << sub_bits) | sub);
+            } else {
+                okeys[k * n + i] = key;
+                static_cast<uint64_t*>(ovals)[k * n + i] = (static_cast<uint64_t>(i) << 16) | sites;
+            }
+        }
+        ++k;
+    });
     if (k > per_config) {
         atomicAdd(reinterpret_cast<unsigned long long*>(&counts[2]), 1ull);
     }
@@ -341,10 +383,14 @@ __global__ void core_emit_kernel(const uint64_t* __restrict__ keys, const uint64
     }
 }
 
-// inv[pair_slot(x, y)] = y << 8 | x for every pair x < y of n_bits sites.
-__global__ void pair_inverse_kernel(int n_bits, uint32_t* __restrict__ inv) {
+// Start of a build: counts = 0, and (inv non-null) inv[pair_slot(x, y)] = y << 8 | x for every pair
+// x < y of n_bits sites.
+__global__ void cores_init_kernel(int64_t* __restrict__ counts, int n_bits, uint32_t* __restrict__ inv) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n_bits * n_bits) {
+    if (t < 4) {
+        counts[t] = 0;
+    }
+    if (inv == nullptr || t >= n_bits * n_bits) {
         return;
     }
     const int x = t % n_bits, y = t / n_bits;
@@ -355,11 +401,14 @@ __global__ void pair_inverse_kernel(int n_bits, uint32_t* __restrict__ inv) {
 
 // Flags of a used sorted core entry: the first entry of its key (a group head, bit 0) and an entry
 // whose core differs from the previous entry's under the same key (two cores merged by equal keys,
-// bit 31).  Unused slots (the sentinel keys, sorted last) get 0; the flag pass writes the number of
+// kFlagBreak); entries of groups of two or more also carry their sign (kFlagSign): the parity of the
+// core's sites in [x, y) (order 2) or below x (order 1), one factor of every element the entry takes
+// part in.  One byte per entry.  Unused slots (the sentinel keys, sorted last) get 0; the flag pass writes the number of
 // used entries to counts[0] and each wave's number of heads to its chunk's counter; a head's group
 // is the heads before its chunk (an exclusive scan of the counters) plus those before it in the chunk.
 constexpr uint32_t kFlagHead = 1u;
-constexpr uint32_t kFlagBreak = 0x80000000u;
+constexpr uint32_t kFlagSign = 2u;
+constexpr uint32_t kFlagBreak = 4u;
 // Bit 31 of starts[g] (g < G): group g holds more than one core (its rows' cores are compared exactly).
 constexpr uint32_t kGroupMixed = 0x80000000u;
 constexpr uint32_t kGroupStart = 0x7FFFFFFFu;
@@ -455,10 +504,64 @@ __device__ __forceinline__ void core_flags(const uint64_t* __restrict__ ckeys, i
         const bool used = k[t] != kKeySentinel;
         const bool head = used && kp[t] != k[t];
         f[t] = !used ? 0u : (head ? kFlagHead : (same ? 0u : kFlagBreak));
+        // the core is empty (parity 0) for an entry alone in its group
+        const int lo = ORDER == 2 ? static_cast<int>(v[t] & 0xff) : 0;
+        const int hi = static_cast<int>((ORDER == 2 ? v[t] >> 8 : v[t]) & 0xff);
+        f[t] |= used && masked_parity<W>(core[t], range_mask<W>(lo, hi)) != 0 ? kFlagSign : 0u;
         if (used && kn[t] == kKeySentinel) {
             counts[0] = base + 64 * t + lane + 1;  // the last used entry
         }
     }
+}
+
+// out = exclusive sums of in[0, n), by the calling block of kBlock threads.
+__device__ __forceinline__ void block_scan(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, int64_t n) {
+    __shared__ uint32_t s_wave[kBlock / 64];
+    constexpr int V = 16;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t carry = 0;
+    for (int64_t base = 0; base < n; base += kBlock * V) {
+        const int64_t at = base + V * static_cast<int64_t>(threadIdx.x);
+        uint32_t v[V], sum = 0;
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            v[k] = at + k < n ? in[at + k] : 0u;
+            sum += v[k];
+        }
+        uint32_t incl = sum;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t o = __shfl_up(incl, d);
+            incl += lane >= d ? o : 0u;
+        }
+        if (lane == 63) {
+            s_wave[wave] = incl;
+        }
+        __syncthreads();
+        uint32_t run = carry + incl - sum;
+#pragma unroll
+        for (int w = 0; w < kBlock / 64; ++w) {
+            run += w < wave ? s_wave[w] : 0u;
+            carry += s_wave[w];
+        }
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            if (at + k < n) {
+                out[at + k] = run;
+            }
+            run += v[k];
+        }
+        __syncthreads();
+    }
+}
+
+// Counters one block scans (16K: four rounds, under 10 us); more go through a device scan.  The kernel
+// writing them does not let its last block do it: the device-scope fence that takes writes back the L2
+// (the flag kernel of 450,000 entries 7 -> 59 us).
+constexpr int64_t kBlockScanMax = 1 << 14;
+
+__global__ __launch_bounds__(kBlock) void block_scan_kernel(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, int64_t n) {
+    block_scan(in, out, n);
 }
 
 // Entries per flag chunk: one wave's kFlagUnroll * 64 consecutive entries.
@@ -485,7 +588,7 @@ __device__ __forceinline__ void store_chunk_heads(const uint32_t (&f)[kFlagUnrol
 // chunk's heads.  Grid: flag_chunks(cap) waves of kFlagChunk entries.
 template <int W, int ORDER>
 __global__ __launch_bounds__(kBlock) void core_flag_unpack_kernel(const uint64_t* __restrict__ entries, int64_t cap,
-                                                                  uint32_t* __restrict__ flag, uint32_t* __restrict__ chunk_heads,
+                                                                  uint8_t* __restrict__ flag, uint32_t* __restrict__ chunk_heads,
                                                                   int sub_bits, const uint32_t* __restrict__ inv,
                                                                   const uint64_t* __restrict__ ckeys, uint32_t* __restrict__ keys,
                                                                   uint64_t* __restrict__ vals, int64_t* __restrict__ counts) {
@@ -504,7 +607,7 @@ __global__ __launch_bounds__(kBlock) void core_flag_unpack_kernel(const uint64_t
     for (int t = 0; t < kFlagUnroll; ++t) {
         const int64_t e = base + 64 * t + lane;
         if (e < cap) {
-            flag[e] = f[t];
+            flag[e] = static_cast<uint8_t>(f[t]);
             keys[e] = k[t];
             vals[e] = v[t];
         }
@@ -514,7 +617,7 @@ __global__ __launch_bounds__(kBlock) void core_flag_unpack_kernel(const uint64_t
 // Flags of sorted (key, value) pairs and each chunk's heads, as core_flag_unpack_kernel.
 template <int W, int ORDER>
 __global__ __launch_bounds__(kBlock) void core_flag_kernel(const uint32_t* __restrict__ keys, const uint64_t* __restrict__ vals, int64_t cap,
-                                                           const uint64_t* __restrict__ ckeys, uint32_t* __restrict__ flag,
+                                                           const uint64_t* __restrict__ ckeys, uint8_t* __restrict__ flag,
                                                            uint32_t* __restrict__ chunk_heads, int64_t* __restrict__ counts) {
     const int lane = threadIdx.x & 63;
     const int64_t base = (blockIdx.x * static_cast<int64_t>(blockDim.x) + (threadIdx.x & ~63)) * kFlagUnroll;
@@ -530,7 +633,7 @@ __global__ __launch_bounds__(kBlock) void core_flag_kernel(const uint32_t* __res
     for (int t = 0; t < kFlagUnroll; ++t) {
         const int64_t e = base + 64 * t + lane;
         if (e < cap) {
-            flag[e] = f[t];
+            flag[e] = static_cast<uint8_t>(f[t]);
         }
     }
 }
@@ -552,7 +655,7 @@ __global__ void key_flag_kernel(const uint32_t* __restrict__ keys, int64_t n, ui
 // next head or the end of the used entries) and the breaks before it from the wave's ballots; the
 // last head of the 64, whose group may run past them, reads on 64 flags at a time with the whole
 // wave.  Grid: flag_chunks(capacity) waves.
-__global__ __launch_bounds__(kBlock) void core_start_kernel(const uint32_t* __restrict__ flag, const uint32_t* __restrict__ chunk_off,
+__global__ __launch_bounds__(kBlock) void core_start_kernel(const uint8_t* __restrict__ flag, const uint32_t* __restrict__ chunk_off,
                                                             uint32_t* __restrict__ starts, int64_t* __restrict__ counts) {
     const int lane = threadIdx.x & 63;
     const int64_t used = counts[0];
@@ -617,6 +720,544 @@ __global__ __launch_bounds__(kBlock) void core_start_kernel(const uint32_t* __re
     }
 }
 
+// ------------------------------------------------------------------------------- group bins --
+// The groups of two or more entries, dealt into bins by size: one bin per size from 2 to 32, then
+// ranges of larger sizes, then what the mixed groups split into (any size).  The entries of a bin's groups are
+// copied next to each other in the form the group kernels use (row | slot << 32 | sign << 63, the
+// slot pair_slot of the removed pair, order 1 the removed site), so
+//   - a wave takes groups of one size: its lane layout is a division by that size, every lane group
+//     runs the same number of steps and the entries are one coalesced read (a wave that took 64
+//     consecutive groups of every size left half of its lanes idle in the groups of 9 to 32);
+//   - the groups of one entry (two thirds of them at 1M molecular configs) are never visited again;
+//   - no pair kernel reads a config or counts a bit: the sign is a factor of the entry.
+// Binning the 91M entries of 1M configs (52 spin orbitals) costs 0.75 ms once per index; one
+// application's pair kernel went from 5.90 to 5.02 ms, the single kernel from 1.57 to 1.12 ms (and 7.6
+// to 5.0 ms for the pair kernel of 200,000 two-word configs).
+// A mixed group (different cores under one key, about 1 in 100) is split by core when it is binned, so
+// the group kernels compare no cores either: its entries move to mvals core by core, and each core's
+// group of two or more takes one of the floor(size / 2) slots the mixed group has in the list.
+// Within a bin the groups keep the key order up to the order inside a block of bin_groups() groups.
+constexpr int kExactMax = 32;
+constexpr int kExactBins = kExactMax - 1;
+constexpr int kBigBins = 7;                       // up to 48, 64, 96, 128, 192, 256 and above
+constexpr int kSplitBin = kExactBins + kBigBins;  // the mixed groups, split by core
+constexpr int kBins = kSplitBin + 1;
+constexpr int kVarBins = kBins - kExactBins;      // bins whose groups are listed with their size
+constexpr int kBinRows = kBins + kVarBins;        // counters per block: groups per bin, entries per listed bin
+constexpr int kBinGroupsMax = 4096;               // groups per block of the two binning kernels, at most
+constexpr uint32_t kSplitSlots = 16;              // list slots per work unit of the split bin
+
+struct CoreBins {
+    uint32_t groups[kBins];
+    uint32_t entry_base[kBins];       // first entry of the bin in mvals
+    uint32_t list_base[kBins];        // listed bins: first entry of the bin in glist
+    uint32_t unit_start[kBins + 1];   // work units before the bin at this position (bins in descending order)
+};
+
+__device__ __forceinline__ int group_bin(uint32_t size, bool mixed) {
+    if (mixed) {
+        return kSplitBin;
+    }
+    if (size <= kExactMax) {
+        return static_cast<int>(size) - 2;
+    }
+    const int lg = 31 - __clz(size - 1u);                     // 33..64: 5, 65..128: 6, 129..256: 7
+    const int half = static_cast<int>(((size - 1u) >> (lg - 1)) & 1u);
+    const int k = 2 * (lg - 5) + half;
+    return kExactBins + (k < kBigBins ? k : kBigBins - 1);
+}
+
+// A work unit of a bin of size g: this many passes of 64 lanes (64 / g groups each), so that a unit of
+// small groups is worth its decoding and keeps a few gathers in flight.
+__host__ __device__ __forceinline__ int unit_passes(int g, int order) {
+    if (order == 1) {
+        return g <= 3 ? 2 : 1;
+    }
+    return g == 2 ? 8 : (g <= 4 ? 4 : (g <= 8 ? 2 : 1));
+}
+
+// Groups per block of the binning kernels: the fewest (a wave walks its part of the block's entries one
+// after another) that keep the counters within what one block scans.
+inline int bin_groups(int64_t cap) {
+    int g = 2 * kBlock;
+    while (g < kBinGroupsMax && (cap + g - 1) / g * kBinRows >= kBlockScanMax) {
+        g <<= 1;
+    }
+    return g;
+}
+
+inline int64_t bin_blocks(int64_t cap) { return (cap + bin_groups(cap) - 1) / bin_groups(cap); }
+
+// Bin table from the bins' groups and entries, thread b of the block calling it with bin b's (every
+// thread of the block calls it).
+__device__ __forceinline__ void bin_table(int b, uint32_t n, uint32_t entries, int order, CoreBins* __restrict__ bins) {
+    __shared__ uint32_t s_entries[kBins], s_units[kBins], s_list[kBins];
+    if (b < kBins) {
+        const bool listed = b >= kExactBins;
+        const int g = b + 2;
+        const uint32_t per_unit = listed ? 1u : static_cast<uint32_t>(64 / g * unit_passes(g, order));
+        s_entries[b] = entries;
+        // the split bin: a slot per two entries of its mixed groups
+        const uint32_t slots = b == kSplitBin ? s_entries[b] / 2u : n;
+        s_units[b] = b == kSplitBin ? (slots + kSplitSlots - 1u) / kSplitSlots : (n + per_unit - 1u) / per_unit;
+        s_list[b] = listed ? slots : 0u;
+        bins->groups[b] = slots;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t e = 0, l = 0, u = 0;
+        for (int k = 0; k < kBins; ++k) {
+            bins->entry_base[k] = e;
+            bins->list_base[k] = l;
+            e += s_entries[k];
+            l += s_list[k];
+        }
+        for (int p = 0; p < kBins; ++p) {
+            bins->unit_start[p] = u;
+            u += s_units[kBins - 1 - p];
+        }
+        bins->unit_start[kBins] = u;
+    }
+    __syncthreads();
+}
+
+// The bin table from the counters, by one block: summed here (hist non-null), or by a device scan.
+__global__ __launch_bounds__(kBlock) void bin_table_kernel(const uint32_t* __restrict__ hist, uint32_t* scan, int64_t nblk, int order,
+                                                           CoreBins* __restrict__ bins) {
+    if (hist != nullptr) {
+        block_scan(hist, scan, kBinRows * nblk + 1);
+        __threadfence_block();
+        __syncthreads();
+    }
+    const int b = threadIdx.x;
+    uint32_t n = 0, entries = 0;
+    if (b < kBins) {
+        n = scan[(b + 1) * nblk] - scan[b * nblk];
+        entries = b >= kExactBins ? scan[(b + kVarBins + 1) * nblk] - scan[(b + kVarBins) * nblk] : n * static_cast<uint32_t>(b + 2);
+    }
+    bin_table(b, n, entries, order, bins);
+}
+
+// hist[r * nblk + block]: groups of bin r among the block's groups (r < kBins), entries of the listed
+// bin r - kVarBins (above).  Every block writes its column; the last element is the scan's end.
+__global__ __launch_bounds__(kBlock) void bin_count_kernel(const uint32_t* __restrict__ starts, const int64_t* __restrict__ counts,
+                                                           int64_t nblk, int per_block, uint32_t* __restrict__ hist) {
+    __shared__ unsigned long long s_bin[kBins];
+    for (int b = threadIdx.x; b < kBins; b += kBlock) {
+        s_bin[b] = 0ull;
+    }
+    __syncthreads();
+    const int64_t groups = counts[1];
+    const int64_t g0 = static_cast<int64_t>(blockIdx.x) * per_block;
+    for (int t = 0; t < per_block; t += kBlock) {
+        const int64_t g = g0 + t + threadIdx.x;
+        if (g < groups) {
+            const uint32_t s = starts[g];
+            const uint32_t size = (starts[g + 1] & kGroupStart) - (s & kGroupStart);
+            if (size >= 2u) {
+                atomicAdd(&s_bin[group_bin(size, (s & kGroupMixed) != 0u)], (1ull << 32) | size);
+            }
+        }
+    }
+    __syncthreads();
+    for (int r = threadIdx.x; r < kBinRows; r += kBlock) {
+        hist[r * nblk + blockIdx.x] = static_cast<uint32_t>(r < kBins ? s_bin[r] >> 32 : s_bin[r - kVarBins]);
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        hist[kBinRows * nblk] = 0u;
+    }
+}
+
+// Splits the mixed group m (group, place in mvals) by core, by one wave: each core's entries go to the group's place in
+// mvals, in the order of their first entries, and take the next of the group's list slots; an entry
+// alone with its core has no partner and is dropped.  The slots of a group placed `a` entries into the
+// bin are [a / 2, (a + size) / 2): disjoint, and at least floor(size / 2) of them.  The rest are empty.
+template <int W, int ORDER>
+__device__ void split_group(const uint32_t* __restrict__ starts, const uint64_t* __restrict__ vals, const uint64_t* __restrict__ ckeys,
+                            const uint2 m, int n_bits, const CoreBins* __restrict__ bins, uint64_t* __restrict__ mvals,
+                            uint2* __restrict__ glist, int lane) {
+    const uint64_t below = (1ull << lane) - 1ull;
+    const auto binned = [&](uint64_t v, const Cfg<W>& core) {
+        const int x = static_cast<int>(v & 0xff), y = static_cast<int>((v >> 8) & 0xff);
+        const uint64_t slot = ORDER == 2 ? static_cast<uint64_t>(pair_slot(x, y, n_bits)) : static_cast<uint64_t>(x);
+        const int odd = ORDER == 2 ? masked_parity<W>(core, range_mask<W>(x, y)) : masked_parity<W>(core, range_mask<W>(0, x));
+        return (odd ? 1ull << 63 : 0ull) | (slot << 32) | (v >> 16);
+    };
+    const auto equal = [](const Cfg<W>& a, const Cfg<W>& b) {
+        bool same = true;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            same = same & (a.w[w] == b.w[w]);
+        }
+        return same;
+    };
+    const auto of_lane = [](const Cfg<W>& c, int l) {  // l wave-uniform
+        Cfg<W> r;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(c.w[w]), l);
+            const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(c.w[w] >> 32), l);
+            r.w[w] = (static_cast<uint64_t>(hi) << 32) | lo;
+        }
+        return r;
+    };
+    const uint32_t s = starts[m.x] & kGroupStart;
+    const uint32_t size = (starts[m.x + 1] & kGroupStart) - s;
+    const uint32_t a = m.y - bins->entry_base[kSplitBin];
+    uint32_t slot = bins->list_base[kSplitBin] + a / 2u;
+    const uint32_t slot_end = bins->list_base[kSplitBin] + (a + size) / 2u;
+    uint32_t out = m.y;
+    for (uint32_t a0 = 0; a0 < size; a0 += 64) {
+        const bool in_a = a0 + lane < size;
+        const uint64_t va = vals[s + (in_a ? a0 + lane : 0u)];
+        const Cfg<W> ca = entry_core<W, ORDER>(ckeys, va);
+        // the entries of this chunk that are the first with their core
+        bool first = in_a;
+        for (uint32_t b0 = 0; b0 <= a0; b0 += 64) {
+            const Cfg<W> cb = b0 == a0 ? ca : entry_core<W, ORDER>(ckeys, vals[s + b0 + lane]);
+            const int nb = static_cast<int>(size - b0 < 64u ? size - b0 : 64u);
+            for (int j = 0; j < nb; ++j) {
+                const bool same = equal(of_lane(cb, j), ca);
+                first = first & !(same & (b0 + static_cast<uint32_t>(j) < a0 + static_cast<uint32_t>(lane)));
+            }
+        }
+        uint64_t firsts = __ballot(first);
+        while (firsts) {
+            const int l = __builtin_ctzll(firsts);
+            firsts &= firsts - 1;
+            const Cfg<W> core = of_lane(ca, l);
+            uint32_t n = 0;
+            for (uint32_t b0 = a0; b0 < size; b0 += 64) {
+                const bool in_b = b0 + lane < size;
+                const uint64_t vb = b0 == a0 ? va : vals[s + (in_b ? b0 + lane : 0u)];
+                const bool same = in_b & equal(b0 == a0 ? ca : entry_core<W, ORDER>(ckeys, vb), core);
+                const uint64_t mask = __ballot(same);
+                if (same) {
+                    mvals[out + n + static_cast<uint32_t>(__popcll(mask & below))] = binned(vb, core);
+                }
+                n += static_cast<uint32_t>(__popcll(mask));
+            }
+            if (n >= 2u) {
+                if (lane == 0) {
+                    glist[slot] = make_uint2(out, n);
+                }
+                ++slot;
+                out += n;
+            }
+        }
+    }
+    for (uint32_t k = slot + lane; k < slot_end; k += 64) {
+        glist[k] = make_uint2(0u, 0u);
+    }
+}
+
+// Copies the entries of the groups of two or more into their bins and lists the groups of the listed
+// bins (first entry in mvals, size).  A block places its per_block groups, then its waves walk their
+// entries with the flags telling where groups start, then split the block's mixed groups, noted in
+// msplit as {group, place in mvals}.
+template <int W, int ORDER>
+__global__ __launch_bounds__(kBlock) void bin_scatter_kernel(const uint32_t* __restrict__ starts, const int64_t* __restrict__ counts,
+                                                             const uint8_t* __restrict__ flag, const uint64_t* __restrict__ vals,
+                                                             const uint64_t* __restrict__ ckeys, const uint32_t* __restrict__ scan, int64_t nblk, int per_block,
+                                                             int n_bits, const CoreBins* __restrict__ bins,
+                                                             uint64_t* __restrict__ mvals, uint2* __restrict__ glist,
+                                                             uint2* __restrict__ msplit) {
+    __shared__ unsigned long long s_rank[kBins];
+    __shared__ uint32_t s_group0[kBins], s_entry0[kBins];
+    __shared__ uint32_t s_move[kBinGroupsMax];  // binned position minus sorted position, kStay: not copied
+    constexpr uint32_t kStay = 0x80000000u;
+    const int64_t groups = counts[1];
+    const int64_t g0 = static_cast<int64_t>(blockIdx.x) * per_block;
+    if (g0 >= groups) {
+        return;  // the whole block
+    }
+    for (int b = threadIdx.x; b < kBins; b += kBlock) {
+        s_rank[b] = 0ull;
+        s_group0[b] = scan[b * nblk + blockIdx.x] - scan[b * nblk];
+        s_entry0[b] = b >= kExactBins ? scan[(b + kVarBins) * nblk + blockIdx.x] - scan[(b + kVarBins) * nblk] : 0u;
+    }
+    __syncthreads();
+    const int here = static_cast<int>(groups - g0 < per_block ? groups - g0 : per_block);
+    for (int t = threadIdx.x; t < here; t += kBlock) {
+        const uint32_t s = starts[g0 + t];
+        const uint32_t first = s & kGroupStart;
+        const uint32_t size = (starts[g0 + t + 1] & kGroupStart) - first;
+        uint32_t move = kStay;
+        if (size >= 2u) {
+            const int b = group_bin(size, (s & kGroupMixed) != 0u);
+            const unsigned long long r = atomicAdd(&s_rank[b], (1ull << 32) | size);
+            const uint32_t rank = s_group0[b] + static_cast<uint32_t>(r >> 32);
+            if (b < kExactBins) {
+                move = bins->entry_base[b] + rank * size - first;
+            } else {
+                const uint32_t at = bins->entry_base[b] + s_entry0[b] + static_cast<uint32_t>(r);
+                if (b == kSplitBin) {
+                    msplit[rank] = make_uint2(static_cast<uint32_t>(g0) + static_cast<uint32_t>(t), at);
+                } else {
+                    glist[bins->list_base[b] + rank] = make_uint2(at, size);
+                    move = at - first;
+                }
+            }
+        }
+        s_move[t] = move;
+    }
+    __threadfence_block();
+    __syncthreads();
+    // wave w: the entries of the block's groups [w, w + 1) * per_block / 4
+    const int lane = threadIdx.x & 63;
+    const int per_wave = per_block / (kBlock / 64);
+    const int lo = (threadIdx.x >> 6) * per_wave;
+    const int hi = lo + per_wave < here ? lo + per_wave : here;
+    const int64_t e0 = lo < here ? starts[g0 + lo] & kGroupStart : 0;
+    const int64_t e1 = lo < here ? starts[g0 + hi] & kGroupStart : 0;
+    const uint64_t upto = lane == 63 ? ~0ull : (1ull << (lane + 1)) - 1ull;
+    int g = lo - 1;  // group of the entry before the 64
+    constexpr int U = 4;
+    for (int64_t base = e0; base < e1; base += 64 * U) {
+        uint32_t f[U];
+        uint64_t v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t e = base + 64 * u + lane;
+            f[u] = e < e1 ? flag[e] : 0u;
+            v[u] = e < e1 ? vals[e] : 0ull;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t e = base + 64 * u + lane;
+            const uint64_t heads = __ballot((f[u] & kFlagHead) != 0u);
+            if (e < e1) {
+                const uint32_t move = s_move[g + __popcll(heads & upto)];
+                if (move != kStay) {
+                    const int x = static_cast<int>(v[u] & 0xff);
+                    const uint64_t slot =
+                        ORDER == 2 ? static_cast<uint64_t>(pair_slot(x, static_cast<int>((v[u] >> 8) & 0xff), n_bits)) : static_cast<uint64_t>(x);
+                    const uint64_t sign = (f[u] & kFlagSign) != 0u ? 1ull << 63 : 0ull;
+                    mvals[static_cast<uint32_t>(e) + move] = sign | (slot << 32) | (v[u] >> 16);
+                }
+            }
+            g += __popcll(heads);
+        }
+    }
+    const uint32_t n_mixed = static_cast<uint32_t>(s_rank[kSplitBin] >> 32);
+    for (uint32_t i = threadIdx.x >> 6; i < n_mixed; i += kBlock / 64) {
+        split_group<W, ORDER>(starts, vals, ckeys, msplit[s_group0[kSplitBin] + i], n_bits, bins, mvals, glist, lane);
+    }
+}
+
+// A small set's whole core index in one block: emission, sort, flags, starts and bins, everything
+// between in LDS.  The general build is some twenty launches of a few microseconds each, whatever the
+// size.  The limit is the LDS: 17 bytes an entry and the sort's power of two.  Entries sort by (key,
+// emission index k * n + row), the order the general build's stable sort gives.
+constexpr int kSmallCores = 8192;
+constexpr int kSmallThreads = 1024;
+
+struct SmallLds {
+    uint64_t entry[kSmallCores];    // key << 32 | emission index
+    uint16_t sites[kSmallCores];    // by emission index: y << 8 | x
+    uint16_t group[kSmallCores];    // by sorted position
+    uint16_t start[kSmallCores + 1];
+    uint16_t move[kSmallCores];     // by group: place in mvals, kSmallStay: not copied
+    uint8_t flag[kSmallCores];
+    uint8_t mixed[kSmallCores];     // by group
+    uint32_t wave_heads[kSmallThreads / 64];
+    unsigned long long rank[kBins];
+    uint32_t used, over, n_mixed;
+};
+constexpr uint32_t kSmallStay = 0xffffu;
+
+template <int W, int ORDER>
+__global__ __launch_bounds__(kSmallThreads) void cores_small_kernel(const uint64_t* __restrict__ ckeys, const uint64_t* __restrict__ cols,
+                                                                    int n, int n_bits, int per_config, uint32_t* __restrict__ keys,
+                                                                    uint64_t* __restrict__ vals, uint32_t* __restrict__ starts,
+                                                                    int64_t* __restrict__ counts, CoreBins* __restrict__ bins,
+                                                                    uint64_t* __restrict__ mvals, uint2* __restrict__ glist,
+                                                                    uint2* __restrict__ msplit) {
+    extern __shared__ uint64_t smem[];
+    SmallLds& L = *reinterpret_cast<SmallLds*>(smem);
+    const int tid = threadIdx.x;
+    const int cap = n * per_config;
+    int p2 = kSmallThreads;
+    while (p2 < cap) {
+        p2 <<= 1;
+    }
+    if (tid == 0) {
+        L.used = 0u;
+        L.over = 0u;
+        L.n_mixed = 0u;
+    }
+    for (int b = tid; b < kBins; b += kSmallThreads) {
+        L.rank[b] = 0ull;
+    }
+    for (int e = cap + tid; e < p2; e += kSmallThreads) {
+        L.entry[e] = ~0ull;
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += kSmallThreads) {
+        int k = 0;
+        emit_cores<W, ORDER>(load_key<W>(ckeys, i), cols, [&](uint32_t key, uint32_t sites) {
+            if (k < per_config) {
+                L.entry[k * n + i] = (static_cast<uint64_t>(key) << 32) | static_cast<uint32_t>(k * n + i);
+                L.sites[k * n + i] = static_cast<uint16_t>(sites);
+            }
+            ++k;
+        });
+        if (k > per_config) {
+            atomicAdd(&L.over, 1u);
+        }
+        atomicAdd(&L.used, static_cast<uint32_t>(k < per_config ? k : per_config));
+        for (; k < per_config; ++k) {
+            L.entry[k * n + i] = ~0ull;
+        }
+    }
+    // bitonic sort of the p2 entries
+    for (int size = 2; size <= p2; size <<= 1) {
+        for (int step = size >> 1; step > 0; step >>= 1) {
+            __syncthreads();
+            for (int t = tid; t < p2 / 2; t += kSmallThreads) {
+                const int a = 2 * t - (t & (step - 1));
+                const uint64_t x = L.entry[a], y = L.entry[a + step];
+                if ((x > y) == ((a & size) == 0)) {
+                    L.entry[a] = y;
+                    L.entry[a + step] = x;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    const int used = static_cast<int>(L.used);
+    const int per = (used + kSmallThreads - 1) / kSmallThreads;  // consecutive entries of a thread
+    const int lo = tid * per < used ? tid * per : used;
+    const int hi = lo + per < used ? lo + per : used;
+    const auto value = [&](int e) {
+        const uint32_t at = static_cast<uint32_t>(L.entry[e]);
+        return (static_cast<uint64_t>(at % static_cast<uint32_t>(n)) << 16) | L.sites[at];
+    };
+    uint32_t heads = 0;
+    Cfg<W> before{};
+    for (int e = lo; e < hi; ++e) {
+        const uint32_t key = static_cast<uint32_t>(L.entry[e] >> 32);
+        const bool with_prev = e > 0 && static_cast<uint32_t>(L.entry[e - 1] >> 32) == key;
+        const bool with_next = e + 1 < used && static_cast<uint32_t>(L.entry[e + 1] >> 32) == key;
+        const uint64_t v = value(e);
+        uint32_t f = with_prev ? 0u : kFlagHead;
+        if (with_prev || with_next) {
+            const Cfg<W> core = entry_core<W, ORDER>(ckeys, v);
+            if (with_prev && e == lo) {
+                before = entry_core<W, ORDER>(ckeys, value(e - 1));
+            }
+            bool same = true;
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                same = same && core.w[w] == before.w[w];
+            }
+            f |= with_prev && !same ? kFlagBreak : 0u;
+            const int a = ORDER == 2 ? static_cast<int>(v & 0xff) : 0;
+            const int b = static_cast<int>((ORDER == 2 ? v >> 8 : v) & 0xff);
+            f |= masked_parity<W>(core, range_mask<W>(a, b)) != 0 ? kFlagSign : 0u;
+            before = core;
+        }
+        heads += with_prev ? 0u : 1u;
+        L.flag[e] = static_cast<uint8_t>(f);
+        keys[e] = key;
+        vals[e] = v;
+    }
+    for (int e = used + tid; e < cap; e += kSmallThreads) {
+        keys[e] = kKeySentinel;
+        vals[e] = 0ull;
+    }
+    // the heads before each thread's entries
+    uint32_t incl = heads;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = __shfl_up(incl, d);
+        incl += (tid & 63) >= d ? o : 0u;
+    }
+    if ((tid & 63) == 63) {
+        L.wave_heads[tid >> 6] = incl;
+    }
+    __syncthreads();
+    uint32_t g = incl - heads, groups = 0;
+    for (int w = 0; w < kSmallThreads / 64; ++w) {
+        g += w < (tid >> 6) ? L.wave_heads[w] : 0u;
+        groups += L.wave_heads[w];
+    }
+    for (int e = lo; e < hi; ++e) {
+        if ((L.flag[e] & kFlagHead) != 0u) {
+            L.start[g] = static_cast<uint16_t>(e);
+            L.mixed[g] = 0;
+            ++g;
+        }
+        L.group[e] = static_cast<uint16_t>(g - 1u);
+    }
+    if (tid == 0) {
+        L.start[groups] = static_cast<uint16_t>(used);
+        counts[0] = used;
+        counts[1] = groups;
+        counts[2] = L.over;
+        counts[3] = 0;
+    }
+    __syncthreads();
+    for (int e = lo; e < hi; ++e) {
+        if ((L.flag[e] & kFlagBreak) != 0u) {
+            L.mixed[L.group[e]] = 1;
+        }
+    }
+    __syncthreads();
+    const int n_groups = static_cast<int>(groups);
+    for (int q = tid; q <= n_groups; q += kSmallThreads) {
+        const uint32_t first = L.start[q];
+        const bool mixed = q < n_groups && L.mixed[q] != 0;
+        starts[q] = first | (mixed ? kGroupMixed : 0u);
+        const uint32_t size = q < n_groups ? L.start[q + 1] - first : 0u;
+        if (size >= 2u) {
+            atomicAdd(&L.rank[group_bin(size, mixed)], (1ull << 32) | size);
+        }
+    }
+    __syncthreads();
+    const unsigned long long mine = tid < kBins ? L.rank[tid] : 0ull;
+    bin_table(tid, static_cast<uint32_t>(mine >> 32), static_cast<uint32_t>(mine), ORDER, bins);
+    if (tid < kBins) {
+        L.rank[tid] = 0ull;
+    }
+    __threadfence_block();
+    __syncthreads();
+    for (int q = tid; q < n_groups; q += kSmallThreads) {
+        const uint32_t first = L.start[q];
+        const uint32_t size = L.start[q + 1] - first;
+        uint32_t move = kSmallStay;
+        if (size >= 2u) {
+            const int b = group_bin(size, L.mixed[q] != 0);
+            const unsigned long long r = atomicAdd(&L.rank[b], (1ull << 32) | size);
+            const uint32_t rank = static_cast<uint32_t>(r >> 32);
+            move = bins->entry_base[b] + static_cast<uint32_t>(r);
+            if (b == kSplitBin) {
+                msplit[rank] = make_uint2(static_cast<uint32_t>(q), move);
+                atomicAdd(&L.n_mixed, 1u);
+                move = kSmallStay;
+            } else if (b >= kExactBins) {
+                glist[bins->list_base[b] + rank] = make_uint2(move, size);
+            }
+        }
+        L.move[q] = static_cast<uint16_t>(move);
+    }
+    __threadfence_block();
+    __syncthreads();
+    for (int e = lo; e < hi; ++e) {
+        const uint32_t q = L.group[e];
+        if (L.move[q] != kSmallStay) {
+            const uint64_t v = value(e);
+            const int x = static_cast<int>(v & 0xff);
+            const uint64_t slot =
+                ORDER == 2 ? static_cast<uint64_t>(pair_slot(x, static_cast<int>((v >> 8) & 0xff), n_bits)) : static_cast<uint64_t>(x);
+            mvals[L.move[q] + static_cast<uint32_t>(e) - L.start[q]] = ((L.flag[e] & kFlagSign) != 0u ? 1ull << 63 : 0ull) | (slot << 32) | (v >> 16);
+        }
+    }
+    for (uint32_t i = tid >> 6; i < L.n_mixed; i += kSmallThreads / 64) {
+        split_group<W, ORDER>(starts, vals, ckeys, msplit[i], n_bits, bins, mvals, glist, tid & 63);
+    }
+}
+
 // Bits of the sub field of a packed core value (order 2: pair slots, order 1: sites) and of the
 // row; the 32-bit value applies when both fit.
 inline int bits_for(int64_t range) {
@@ -660,6 +1301,7 @@ int cores_layout(Carver& cv, int n_qubytes, int64_t n, int max_occupied, int ord
     c.keys = cv.take<uint32_t>(cap);
     c.vals = cv.take<uint64_t>(cap);
     c.starts = cv.take<uint32_t>(cap + 1);
+    c.bins = cv.take<CoreBins>(1);
     size_t tmp = 0;
     {
         uint64_t* v = nullptr;
@@ -678,11 +1320,17 @@ int cores_layout(Carver& cv, int n_qubytes, int64_t n, int max_occupied, int ord
             return set_error(QMB_ERR_HIP, "rocprim exclusive_scan size query failed");
         }
         tmp = tmp > scan ? tmp : scan;
+        const size_t bin_counters = static_cast<size_t>(kBinRows * bin_blocks(static_cast<int64_t>(cap)) + 1);
+        if (rocprim::exclusive_scan(nullptr, scan, u, u, 0u, bin_counters, rocprim::plus<uint32_t>()) != hipSuccess) {
+            return set_error(QMB_ERR_HIP, "rocprim exclusive_scan size query failed");
+        }
+        tmp = tmp > scan ? tmp : scan;
     }
     const size_t s0 = cv.off;
+    const size_t bin_bytes = 2 * static_cast<size_t>(kBinRows * bin_blocks(static_cast<int64_t>(cap)) + 1) * sizeof(uint32_t) + 512;
     const size_t inv_bytes = static_cast<size_t>(8 * n_qubytes) * (8 * n_qubytes) / 2 * sizeof(uint32_t) + 256;
     const size_t chunk_bytes = 2 * static_cast<size_t>(flag_chunks(static_cast<int64_t>(cap))) * sizeof(uint32_t) + 512;
-    void* s = cv.take_bytes(2 * cap * sizeof(uint64_t) + cap * sizeof(uint32_t) + chunk_bytes + inv_bytes + tmp + 4096);
+    void* s = cv.take_bytes(2 * cap * sizeof(uint64_t) + cap + chunk_bytes + bin_bytes + inv_bytes + tmp + 4096);
     if (scratch) {
         *scratch = s;
     }
@@ -698,14 +1346,13 @@ int cores_layout(Carver& cv, int n_qubytes, int64_t n, int max_occupied, int ord
 
 // ------------------------------------------------------------------------------ group kernel --
 struct PairParams {
-    const double2* coef;    // merged pair-excitation coefficients, [pair_slot][pair_slot]
+    const double2* coef;    // merged pair-excitation coefficients with their own sites' sign, [pair_slot][pair_slot]
     const double* coef_re;  // their real parts when every coefficient is real, else null
     int64_t n_pairs;
-    int n_bits;
     int particle_cut;
-    const uint64_t* ckeys;  // config words of the set, [n][W]
-    const uint64_t* vals;   // sorted entries
-    const uint32_t* starts;
+    const uint64_t* mvals;  // binned entries
+    const uint2* glist;
+    const CoreBins* bins;
     const int64_t* counts;
     const double2* in;
     double2* out;
@@ -713,202 +1360,90 @@ struct PairParams {
     double2* out2;
 };
 
-// Sites in [a, b), a <= b: L(a) ^ L(b) with L(s) the sites below s.
-template <int W>
-__device__ __forceinline__ Cfg<W> range_mask(int a, int b) {
-    Cfg<W> m;
-    if (W == 1) {
-        m.w[0] = (1ull << b) - (1ull << a);  // sites of a one-word config are < 64
-    } else {
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            const int lo = a - 64 * w, hi = b - 64 * w;
-            const uint64_t mh = hi <= 0 ? 0ull : (hi >= 64 ? ~0ull : (1ull << hi) - 1ull);
-            const uint64_t ml = lo <= 0 ? 0ull : (lo >= 64 ? ~0ull : (1ull << lo) - 1ull);
-            m.w[w] = mh & ~ml;
-        }
-    }
-    return m;
-}
-
-template <int W>
-__device__ __forceinline__ int masked_parity(const Cfg<W>& c, const Cfg<W>& m) {
-    int par = 0;
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-        par ^= __popcll(c.w[w] & m.w[w]);
-    }
-    return par & 1;
-}
-
-// pair_parity(c) = popcount(c & (L(a) ^ L(b) ^ L(x) ^ L(y))) mod 2 for a < b, x < y.
-template <int W>
-__device__ __forceinline__ int pair_parity(const Cfg<W>& c, int a, int b, int x, int y) {
-    const Cfg<W> m1 = range_mask<W>(a, b);
-    const Cfg<W> m2 = range_mask<W>(x, y);
-    int par = 0;
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-        par ^= __popcll(c.w[w] & (m1.w[w] ^ m2.w[w]));
-    }
-    return par & 1;
-}
-
-// One staged group entry (b: a config of the group, removed sites q0 < q1), shared by the wave
-// through LDS: what every row a of the group needs of it, so the per-pair work is a few mask
-// operations, one coefficient load and the multiply-adds.
-template <int W>
-struct PairStage {
-    double2 g;          // in[row]
-    uint64_t bits[W];   // the sites q0 and q1 (all ones for an empty slot: it meets every row)
-    uint32_t part;      // the entry's part of the coefficient index: pair_slot(q0, q1) (ADJ), times n_pairs (!ADJ)
-    uint32_t ebit;      // parity of the group core's sites in [q0, q1)
-    uint64_t m[W];      // sites in [q0, q1)
-    uint32_t row;       // config row of the entry
-    uint32_t pad;
-    double2 g2;         // in2[row] of a two-vector pass
+// The lanes' entries as the rows of a group read them, in this wave's LDS: the amplitude with the
+// entry's sign and the entry's part of the coefficient index (order 1: its site).
+struct GroupStage {
+    double2 g[128];
+    uint32_t part[128];
 };
+struct GroupStage2 {
+    double2 g[128];
+    double2 g2[128];
+    uint32_t part[128];
+};
+template <int NV>
+struct StageOf {
+    using type = GroupStage;
+};
+template <>
+struct StageOf<2> {
+    using type = GroupStage2;
+};
+template <int NV>
+using Stage = typename StageOf<NV>::type;
 constexpr int kWavesPerBlock = kBlock / 64;
-constexpr size_t kPairStageBytes = kWavesPerBlock * 64 * sizeof(PairStage<2>);
-static_assert(sizeof(PairStage<1>) <= sizeof(PairStage<2>) && sizeof(PairStage<2>) % 16 == 0, "stage slot layout");
 
-__device__ __forceinline__ double2 shfl_d2(const double2& v, int lane) {
-    return make_double2(__shfl(v.x, lane), __shfl(v.y, lane));
+__device__ __forceinline__ double2 signed_by(const double2& v, uint32_t flip) {
+    const int f = static_cast<int>(flip << 31);
+    return make_double2(__hiloint2double(__double2hiint(v.x) ^ f, __double2loint(v.x)), __hiloint2double(__double2hiint(v.y) ^ f, __double2loint(v.y)));
 }
 
-// Coefficient gathers kept in flight per lane in pair_group: 4 in the one-vector pair kernel; 3 in
-// the two-vector pair kernel and the batched kernel, whose accumulators and other paths hold more
-// registers (4 there spills).
-constexpr int kPairBatch = 4;
-constexpr int kPairBatchInBatch = 3;
-
-template <int W>
-__device__ __forceinline__ Cfg<W> site_bits(int a, int b) {
-    Cfg<W> m;
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-        m.w[w] = ((a >> 6) == w ? (1ull << (a & 63)) : 0ull) | ((b >> 6) == w ? (1ull << (b & 63)) : 0ull);
-    }
-    return m;
-}
-
-// Stages entry b (value vb) of a group whose first core is core0.  An inactive slot gets all-ones
-// site bits, so every row sees it as overlapping and skips it.
-template <int W, bool ADJ, int NV>
-__device__ __forceinline__ PairStage<W> stage_entry(const PairParams& p, bool act, uint64_t vb, const Cfg<W>& core0, bool fermi) {
-    PairStage<W> st;
-    if (act) {
-        const int q0 = static_cast<int>(vb & 0xff);
-        const int q1 = static_cast<int>((vb >> 8) & 0xff);
-        st.row = static_cast<uint32_t>(vb >> 16);
-        st.g = p.in[st.row];
-        st.g2 = NV == 2 ? p.in2[st.row] : make_double2(0.0, 0.0);
-        const Cfg<W> mq = range_mask<W>(q0, q1);
-        const Cfg<W> bq = site_bits<W>(q0, q1);
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            st.m[w] = fermi ? mq.w[w] : 0ull;  // zero for hard-core bosons: no sign
-            st.bits[w] = bq.w[w];
-        }
-        const int64_t slot = pair_slot(q0, q1, p.n_bits);
-        st.part = static_cast<uint32_t>(ADJ ? slot : slot * p.n_pairs);
-        st.ebit = fermi ? static_cast<uint32_t>(masked_parity<W>(core0, mq)) : 0u;
-    } else {
-        st.row = 0;
-        st.g = make_double2(0.0, 0.0);
-        st.g2 = make_double2(0.0, 0.0);
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            st.m[w] = 0;
-            st.bits[w] = ~0ull;
-        }
-        st.part = 0;
-        st.ebit = 0;
-    }
-    st.pad = 0;
-    return st;
-}
-
-// What row a (removed sites r0 < r1, core `core`) keeps while it walks the staged entries.
-template <int W>
-struct PairRow {
-    Cfg<W> core;   // the row's config without r0, r1
-    Cfg<W> bits;   // r0 and r1
-    Cfg<W> mr;     // sites in [r0, r1)
-    int64_t part;  // the row's part of the coefficient index
-    int rbit;      // parity(core & [r0, r1)) ^ 1
+// A binned entry: row | slot << 32 | sign << 63.
+struct Entry {
+    uint32_t row;
+    uint32_t slot;
+    uint32_t sign;
 };
+__device__ __forceinline__ Entry binned_entry(uint64_t v, bool fermi) {
+    return Entry{static_cast<uint32_t>(v), static_cast<uint32_t>(v >> 32) & 0xffffu, fermi ? static_cast<uint32_t>(v >> 63) : 0u};
+}
 
-// Contribution of staged entry st to row ra, or false when the pair is not a connection: the
-// removed pairs overlap (which includes the row itself), or -- in a group where different cores
-// share the hash (mixed) -- the entry's core differs.  Signs (fermions):
-//   ADJ:  A_ba = (-1)^(rbit ^ ebit ^ parity(bits_a & [q0, q1))) T[Pa][Pb], applied conjugated
-//   !ADJ: A_ab = (-1)^(rbit ^ ebit ^ parity(bits_b & [r0, r1))) T[Pb][Pa]
-// with ebit taken from the row's own core in a mixed group.
-template <int W, bool ADJ, bool REAL>
-__device__ __forceinline__ bool pair_term(const PairParams& p, const PairRow<W>& ra, const PairStage<W>& st, bool mixed, bool en,
-                                          double2& x) {
-    uint64_t meet = 0;
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-        meet |= ra.bits.w[w] & st.bits[w];
+template <int NV, typename P>
+__device__ __forceinline__ void stage_lane(const P& p, Stage<NV>& st, int at, bool act, const Entry& e, uint32_t part) {
+    double2 g = make_double2(0.0, 0.0), g2 = g;
+    if (act) {
+        g = signed_by(p.in[e.row], e.sign);
+        if constexpr (NV == 2) {
+            g2 = signed_by(p.in2[e.row], e.sign);
+        }
     }
-    bool ok = en && meet == 0ull;
-    int ebit = static_cast<int>(st.ebit);
-    if (mixed) {
-        if (ok) {
-            const Cfg<W> cb = load_key<W>(p.ckeys, static_cast<int64_t>(st.row));
+    st.g[at] = g;
+    if constexpr (NV == 2) {
+        st.g2[at] = g2;
+    }
+    st.part[at] = part;
+}
+
+// out[row] += sign * (re, im) of the wave's active lanes (every lane calls it).  The sums go through the
+// lanes' own stage slots [at0, at0 + 64), so that neighbouring lanes hold the two components of one
+// row: their FP64 atomics leave as one 16-byte request instead of two.  The small pair groups are
+// bound by these requests: sizes 3 and 4 of 1M molecular configs took 0.96 ms with an instruction per
+// component, 0.51 ms so, and 0.31 ms without any atomics.
+template <int NV, typename P>
+__device__ __forceinline__ void add_rows(const P& p, Stage<NV>& st, int at0, int lane, bool act, const Entry& e, const double (&re)[NV],
+                                         const double (&im)[NV]) {
+    st.part[at0 + lane] = act ? e.row : ~0u;
 #pragma unroll
-            for (int w = 0; w < W; ++w) {
-                ok = ok && ((cb.w[w] ^ st.bits[w]) == ra.core.w[w]);
+    for (int v = 0; v < NV; ++v) {
+        st.g[at0 + lane] = signed_by(make_double2(re[v], im[v]), e.sign);
+        __builtin_amdgcn_wave_barrier();
+        double* out = reinterpret_cast<double*>(v == 0 ? p.out : p.out2);
+        const double* sums = reinterpret_cast<const double*>(st.g + at0);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const double x = sums[64 * h + lane];
+            const uint32_t row = st.part[at0 + 32 * h + (lane >> 1)];
+            if (row != ~0u && x != 0.0) {
+                unsafeAtomicAdd(&out[2 * static_cast<int64_t>(row) + (lane & 1)], x);
             }
         }
-        Cfg<W> mq;
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            mq.w[w] = st.m[w];
-        }
-        ebit = masked_parity<W>(ra.core, mq);
+        __builtin_amdgcn_wave_barrier();
     }
-    // only the lanes with a connection load a coefficient
-    x = make_double2(0.0, 0.0);
-    if (ok) {
-        const int64_t idx = ra.part + static_cast<int64_t>(st.part);
-        x = REAL ? make_double2(p.coef_re[idx], 0.0) : p.coef[idx];
-    }
-    // The sign's parity in bit 0: rbit ^ ebit plus the other pair's sites inside this pair's range
-    // (the range masks, rbit and ebit are zero for hard-core bosons).  Adding par << 31 to the high
-    // word flips the sign bit by bit 0 of par alone, without a branch.
-    uint32_t par = static_cast<uint32_t>(ra.rbit ^ ebit);
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-        const uint64_t m = ADJ ? (ra.bits.w[w] & st.m[w]) : (st.bits[w] & ra.mr.w[w]);
-        par += static_cast<uint32_t>(__popc(static_cast<uint32_t>(m))) + static_cast<uint32_t>(__popc(static_cast<uint32_t>(m >> 32)));
-    }
-    const int flip = static_cast<int>(par << 31);
-    x.x = __hiloint2double(__double2hiint(x.x) + flip, __double2loint(x.x));
-    if (!REAL) {
-        x.y = __hiloint2double(__double2hiint(x.y) + flip, __double2loint(x.y));
-    }
-    return ok;
 }
 
-template <int W>
-__device__ __forceinline__ PairRow<W> pair_row(const PairParams& p, const Cfg<W>& core, int r0, int r1, bool adj, bool fermi) {
-    PairRow<W> ra;
-    ra.core = core;
-    ra.bits = site_bits<W>(r0, r1);
-    ra.mr = range_mask<W>(r0, r1);
-    const int64_t slot = pair_slot(r0, r1, p.n_bits);
-    ra.part = adj ? slot * p.n_pairs : slot;
-    ra.rbit = fermi ? (masked_parity<W>(ra.core, ra.mr) ^ 1) : 0;
-    if (!fermi) {
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            ra.mr.w[w] = 0ull;  // no sign for hard-core bosons
-        }
-    }
-    return ra;
+template <bool REAL>
+__device__ __forceinline__ double2 pair_coef(const PairParams& p, uint32_t idx) {
+    return REAL ? make_double2(p.coef_re[idx], 0.0) : p.coef[idx];
 }
 
 // acc += x g (!ADJ) or conj(x) g (ADJ); a real table skips the imaginary part of x.
@@ -926,360 +1461,200 @@ __device__ __forceinline__ void pair_madd(const double2& x, const double2& g, do
     }
 }
 
-// One wave, one group of entries [s, e) (wave-uniform).  Lane = row a; the group's entries b are
-// staged 64 at a time in this wave's LDS slots and read back as broadcasts.
-//   ADJ:  out[a] += sum_b conj(A_ba) in[b]
-//   !ADJ: out[a] += sum_b A_ab in[b]
-// !ADJ reads T[Pb][Pa]: one table row per entry, at the columns of the lanes' rows.
-// s_raw: the group's start with its kGroupMixed bit.  In a group of one core every row's core is
-// the first entry's, so only that entry's config is read; a mixed group (different cores with
-// equal keys) reads every row's own config and checks every pair exactly.
-template <int W, bool ADJ, int B, int NV, bool REAL>
-__device__ void pair_group(const PairParams& p, uint32_t s_raw, uint32_t e, int lane, PairStage<W>* stage) {
-    const uint32_t s = s_raw & kGroupStart;
-    const bool mixed = (s_raw & kGroupMixed) != 0u;
-    const uint64_t v0 = p.vals[s];
-    const Cfg<W> core0 = entry_core<W, 2>(p.ckeys, v0);
+// With the sign split into one factor per entry and a part the table holds (pair_own_parity), a group
+// of entries (row_e, slot_e, sign_e) contributes
+//   ADJ:  out[row_a] += sign_a sum_b sign_b conj(T[slot_a][slot_b]) in[row_b]
+//   !ADJ: out[row_a] += sign_a sum_b sign_b T[slot_b][slot_a] in[row_b]
+// T being zero where the two pairs share a site (no pair excitation has fewer than four sites), which
+// includes a row with itself.  Per (row, entry) that is an LDS read, one gather and the multiply-adds.
+
+// Groups of G = 2..8 entries, lane = row, PU passes of 64 / G groups side by side.  Each row meets the
+// other G - 1 entries in turn (its own left out), all gathers of the lane in flight at once.  A zero
+// coefficient adds nothing, so a non-finite amplitude reaches only the rows it is connected to.
+template <bool ADJ, bool REAL, int NV, int G, int PU>
+__device__ __forceinline__ void pair_small(const PairParams& p, uint32_t e0, uint32_t e_end, int passes, int lane, Stage<NV>& st) {
+    constexpr int L = 64 / G * G;
     const bool fermi = p.particle_cut == 1;
-    for (uint32_t a0 = s; a0 < e; a0 += 64) {
-        const uint32_t a = a0 + lane;
-        const bool act = a < e;
-        const uint64_t va = act ? p.vals[a] : v0;
-        const PairRow<W> ra = pair_row<W>(p, mixed ? entry_core<W, 2>(p.ckeys, va) : core0, static_cast<int>(va & 0xff),
-                                          static_cast<int>((va >> 8) & 0xff), ADJ, fermi);
-        const int64_t ia = static_cast<int64_t>(va >> 16);
-        double acc_re[NV] = {}, acc_im[NV] = {};
-        for (uint32_t b0 = s; b0 < e; b0 += 64) {
-            const uint32_t bl = b0 + lane;
-            stage[lane] = stage_entry<W, ADJ, NV>(p, bl < e, bl < e ? p.vals[bl] : 0ull, core0, fermi);
-            __builtin_amdgcn_wave_barrier();
-            const int nb = static_cast<int>(e - b0 < 64u ? e - b0 : 64u);
-            for (int u = 0; u < nb; u += B) {
-                double2 x[B], g[B], g2[B];
-                bool ok[B];
+    const int ri = lane % G;
+    const int lead = lane - ri;
+    for (int q0 = 0; q0 < passes; q0 += PU) {
+        Entry e[PU];
+        bool act[PU];
+        uint32_t mine[PU];
+        if (e0 + static_cast<uint32_t>(q0 * L) >= e_end) {
+            return;  // the whole wave
+        }
 #pragma unroll
-                for (int k = 0; k < B; ++k) {
-                    const PairStage<W>& st = stage[(u + k) & 63];
-                    g[k] = st.g;
-                    g2[k] = NV == 2 ? st.g2 : make_double2(0.0, 0.0);
-                    // slots past nb hold entries of the previous chunk or nothing: bounded by u + k < nb
-                    ok[k] = pair_term<W, ADJ, REAL>(p, ra, st, mixed, act && (u + k < nb), x[k]);
+        for (int q = 0; q < PU; ++q) {
+            const uint32_t at = e0 + static_cast<uint32_t>((q0 + q) * L + lane);
+            act[q] = lane < L && at < e_end;
+            e[q] = binned_entry(act[q] ? p.mvals[at] : 0ull, fermi);
+        }
+#pragma unroll
+        for (int q = 0; q < PU; ++q) {
+            const uint32_t wide = e[q].slot * static_cast<uint32_t>(p.n_pairs);
+            mine[q] = ADJ ? wide : e[q].slot;
+            stage_lane<NV>(p, st, 64 * q + lane, act[q], e[q], ADJ ? e[q].slot : wide);
+        }
+        __builtin_amdgcn_wave_barrier();
+        double2 x[PU][G - 1];
+        int pl[G - 1];
+#pragma unroll
+        for (int u = 1; u < G; ++u) {
+            const int r = ri + u;
+            pl[u - 1] = (lead + (r >= G ? r - G : r)) & 63;
+        }
+#pragma unroll
+        for (int q = 0; q < PU; ++q) {
+#pragma unroll
+            for (int u = 0; u < G - 1; ++u) {
+                x[q][u] = make_double2(0.0, 0.0);
+                if (act[q]) {
+                    x[q][u] = pair_coef<REAL>(p, st.part[64 * q + pl[u]] + mine[q]);
                 }
+            }
+        }
 #pragma unroll
-                for (int k = 0; k < B; ++k) {
-                    // x[k] is zero where there is no connection, so the multiply-add needs no select
-                    // (a non-finite input amplitude then also reaches the rows of its group it is
-                    // not connected to)
-                    (void)ok[k];
-                    pair_madd<ADJ, REAL>(x[k], g[k], acc_re[0], acc_im[0]);
-                    if (NV == 2) {
-                        pair_madd<ADJ, REAL>(x[k], g2[k], acc_re[NV - 1], acc_im[NV - 1]);
+        for (int q = 0; q < PU; ++q) {
+            double re[NV] = {}, im[NV] = {};
+#pragma unroll
+            for (int u = 0; u < G - 1; ++u) {
+                if (x[q][u].x != 0.0 || (!REAL && x[q][u].y != 0.0)) {
+                    pair_madd<ADJ, REAL>(x[q][u], st.g[64 * q + pl[u]], re[0], im[0]);
+                    if constexpr (NV == 2) {
+                        pair_madd<ADJ, REAL>(x[q][u], st.g2[64 * q + pl[u]], re[1], im[1]);
                     }
                 }
             }
+            add_rows<NV>(p, st, 64 * q, lane, act[q], e[q], re, im);
+        }
+    }
+}
+
+// Steps b of a walk over `nb` staged entries from slot `lead`, each lane's row against the same entry
+// of its group: the lanes of a group read one table row (!ADJ), their columns ascending.  B gathers
+// in flight.  Zero coefficients are multiplied in (a non-finite amplitude reaches the whole group).
+template <bool ADJ, bool REAL, int NV, int B>
+__device__ __forceinline__ void pair_walk(const PairParams& p, const Stage<NV>& st, int lead, int nb, uint32_t mine, double (&re)[NV],
+                                          double (&im)[NV]) {
+    for (int u = 0; u < nb; u += B) {
+        double2 x[B];
+#pragma unroll
+        for (int k = 0; k < B; ++k) {
+            x[k] = make_double2(0.0, 0.0);
+            if (u + k < nb) {  // wave-uniform
+                x[k] = pair_coef<REAL>(p, st.part[lead + u + k] + mine);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < B; ++k) {
+            if (u + k < nb) {
+                pair_madd<ADJ, REAL>(x[k], st.g[lead + u + k], re[0], im[0]);
+                if constexpr (NV == 2) {
+                    pair_madd<ADJ, REAL>(x[k], st.g2[lead + u + k], re[1], im[1]);
+                }
+            }
+        }
+    }
+}
+
+// Groups of g = 9..32 entries, lane = row, 64 / g groups to a pass.
+template <bool ADJ, bool REAL, int NV, int B>
+__device__ __forceinline__ void pair_rows(const PairParams& p, int g, uint32_t e0, uint32_t e_end, int lane, Stage<NV>& st) {
+    const bool fermi = p.particle_cut == 1;
+    const int lanes = 64 / g * g;
+    const uint32_t at = e0 + static_cast<uint32_t>(lane);
+    const bool act = lane < lanes && at < e_end;
+    const int lead = act ? lane / g * g : 0;
+    const Entry e = binned_entry(act ? p.mvals[at] : 0ull, fermi);
+    const uint32_t wide = e.slot * static_cast<uint32_t>(p.n_pairs);
+    stage_lane<NV>(p, st, lane, act, e, ADJ ? e.slot : wide);
+    __builtin_amdgcn_wave_barrier();
+    double re[NV] = {}, im[NV] = {};
+    pair_walk<ADJ, REAL, NV, B>(p, st, lead, g, ADJ ? wide : e.slot, re, im);
+    add_rows<NV>(p, st, 0, lane, act, e, re, im);
+}
+
+// One group of any size from mvals[s]: 64 rows at a time against its entries, 64 staged
+// at a time.
+template <bool ADJ, bool REAL, int NV, int B>
+__device__ __forceinline__ void pair_big(const PairParams& p, uint32_t s, uint32_t size, int lane, Stage<NV>& st) {
+    const bool fermi = p.particle_cut == 1;
+    const auto wide = [&](const Entry& e) { return e.slot * static_cast<uint32_t>(p.n_pairs); };
+    for (uint32_t a0 = 0; a0 < size; a0 += 64) {
+        const bool act = a0 + lane < size;
+        const Entry e = binned_entry(act ? p.mvals[s + a0 + lane] : 0ull, fermi);
+        const uint32_t mine = ADJ ? wide(e) : e.slot;
+        double re[NV] = {}, im[NV] = {};
+        for (uint32_t b0 = 0; b0 < size; b0 += 64) {
+            const bool in = b0 + lane < size;
+            const Entry b = b0 == a0 ? e : binned_entry(in ? p.mvals[s + b0 + lane] : 0ull, fermi);
+            stage_lane<NV>(p, st, lane, in, b, ADJ ? b.slot : wide(b));
+            __builtin_amdgcn_wave_barrier();
+            pair_walk<ADJ, REAL, NV, B>(p, st, 0, static_cast<int>(size - b0 < 64u ? size - b0 : 64u), mine, re, im);
             __builtin_amdgcn_wave_barrier();
         }
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            if (act && (acc_re[v] != 0.0 || acc_im[v] != 0.0)) {
-                double2* o = v == 0 ? p.out : p.out2;
-                unsafeAtomicAdd(&o[ia].x, acc_re[v]);
-                unsafeAtomicAdd(&o[ia].y, acc_im[v]);
-            }
-        }
+        add_rows<NV>(p, st, 0, lane, act, e, re, im);
     }
 }
 
-// A pass over groups of 9..32 entries, lane = row: whole groups are taken from `mask` in lane order
-// while their rows fit the 64 lanes, a group's rows consecutive from `lead`.  nmax: the largest
-// group of the pass.  Lanes past the pass's groups get s = e = 0.
-struct RowLane {
-    uint32_t s, e;  // the lane's group (s with its kGroupMixed bit)
-    int lead;       // lane of the group's first row
-    int nmax;
-};
-
-__device__ __forceinline__ RowLane row_pass(uint64_t& mask, uint32_t gs_l, uint32_t ge_l, int lane) {
-    RowLane f{0u, 0u, 0, 0};
-    int used = 0;
-    while (mask) {
-        const int l = __builtin_ctzll(mask);
-        const uint32_t sj = __builtin_amdgcn_readlane(gs_l, l);
-        const uint32_t ej = __builtin_amdgcn_readlane(ge_l, l);
-        const int nj = static_cast<int>(ej - (sj & kGroupStart));
-        if (used + nj > 64) {
-            break;
-        }
-        mask &= mask - 1;
-        if (lane >= used && lane < used + nj) {
-            f.s = sj;
-            f.e = ej;
-            f.lead = used;
-        }
-        used += nj;
-        f.nmax = nj > f.nmax ? nj : f.nmax;
-    }
-    return f;
+// The bin and the unit within it of unit u (every lane calls it, u wave-uniform): the last position
+// whose first unit is <= u.
+__device__ __forceinline__ int unit_bin(const CoreBins* bins, uint32_t u, int lane, uint32_t* local) {
+    const uint32_t first = bins->unit_start[lane < kBins ? lane : kBins];
+    const uint64_t upto = __ballot(lane < kBins && first <= u);
+    const int pos = 63 - __builtin_clzll(upto);
+    *local = u - static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(first), pos));
+    return kBins - 1 - pos;
 }
 
-// Groups of 9..32 entries laid out by row_pass (a 9-entry group takes 9 lanes, so 7 of them share a
-// pass).  A group's entries are its rows, so each lane stages its own entry in its LDS slot and the
-// rows of a group walk the slots of that group, as in pair_group.
-template <int W, bool ADJ, int B, int NV, bool REAL>
-__device__ void pair_group_rows(const PairParams& p, uint64_t mask, uint32_t gs_l, uint32_t ge_l, int lane, PairStage<W>* stage) {
-    const bool fermi = p.particle_cut == 1;
-    while (mask) {
-        const RowLane f = row_pass(mask, gs_l, ge_l, lane);
-        const bool mixed = (f.s & kGroupMixed) != 0u;
-        const uint32_t s = f.s & kGroupStart;
-        const int g = static_cast<int>(f.e - s);  // 0 for a lane without a group
-        const int ri = lane - f.lead;
-        const bool act = ri < g;
-        const uint64_t va = act ? p.vals[s + static_cast<uint32_t>(ri)] : 0ull;
-        const int64_t ia = static_cast<int64_t>(va >> 16);
-        const int r0 = static_cast<int>(va & 0xff);
-        const int r1 = static_cast<int>((va >> 8) & 0xff);
-        // the group's first row reads its config for the group (a mixed group: every row its own)
-        Cfg<W> own;
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            own.w[w] = act && (mixed || ri == 0) ? p.ckeys[ia * W + w] : 0ull;
-        }
-        if (act) {
-            flip_site<W>(own, r0);
-            flip_site<W>(own, r1);
-        }
-        // the group's first core, from the lane holding its first row (every lane runs every shuffle)
-        Cfg<W> core0;
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            core0.w[w] = shfl_u64(own.w[w], f.lead);
-        }
-        const PairRow<W> ra = pair_row<W>(p, mixed ? own : core0, r0, r1, ADJ, fermi);
-        // the exact per-pair check runs wave-wide when any group of the pass is mixed: a row of a
-        // group of one core holds its true core (core0) and passes it for its connections
-        const bool wmixed = __ballot(mixed) != 0ull;
-        // this lane's entry (its own row), staged for the rows of its group
-        stage[lane] = stage_entry<W, ADJ, NV>(p, act, va, core0, fermi);
-        double acc_re[NV] = {}, acc_im[NV] = {};
-        __builtin_amdgcn_wave_barrier();
-        for (int u = 0; u < f.nmax; u += B) {
-            double2 x[B], gv[B], gv2[B];
-            bool ok[B];
-#pragma unroll
-            for (int k = 0; k < B; ++k) {
-                const int uu = u + k;
-                // slots past the group belong to other groups or to no group: bounded by uu < g
-                const PairStage<W>& st = stage[(f.lead + uu) & 63];
-                gv[k] = st.g;
-                gv2[k] = NV == 2 ? st.g2 : make_double2(0.0, 0.0);
-                ok[k] = pair_term<W, ADJ, REAL>(p, ra, st, wmixed, act && uu < g, x[k]);
-            }
-#pragma unroll
-            for (int k = 0; k < B; ++k) {
-                (void)ok[k];  // x[k] is zero where there is no connection
-                pair_madd<ADJ, REAL>(x[k], gv[k], acc_re[0], acc_im[0]);
-                if (NV == 2) {
-                    pair_madd<ADJ, REAL>(x[k], gv2[k], acc_re[NV - 1], acc_im[NV - 1]);
-                }
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            if (act && (acc_re[v] != 0.0 || acc_im[v] != 0.0)) {
-                double2* o = v == 0 ? p.out : p.out2;
-                unsafeAtomicAdd(&o[ia].x, acc_re[v]);
-                unsafeAtomicAdd(&o[ia].y, acc_im[v]);
-            }
-        }
+// The groups of a listed unit: one group of a bin above 32 entries, or kSplitSlots slots of the split
+// bin, most of them empty.  f(first entry, size) runs for each, wave-uniform.
+template <typename P, typename F>
+__device__ __forceinline__ void for_listed(const P& p, int bin, uint32_t local, int lane, F&& f) {
+    if (bin != kSplitBin) {
+        const uint2 group = p.glist[p.bins->list_base[bin] + local];
+        f(group.x, group.y);
+        return;
+    }
+    const uint32_t slot = local * kSplitSlots + static_cast<uint32_t>(lane);
+    const bool in = lane < static_cast<int>(kSplitSlots) && slot < p.bins->groups[kSplitBin];
+    const uint2 mine = in ? p.glist[p.bins->list_base[kSplitBin] + slot] : make_uint2(0u, 0u);
+    uint64_t full = __ballot(mine.y != 0u);
+    while (full) {
+        const int l = __builtin_ctzll(full);
+        full &= full - 1;
+        f(__builtin_amdgcn_readlane(mine.x, l), __builtin_amdgcn_readlane(mine.y, l));
     }
 }
 
-// A pass over groups of 2..8 entries with their ordered (row, entry) pairs side by side: whole
-// groups are taken from `mask` in lane order while their pairs fit the 64 lanes.  A group of g
-// entries takes g (g - 1) lanes from `lead`, row a's g - 1 pairs consecutive (entry b = j, or j + 1
-// from j = a on), so no lane pairs a row with itself; a 3-entry group takes 6 lanes instead of a
-// 4 x 4 block.  Lanes past the pass's groups get s = e = 0.
-struct FlatLane {
-    uint32_t s, e;  // the lane's group (s with its kGroupMixed bit)
-    int ai, bi;     // row and entry in the group
-    int j, d;       // position in row ai's run of d = g - 1 lanes
-    int lead;       // lane of the group's first pair (row 0, j = 0)
-    int rowb;       // lane of row bi's first pair
-};
+// Coefficient gathers in flight per lane of the larger groups.
+constexpr int kPairBatch = 8;
 
-__device__ __forceinline__ FlatLane flat_pass(uint64_t& mask, uint32_t gs_l, uint32_t ge_l, int lane) {
-    FlatLane f{0u, 0u, 0, 0, 0, 1, 0, 0};
-    int used = 0;
-    while (mask) {
-        const int l = __builtin_ctzll(mask);
-        const uint32_t sj = __builtin_amdgcn_readlane(gs_l, l);
-        const uint32_t ej = __builtin_amdgcn_readlane(ge_l, l);
-        const int nj = static_cast<int>(ej - (sj & kGroupStart));
-        const int len = nj * (nj - 1);
-        if (used + len > 64) {
-            break;
+// One work unit of the pair bins.
+template <bool ADJ, bool REAL, int NV, int B>
+__device__ __forceinline__ void pair_unit(const PairParams& p, uint32_t u, int lane, Stage<NV>& st) {
+    uint32_t local;
+    const int bin = unit_bin(p.bins, u, lane, &local);
+    if (bin < kExactBins) {
+        const int g = bin + 2;
+        const int passes = unit_passes(g, 2);
+        const uint32_t base = p.bins->entry_base[bin];
+        const uint32_t e0 = base + local * static_cast<uint32_t>(64 / g * g * passes);
+        const uint32_t e_end = base + p.bins->groups[bin] * static_cast<uint32_t>(g);
+        switch (g) {
+            case 2: pair_small<ADJ, REAL, NV, 2, 2>(p, e0, e_end, passes, lane, st); break;
+            case 3: pair_small<ADJ, REAL, NV, 3, 2>(p, e0, e_end, passes, lane, st); break;
+            case 4: pair_small<ADJ, REAL, NV, 4, 2>(p, e0, e_end, passes, lane, st); break;
+            case 5: pair_small<ADJ, REAL, NV, 5, 1>(p, e0, e_end, passes, lane, st); break;
+            case 6: pair_small<ADJ, REAL, NV, 6, 1>(p, e0, e_end, passes, lane, st); break;
+            case 7: pair_small<ADJ, REAL, NV, 7, 1>(p, e0, e_end, passes, lane, st); break;
+            case 8: pair_small<ADJ, REAL, NV, 8, 1>(p, e0, e_end, passes, lane, st); break;
+            default: pair_rows<ADJ, REAL, NV, B>(p, g, e0, e_end, lane, st); break;
         }
-        mask &= mask - 1;
-        if (lane >= used && lane < used + len) {
-            f.s = sj;
-            f.e = ej;
-            f.lead = used;
-        }
-        used += len;
+        return;
     }
-    const int g = static_cast<int>(f.e - (f.s & kGroupStart));
-    f.d = g > 1 ? g - 1 : 1;
-    const uint32_t k = static_cast<uint32_t>(lane - f.lead);
-    f.ai = static_cast<int>(k / static_cast<uint32_t>(f.d));
-    f.j = static_cast<int>(k) - f.ai * f.d;
-    f.bi = f.j + (f.j >= f.ai ? 1 : 0);
-    f.rowb = f.lead + f.bi * f.d;
-    return f;
-}
-
-// Sums each row's run of d lanes into its first lane (j = 0); d <= 7.
-__device__ __forceinline__ void flat_row_sum(double& re, double& im, int j, int d) {
-    for (int m = 1; m < 8; m <<= 1) {
-        const double ore = __shfl_down(re, m);
-        const double oim = __shfl_down(im, m);
-        if (j + m < d) {
-            re += ore;
-            im += oim;
-        }
-    }
-}
-
-// Groups of 2..8 entries laid out by flat_pass: one lane per ordered (row a, entry b) pair.  Each
-// lane checks its pair exactly (cores compared through a shuffle from the lane holding row b), the
-// rows are summed over their runs, and the first lane of each row adds the sum.  `mask` holds the
-// lanes of the 64-group chunk whose group has 2..8 entries; (gs_l, ge_l) is that lane's group.
-template <int W, bool ADJ, int NV>
-__device__ void pair_flat_class(const PairParams& p, uint64_t mask, uint32_t gs_l, uint32_t ge_l, int lane) {
-    const bool fermi = p.particle_cut == 1;
-    while (mask) {
-        const FlatLane f = flat_pass(mask, gs_l, ge_l, lane);
-        const bool mixed = (f.s & kGroupMixed) != 0u;
-        const uint32_t s = f.s & kGroupStart;
-        const bool act = f.e > s;
-        const uint64_t va = act ? p.vals[s + f.ai] : 0ull;
-        const uint64_t vb = act ? p.vals[s + f.bi] : 0ull;
-        const int64_t ia = static_cast<int64_t>(va >> 16);
-        const int r0 = static_cast<int>(va & 0xff), r1 = static_cast<int>((va >> 8) & 0xff);
-        const int q0 = static_cast<int>(vb & 0xff), q1 = static_cast<int>((vb >> 8) & 0xff);
-        // the coefficient and the input row need only the entries: loaded beside the stored configs
-        // and dropped below when the cores differ (entry 0 of the table and row 0 of the input are
-        // always there)
-        const bool pre = act && q0 != r0 && q0 != r1 && q1 != r0 && q1 != r1;
-        const int64_t idx = !pre ? 0
-                                 : (ADJ ? pair_slot(r0, r1, p.n_bits) * p.n_pairs + pair_slot(q0, q1, p.n_bits)
-                                        : pair_slot(q0, q1, p.n_bits) * p.n_pairs + pair_slot(r0, r1, p.n_bits));
-        const double2 x = p.coef_re ? make_double2(p.coef_re[idx], 0.0) : p.coef[idx];
-        const int64_t ib = pre ? static_cast<int64_t>(vb >> 16) : 0;
-        double2 gv[NV];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            gv[v] = (v == 0 ? p.in : p.in2)[ib];
-        }
-        // the lanes of the group's first row read its config for the group (a mixed group: every
-        // row its own)
-        Cfg<W> own;
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            own.w[w] = act && (mixed || f.ai == 0) ? p.ckeys[ia * W + w] : 0ull;
-        }
-        if (act) {
-            flip_site<W>(own, r0);
-            flip_site<W>(own, r1);
-        }
-        // every lane runs every shuffle (a short-circuit would leave lanes out)
-        Cfg<W> core;
-        bool same = true;
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            const uint64_t c0 = shfl_u64(own.w[w], f.lead);
-            core.w[w] = mixed ? own.w[w] : c0;
-            const bool eq = shfl_u64(own.w[w], f.rowb) == own.w[w];
-            same = same & eq;
-        }
-        const bool ok = pre && (same || !mixed);
-        double acc_re[NV] = {}, acc_im[NV] = {};
-        if (ok) {
-            int sg;
-            if (ADJ) {
-                Cfg<W> ca = core;
-                flip_site<W>(ca, r0);
-                flip_site<W>(ca, r1);
-                sg = fermi ? pair_parity<W>(ca, r0, r1, q0, q1) : 0;
-            } else {
-                Cfg<W> cb = core;
-                flip_site<W>(cb, q0);
-                flip_site<W>(cb, q1);
-                sg = fermi ? pair_parity<W>(cb, r0, r1, q0, q1) : 0;
-            }
-            const double xr = sg ? -x.x : x.x;
-            const double xi = sg ? -x.y : x.y;
-#pragma unroll
-            for (int v = 0; v < NV; ++v) {
-                if (ADJ) {
-                    acc_re[v] = xr * gv[v].x + xi * gv[v].y;
-                    acc_im[v] = xr * gv[v].y - xi * gv[v].x;
-                } else {
-                    acc_re[v] = xr * gv[v].x - xi * gv[v].y;
-                    acc_im[v] = xr * gv[v].y + xi * gv[v].x;
-                }
-            }
-        }
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            flat_row_sum(acc_re[v], acc_im[v], f.j, f.d);
-            if (f.j == 0 && act && (acc_re[v] != 0.0 || acc_im[v] != 0.0)) {
-                double2* o = v == 0 ? p.out : p.out2;
-                unsafeAtomicAdd(&o[ia].x, acc_re[v]);
-                unsafeAtomicAdd(&o[ia].y, acc_im[v]);
-            }
-        }
-    }
-}
-
-// The groups above 8 entries of a 64-group chunk: packed several to a wave up to 32 entries (PACK),
-// then one wave per group.
-template <int W, bool ADJ, int B, int NV, bool PACK, bool REAL>
-__device__ __forceinline__ void pair_chunk_groups(const PairParams& p, uint32_t gs, uint32_t ge, uint32_t sz, int lane,
-                                                  PairStage<W>* stage) {
-    if (PACK) {
-        pair_group_rows<W, ADJ, B, NV, REAL>(p, __ballot(sz > 8u && sz <= 32u), gs, ge, lane, stage);
-    }
-    uint64_t big = __ballot(sz > (PACK ? 32u : 8u));
-    while (big) {
-        const int l = __builtin_ctzll(big);
-        big &= big - 1;
-        pair_group<W, ADJ, B, NV, REAL>(p, __shfl(gs, l), __shfl(ge, l), lane, stage);
-    }
-}
-
-// The pair work of the groups [g0, g0 + 64): groups of up to 8 entries with their ordered pairs
-// side by side (pair_flat_class), larger ones packed or a row block at a time (pair_group).
-template <int W, bool ADJ, int B, int NV, bool PACK = true>
-__device__ __forceinline__ void pair_chunk(const PairParams& p, int64_t groups, int64_t g0, int lane, char* stage_bytes) {
-    const int64_t gg = g0 + lane;
-    uint32_t gs = 0, ge = 0;  // gs keeps the group's kGroupMixed bit for the group functions
-    if (gg < groups) {
-        gs = p.starts[gg];
-        ge = p.starts[gg + 1] & kGroupStart;
-    }
-    const uint32_t sz = ge - (gs & kGroupStart);
-    pair_flat_class<W, ADJ, NV>(p, __ballot(sz >= 2u && sz <= 8u), gs, ge, lane);
-    // each wave owns 64 slots of the largest stage size: waves of one block may run different W
-    PairStage<W>* stage = reinterpret_cast<PairStage<W>*>(stage_bytes + (threadIdx.x >> 6) * 64 * sizeof(PairStage<2>));
-    // PACK: groups of 9..32 entries several to a wave (else one group per wave)
-    // a real table (wave-uniform) takes the loops specialised for 8-byte coefficients
-    if (p.coef_re != nullptr) {
-        pair_chunk_groups<W, ADJ, B, NV, PACK, true>(p, gs, ge, sz, lane, stage);
-    } else {
-        pair_chunk_groups<W, ADJ, B, NV, PACK, false>(p, gs, ge, sz, lane, stage);
-    }
+    for_listed(p, bin, local, lane, [&](uint32_t s, uint32_t size) { pair_big<ADJ, REAL, NV, B>(p, s, size, lane, st); });
 }
 
 __device__ __forceinline__ void mark_overflow(double2* out) {
@@ -1287,24 +1662,22 @@ __device__ __forceinline__ void mark_overflow(double2* out) {
     out[0] = make_double2(__longlong_as_double(0x7ff8000000000000ll), __longlong_as_double(0x7ff8000000000000ll));
 }
 
-// Persistent waves over the groups, 64 groups per step.  Every wave leaves when the group count
-// is done.
-template <int W, bool ADJ, int NV = 1>
+// Persistent waves over the units of the bins.  Every wave leaves when the units are done.
+template <bool ADJ, bool REAL, int NV>
 __global__ __launch_bounds__(kBlock) void pair_kernel(PairParams p) {
+    __shared__ Stage<NV> stages[kWavesPerBlock];
     const int lane = threadIdx.x & 63;
-    const int64_t wave = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) >> 6;
-    const int64_t nwaves = (static_cast<int64_t>(gridDim.x) * kBlock) >> 6;
+    const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6))));
+    const uint32_t nwaves = gridDim.x * kWavesPerBlock;
     if (p.counts[2] != 0) {
         if (wave == 0 && lane == 0) {
             mark_overflow(p.out);
         }
         return;
     }
-    __shared__ __align__(16) char stage[kPairStageBytes];
-    const int64_t groups = p.counts[1];
-    for (int64_t g0 = wave * 64; g0 < groups; g0 += nwaves * 64) {
-        // two vectors hold twice the accumulators: fewer coefficient gathers in flight per lane
-        pair_chunk<W, ADJ, NV == 1 ? kPairBatch : kPairBatchInBatch, NV>(p, groups, g0, lane, stage);
+    const uint32_t units = p.bins->unit_start[kBins];
+    for (uint32_t u = wave; u < units; u += nwaves) {
+        pair_unit<ADJ, REAL, NV, NV == 1 ? kPairBatch : kPairBatch / 2>(p, u, lane, stages[threadIdx.x >> 6]);
     }
 }
 
@@ -1320,7 +1693,10 @@ __global__ void singles_fill_kernel(const int16_t* __restrict__ site, const uint
         SingleExcitation e;
         if (c.status == kCompileOk && single_excitation(c.rec, particle_cut, &e)) {
             const double2 v0 = coef[t];
-            const double2 v = e.delta ? make_double2(-v0.x, -v0.y) : v0;
+            // single_parity(core + r) = popcount(core & (L(r) ^ L(p))) + (r < p): the last part is the
+            // table's, the rest a sign per (core, site)
+            const int flip = e.delta ^ ((particle_cut == 1 && e.r < e.p) ? 1 : 0);
+            const double2 v = flip ? make_double2(-v0.x, -v0.y) : v0;
             const int64_t rp = static_cast<int64_t>(e.r) * n_bits + e.p;
             if (e.k < 0 || !e.kocc) {
                 // holds whenever k is empty
@@ -1364,15 +1740,16 @@ int singles_layout(Carver& cv, int n_qubytes, qmb_singles* out) {
 }
 
 struct SingleParams {
-    const double2* a;
+    const double2* a;       // the single-excitation table with the sign of r < p in it
     const double2* kd;
     const double* a_re;   // their real parts when every coefficient is real, else null
     const double* kd_re;
     int n_bits;
     int particle_cut;
     const uint64_t* ckeys;
-    const uint64_t* vals;
-    const uint32_t* starts;
+    const uint64_t* mvals;  // binned entries
+    const uint2* glist;
+    const CoreBins* bins;
     const int64_t* counts;
     const double2* in;
     double2* out;
@@ -1380,6 +1757,8 @@ struct SingleParams {
     double2* out2;
 };
 
+// Parity of the sites of c between r and p (core sites: the sign left when the table holds that of
+// r < p).
 template <int W>
 __device__ __forceinline__ int single_parity(const Cfg<W>& c, int r, int p) {
     return masked_parity<W>(c, range_mask<W>(r < p ? r : p, r < p ? p : r));
@@ -1435,302 +1814,130 @@ __device__ __forceinline__ double2 single_element(const SingleParams& p, const C
     return masked_row_sum<W, double2, CH>(p.kd + rq * p.n_bits, core, p.a[rq]);
 }
 
-// One wave, one group of order-1 entries [s, e): rows a (config = core + r) against entries b
-// (config = core + q), q != r:
-//   ADJ:  out[a] += conj(M_ba) in[b],  M_ba = (-1)^single_parity(c_a; r, q) (A[r][q] + sum_{k in core} K[r][q][k])
-//   !ADJ: out[a] += M_ab in[b],        M_ab = (-1)^single_parity(c_b; q, r) (A[q][r] + sum_{k in core} K[q][r][k])
-// s_raw: the group's start with its kGroupMixed bit (see pair_group).
-template <int W, bool ADJ, int NV, int CH>
-__device__ void single_group(const SingleParams& p, uint32_t s_raw, uint32_t e, int lane) {
-    const uint32_t s = s_raw & kGroupStart;
-    const bool mixed = (s_raw & kGroupMixed) != 0u;
-    const uint64_t v0 = p.vals[s];
-    const Cfg<W> core0 = entry_core<W, 1>(p.ckeys, v0);
-    const bool fermi = p.particle_cut == 1;
-    for (uint32_t a0 = s; a0 < e; a0 += 64) {
-        const uint32_t a = a0 + lane;
-        const bool act = a < e;
-        const uint64_t va = act ? p.vals[a] : v0;
-        const int64_t ia = static_cast<int64_t>(va >> 16);
-        const int r = static_cast<int>(va & 0xff);
-        const Cfg<W> core = mixed ? entry_core<W, 1>(p.ckeys, va) : core0;
-        Cfg<W> ca = core;
-        flip_site<W>(ca, r);
-        double acc_re[NV] = {}, acc_im[NV] = {};
-        for (uint32_t b0 = s; b0 < e; b0 += 64) {
-            const uint32_t bl = b0 + lane;
-            const bool bin = bl < e;
-            const uint64_t vbl = bin ? p.vals[bl] : 0ull;
-            const double2 gbl = bin ? p.in[vbl >> 16] : make_double2(0.0, 0.0);
-            const double2 gbl2 = (NV == 2 && bin) ? p.in2[vbl >> 16] : make_double2(0.0, 0.0);
-            const int nb = static_cast<int>(e - b0 < 64u ? e - b0 : 64u);
-            for (int u = 0; u < nb; ++u) {
-                const uint64_t vb = shfl_u64(vbl, u);
-                const double2 g = shfl_d2(gbl, u);
-                const double2 g2 = NV == 2 ? shfl_d2(gbl2, u) : make_double2(0.0, 0.0);
-                const int q = static_cast<int>(vb & 0xff);
-                bool ok = act && (b0 + static_cast<uint32_t>(u) != a) && q != r;
-                if (mixed && ok) {
-                    Cfg<W> cb = load_key<W>(p.ckeys, static_cast<int64_t>(vb >> 16));
-                    flip_site<W>(cb, q);
-#pragma unroll
-                    for (int w = 0; w < W; ++w) {
-                        ok = ok && cb.w[w] == core.w[w];
-                    }
-                }
-                if (!ok) {
-                    continue;
-                }
-                double2 x;
-                int sg;
-                if (ADJ) {
-                    x = single_element<W, CH>(p, core, r, q);
-                    sg = fermi ? single_parity<W>(ca, r, q) : 0;
-                } else {
-                    Cfg<W> cb = core;
-                    flip_site<W>(cb, q);
-                    x = single_element<W, CH>(p, core, q, r);
-                    sg = fermi ? single_parity<W>(cb, q, r) : 0;
-                }
-                const double xr = sg ? -x.x : x.x;
-                const double xi = sg ? -x.y : x.y;
-#pragma unroll
-                for (int v = 0; v < NV; ++v) {
-                    const double2 gg = v == 0 ? g : g2;
-                    if (ADJ) {
-                        acc_re[v] += xr * gg.x + xi * gg.y;
-                        acc_im[v] += xr * gg.y - xi * gg.x;
-                    } else {
-                        acc_re[v] += xr * gg.x - xi * gg.y;
-                        acc_im[v] += xr * gg.y + xi * gg.x;
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            if (act && (acc_re[v] != 0.0 || acc_im[v] != 0.0)) {
-                double2* o = v == 0 ? p.out : p.out2;
-                unsafeAtomicAdd(&o[ia].x, acc_re[v]);
-                unsafeAtomicAdd(&o[ia].y, acc_im[v]);
-            }
-        }
+// acc += x g (!ADJ) or conj(x) g (ADJ).
+template <bool ADJ>
+__device__ __forceinline__ void single_madd(const double2& x, const double2& g, double& re, double& im) {
+    if (ADJ) {
+        re += x.x * g.x + x.y * g.y;
+        im += x.x * g.y - x.y * g.x;
+    } else {
+        re += x.x * g.x - x.y * g.y;
+        im += x.x * g.y + x.y * g.x;
     }
 }
 
-// Single-excitation groups of 9..32 entries laid out by row_pass; a group's entries are its rows,
-// read from the lanes of the group by shuffles (as single_group reads its staged entries), so
-// several groups share a wave.
+// Order-1 groups: rows a (config = core + r) against entries b (config = core + q), the sign split into
+// one factor per entry (the core's sites below its site) and the table's part:
+//   ADJ:  out[a] += sign_a sum_b sign_b conj(M[r][q]) in[b],  M[r][q] = A[r][q] + sum_{k in core} K[r][q][k]
+//   !ADJ: out[a] += sign_a sum_b sign_b M[q][r] in[b]
+// Groups of g = 2..32 entries, lane = row, 64 / g groups to a pass; each row meets the other g - 1
+// entries in turn.
 template <int W, bool ADJ, int NV, int CH>
-__device__ void single_group_rows(const SingleParams& p, uint64_t mask, uint32_t gs_l, uint32_t ge_l, int lane) {
+__device__ __forceinline__ void single_rows(const SingleParams& p, int g, uint32_t e0, uint32_t e_end, int lane, Stage<NV>& st) {
     const bool fermi = p.particle_cut == 1;
-    while (mask) {
-        const RowLane f = row_pass(mask, gs_l, ge_l, lane);
-        const bool mixed = (f.s & kGroupMixed) != 0u;
-        const uint32_t s = f.s & kGroupStart;
-        const int g = static_cast<int>(f.e - s);  // 0 for a lane without a group
-        const int ri = lane - f.lead;
-        const bool act = ri < g;
-        const uint64_t va = act ? p.vals[s + static_cast<uint32_t>(ri)] : 0ull;
-        const int64_t ia = static_cast<int64_t>(va >> 16);
-        const int r = static_cast<int>(va & 0xff);
-        // the group's first row reads its config for the group (a mixed group: every row its own)
-        Cfg<W> own;
+    const int lanes = 64 / g * g;
+    const uint32_t at = e0 + static_cast<uint32_t>(lane);
+    const bool act = lane < lanes && at < e_end;
+    const int lead = act ? lane / g * g : 0;
+    const int ri = lane - lead;
+    const Entry e = binned_entry(act ? p.mvals[at] : 0ull, fermi);
+    // the group's first row reads its config for the group
+    Cfg<W> own;
 #pragma unroll
-        for (int w = 0; w < W; ++w) {
-            own.w[w] = act && (mixed || ri == 0) ? p.ckeys[ia * W + w] : 0ull;
-        }
-        if (act) {
-            flip_site<W>(own, r);
-        }
-        Cfg<W> core;
+    for (int w = 0; w < W; ++w) {
+        own.w[w] = act && ri == 0 ? p.ckeys[static_cast<int64_t>(e.row) * W + w] : 0ull;
+    }
+    if (act) {
+        flip_site<W>(own, static_cast<int>(e.slot));
+    }
+    stage_lane<NV>(p, st, lane, act, e, e.slot);
+    Cfg<W> core;
 #pragma unroll
-        for (int w = 0; w < W; ++w) {
-            const uint64_t c0 = shfl_u64(own.w[w], f.lead);  // every lane runs every shuffle
-            core.w[w] = mixed ? own.w[w] : c0;
-        }
-        // the exact per-pair check runs wave-wide when any group of the pass is mixed (a row of a
-        // group of one core holds its true core and passes it)
-        const bool wmixed = __ballot(mixed) != 0ull;
-        Cfg<W> ca = core;
-        flip_site<W>(ca, r);
-        const double2 gin = act ? p.in[ia] : make_double2(0.0, 0.0);
-        const double2 gin2 = (NV == 2 && act) ? p.in2[ia] : make_double2(0.0, 0.0);
-        double acc_re[NV] = {}, acc_im[NV] = {};
-        for (int u = 0; u < f.nmax; ++u) {
-            // lanes past the group belong to other groups or to no group: bounded by u < g
-            const int src = (f.lead + u) & 63;
-            const uint64_t vb = shfl_u64(va, src);
-            const double2 gb = shfl_d2(gin, src);
-            const double2 gb2 = NV == 2 ? shfl_d2(gin2, src) : make_double2(0.0, 0.0);
-            const int q = static_cast<int>(vb & 0xff);
-            bool ok = act && u < g && u != ri && q != r;
-            if (wmixed && ok) {
-                Cfg<W> cb = load_key<W>(p.ckeys, static_cast<int64_t>(vb >> 16));
-                flip_site<W>(cb, q);
-#pragma unroll
-                for (int w = 0; w < W; ++w) {
-                    ok = ok && cb.w[w] == core.w[w];
-                }
+    for (int w = 0; w < W; ++w) {
+        core.w[w] = shfl_u64(own.w[w], lead);  // every lane runs every shuffle
+    }
+    __builtin_amdgcn_wave_barrier();
+    double re[NV] = {}, im[NV] = {};
+    if (act) {
+        const int r = static_cast<int>(e.slot);
+        for (int u = 1; u < g; ++u) {
+            const int b = lead + (ri + u >= g ? ri + u - g : ri + u);
+            const int q = static_cast<int>(st.part[b]);
+            const double2 x = ADJ ? single_element<W, CH>(p, core, r, q) : single_element<W, CH>(p, core, q, r);
+            single_madd<ADJ>(x, st.g[b], re[0], im[0]);
+            if constexpr (NV == 2) {
+                single_madd<ADJ>(x, st.g2[b], re[1], im[1]);
             }
-            if (!ok) {
+        }
+    }
+    add_rows<NV>(p, st, 0, lane, act, e, re, im);
+}
+
+// One group of any size from mvals[s], lane = row.
+template <int W, bool ADJ, int NV, int CH>
+__device__ void single_group(const SingleParams& p, uint32_t s, uint32_t size, int lane, Stage<NV>& st) {
+    const bool fermi = p.particle_cut == 1;
+    const Entry first = binned_entry(p.mvals[s], fermi);
+    Cfg<W> core = load_key<W>(p.ckeys, static_cast<int64_t>(first.row));
+    flip_site<W>(core, static_cast<int>(first.slot));
+    for (uint32_t a0 = 0; a0 < size; a0 += 64) {
+        const bool act = a0 + lane < size;
+        const Entry e = binned_entry(p.mvals[s + (act ? a0 + lane : 0u)], fermi);
+        const int r = static_cast<int>(e.slot);
+        double re[NV] = {}, im[NV] = {};
+        for (uint32_t b = 0; b < size; ++b) {
+            const Entry eb = binned_entry(p.mvals[s + b], fermi);
+            const int q = static_cast<int>(eb.slot);
+            if (!act || q == r) {
                 continue;
             }
-            double2 x;
-            int sg;
-            if (ADJ) {
-                x = single_element<W, CH>(p, core, r, q);
-                sg = fermi ? single_parity<W>(ca, r, q) : 0;
-            } else {
-                Cfg<W> cb = core;
-                flip_site<W>(cb, q);
-                x = single_element<W, CH>(p, core, q, r);
-                sg = fermi ? single_parity<W>(cb, q, r) : 0;
-            }
-            const double xr = sg ? -x.x : x.x;
-            const double xi = sg ? -x.y : x.y;
-#pragma unroll
-            for (int v = 0; v < NV; ++v) {
-                const double2 gg = v == 0 ? gb : gb2;
-                if (ADJ) {
-                    acc_re[v] += xr * gg.x + xi * gg.y;
-                    acc_im[v] += xr * gg.y - xi * gg.x;
-                } else {
-                    acc_re[v] += xr * gg.x - xi * gg.y;
-                    acc_im[v] += xr * gg.y + xi * gg.x;
-                }
+            const double2 x = ADJ ? single_element<W, CH>(p, core, r, q) : single_element<W, CH>(p, core, q, r);
+            single_madd<ADJ>(x, signed_by(p.in[eb.row], eb.sign), re[0], im[0]);
+            if constexpr (NV == 2) {
+                single_madd<ADJ>(x, signed_by(p.in2[eb.row], eb.sign), re[1], im[1]);
             }
         }
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            if (act && (acc_re[v] != 0.0 || acc_im[v] != 0.0)) {
-                double2* o = v == 0 ? p.out : p.out2;
-                unsafeAtomicAdd(&o[ia].x, acc_re[v]);
-                unsafeAtomicAdd(&o[ia].y, acc_im[v]);
-            }
-        }
+        add_rows<NV>(p, st, 0, lane, act, e, re, im);
     }
 }
 
-// Single-excitation groups of 2..8 entries laid out by flat_pass, as pair_flat_class.
+// One work unit of the single bins.
 template <int W, bool ADJ, int NV, int CH>
-__device__ void single_flat_class(const SingleParams& p, uint64_t mask, uint32_t gs_l, uint32_t ge_l, int lane) {
-    const bool fermi = p.particle_cut == 1;
-    while (mask) {
-        const FlatLane f = flat_pass(mask, gs_l, ge_l, lane);
-        const bool mixed = (f.s & kGroupMixed) != 0u;
-        const uint32_t s = f.s & kGroupStart;
-        const bool act = f.e > s;
-        const uint64_t va = act ? p.vals[s + f.ai] : 0ull;
-        const uint64_t vb = act ? p.vals[s + f.bi] : 0ull;
-        const int64_t ia = static_cast<int64_t>(va >> 16);
-        const int r = static_cast<int>(va & 0xff);
-        const int q = static_cast<int>(vb & 0xff);
-        // the input row needs only the entry: loaded beside the stored configs (row 0 when unused)
-        const bool pre = act && q != r;
-        const int64_t ib = pre ? static_cast<int64_t>(vb >> 16) : 0;
-        double2 gv[NV];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            gv[v] = (v == 0 ? p.in : p.in2)[ib];
-        }
-        // the lanes of the group's first row read its config for the group (a mixed group: every
-        // row its own)
-        Cfg<W> own;
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            own.w[w] = act && (mixed || f.ai == 0) ? p.ckeys[ia * W + w] : 0ull;
-        }
-        if (act) {
-            flip_site<W>(own, r);
-        }
-        // every lane runs every shuffle (a short-circuit would leave lanes out)
-        Cfg<W> core;
-        bool same = true;
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            const uint64_t c0 = shfl_u64(own.w[w], f.lead);
-            core.w[w] = mixed ? own.w[w] : c0;
-            const bool eq = shfl_u64(own.w[w], f.rowb) == own.w[w];
-            same = same & eq;
-        }
-        const bool ok = pre && (same || !mixed);
-        double acc_re[NV] = {}, acc_im[NV] = {};
-        if (ok) {
-            double2 x;
-            int sg;
-            if (ADJ) {
-                Cfg<W> ca = core;
-                flip_site<W>(ca, r);
-                x = single_element<W, CH>(p, core, r, q);
-                sg = fermi ? single_parity<W>(ca, r, q) : 0;
-            } else {
-                Cfg<W> cb = core;
-                flip_site<W>(cb, q);
-                x = single_element<W, CH>(p, core, q, r);
-                sg = fermi ? single_parity<W>(cb, q, r) : 0;
-            }
-            const double xr = sg ? -x.x : x.x;
-            const double xi = sg ? -x.y : x.y;
-#pragma unroll
-            for (int v = 0; v < NV; ++v) {
-                if (ADJ) {
-                    acc_re[v] = xr * gv[v].x + xi * gv[v].y;
-                    acc_im[v] = xr * gv[v].y - xi * gv[v].x;
-                } else {
-                    acc_re[v] = xr * gv[v].x - xi * gv[v].y;
-                    acc_im[v] = xr * gv[v].y + xi * gv[v].x;
-                }
+__device__ __forceinline__ void single_unit(const SingleParams& p, uint32_t u, int lane, Stage<NV>& st) {
+    uint32_t local;
+    const int bin = unit_bin(p.bins, u, lane, &local);
+    if (bin < kExactBins) {
+        const int g = bin + 2;
+        const int passes = unit_passes(g, 1);
+        const uint32_t base = p.bins->entry_base[bin];
+        const uint32_t e_end = base + p.bins->groups[bin] * static_cast<uint32_t>(g);
+        const uint32_t step = static_cast<uint32_t>(64 / g * g);
+        for (int k = 0; k < passes; ++k) {
+            const uint32_t e0 = base + (local * static_cast<uint32_t>(passes) + static_cast<uint32_t>(k)) * step;
+            if (e0 < e_end) {  // wave-uniform
+                single_rows<W, ADJ, NV, CH>(p, g, e0, e_end, lane, st);
             }
         }
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            flat_row_sum(acc_re[v], acc_im[v], f.j, f.d);
-            if (f.j == 0 && act && (acc_re[v] != 0.0 || acc_im[v] != 0.0)) {
-                double2* o = v == 0 ? p.out : p.out2;
-                unsafeAtomicAdd(&o[ia].x, acc_re[v]);
-                unsafeAtomicAdd(&o[ia].y, acc_im[v]);
-            }
-        }
+        return;
     }
-}
-
-template <int W, bool ADJ, int NV, int CH, bool PACK = true>
-__device__ __forceinline__ void single_chunk(const SingleParams& p, int64_t groups, int64_t g0, int lane) {
-    const int64_t gg = g0 + lane;
-    uint32_t gs = 0, ge = 0;  // gs keeps the group's kGroupMixed bit for the group functions
-    if (gg < groups) {
-        gs = p.starts[gg];
-        ge = p.starts[gg + 1] & kGroupStart;
-    }
-    const uint32_t sz = ge - (gs & kGroupStart);
-    single_flat_class<W, ADJ, NV, CH>(p, __ballot(sz >= 2u && sz <= 8u), gs, ge, lane);
-    // PACK: groups of 9..32 entries several to a wave (else one group per wave)
-    if (PACK) {
-        single_group_rows<W, ADJ, NV, CH>(p, __ballot(sz > 8u && sz <= 32u), gs, ge, lane);
-    }
-    uint64_t big = __ballot(sz > (PACK ? 32u : 8u));
-    while (big) {
-        const int l = __builtin_ctzll(big);
-        big &= big - 1;
-        single_group<W, ADJ, NV, CH>(p, __shfl(gs, l), __shfl(ge, l), lane);
-    }
+    for_listed(p, bin, local, lane, [&](uint32_t s, uint32_t size) { single_group<W, ADJ, NV, CH>(p, s, size, lane, st); });
 }
 
 template <int W, bool ADJ, int NV = 1>
 __global__ __launch_bounds__(kBlock) void single_kernel(SingleParams p) {
+    __shared__ Stage<NV> stages[kWavesPerBlock];
     const int lane = threadIdx.x & 63;
-    const int64_t wave = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) >> 6;
-    const int64_t nwaves = (static_cast<int64_t>(gridDim.x) * kBlock) >> 6;
+    const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6))));
+    const uint32_t nwaves = gridDim.x * kWavesPerBlock;
     if (p.counts[2] != 0) {
         if (wave == 0 && lane == 0) {
             mark_overflow(p.out);
         }
         return;
     }
-    const int64_t groups = p.counts[1];
-    for (int64_t g0 = wave * 64; g0 < groups; g0 += nwaves * 64) {
-        single_chunk<W, ADJ, NV, kSingleLoads>(p, groups, g0, lane);
+    const uint32_t units = p.bins->unit_start[kBins];
+    for (uint32_t u = wave; u < units; u += nwaves) {
+        single_unit<W, ADJ, NV, kSingleLoads>(p, u, lane, stages[threadIdx.x >> 6]);
     }
 }
 
@@ -1937,9 +2144,9 @@ struct HopParams {
 // out over the lanes, one (row, entry) per lane per round, so their elements and coefficient loads
 // run side by side; each row's sum collects in LDS and is added to out[a] without atomics (each row
 // has one entry).
-//   ADJ:  out[a] += conj(M_ba) in[b],  M_ba = (-1)^single_parity(c_a; r, q) (A[r][q] + sum_{k in core} K[r][q][k])
-//   !ADJ: out[a] += M_ab in[b],        M_ab = (-1)^single_parity(c_b; q, r) (A[q][r] + sum_{k in core} K[q][r][k])
-// with r the site of a, q the site of b (c_a = core + r, c_b = core + q), as in single_group.
+//   ADJ:  out[a] += conj(M_ba) in[b],  M_ba = (-1)^single_parity(core; r, q) (A[r][q] + sum_{k in core} K[r][q][k])
+//   !ADJ: out[a] += M_ab in[b],        M_ab = (-1)^single_parity(core; q, r) (A[q][r] + sum_{k in core} K[q][r][k])
+// with r the site of a, q the site of b (c_a = core + r, c_b = core + q), as in single_rows.
 constexpr int kHopList = 256;  // connections listed per round, per wave
 
 template <int W>
@@ -2119,9 +2326,7 @@ __global__ __launch_bounds__(kBlock) void hop_kernel(HopParams p) {
                     }
                     Cfg<W> core = cx;
                     flip_site<W>(core, r);
-                    Cfg<W> cb = core;
-                    flip_site<W>(cb, q);
-                    const int sg = fermi ? (ADJ ? single_parity<W>(cx, r, q) : single_parity<W>(cb, q, r)) : 0;
+                    const int sg = fermi ? single_parity<W>(core, r, q) : 0;
                     double2 x;
                     if (plain) {
                         const int64_t rq = ADJ ? static_cast<int64_t>(r) * p.s.n_bits + q : static_cast<int64_t>(q) * p.s.n_bits + r;
@@ -2249,15 +2454,17 @@ struct BatchItemDev {
     const double2* pcoef;
     const double* pcoef_re;
     int64_t n_pairs;
-    const uint64_t* pvals;
-    const uint32_t* pstarts;
+    const uint64_t* pmvals;
+    const uint2* pglist;
+    const CoreBins* pbins;
     const int64_t* pcounts;
     const double2* sa;
     const double2* skd;
     const double* sa_re;
     const double* skd_re;
-    const uint64_t* svals;
-    const uint32_t* sstarts;
+    const uint64_t* smvals;
+    const uint2* sglist;
+    const CoreBins* sbins;
     const int64_t* scounts;
     const double2* in;
     double2* out;
@@ -2288,27 +2495,29 @@ __device__ void diag_rows(const BatchItemDev& it, int64_t r0, int lane) {
 }
 
 // PART 1: the pair units (type 0); PART 2: the single-excitation (type 1) and diagonal (type 2)
-// units.  Both pack the groups of 9..32 entries several to a wave.
+// units.
 template <int W, bool ADJ, int NV, int PART>
-__device__ void batch_unit(const BatchItemDev& it, int type, int64_t local, int lane, char* stage) {
+__device__ void batch_unit(const BatchItemDev& it, int type, int64_t local, int lane, Stage<NV>& stage) {
     if (PART == 1 && type == 0) {
         PairParams p{};
         p.coef = it.pcoef;
         p.coef_re = it.pcoef_re;
         p.n_pairs = it.n_pairs;
-        p.n_bits = it.n_bits;
         p.particle_cut = it.particle_cut;
-        p.ckeys = it.ckeys;
-        p.vals = it.pvals;
-        p.starts = it.pstarts;
+        p.mvals = it.pmvals;
+        p.glist = it.pglist;
+        p.bins = it.pbins;
         p.counts = it.pcounts;
         p.in = it.in;
         p.out = it.out;
         p.in2 = it.in2;
         p.out2 = it.out2;
-        const int64_t groups = it.pcounts[1];
-        if (local * 64 < groups && it.pcounts[2] == 0) {
-            pair_chunk<W, ADJ, kPairBatchInBatch, NV, true>(p, groups, local * 64, lane, stage);
+        if (it.pcounts[2] == 0) {
+            if (p.coef_re != nullptr) {
+                pair_unit<ADJ, true, NV, kPairBatch / 2>(p, static_cast<uint32_t>(local), lane, stage);
+            } else {
+                pair_unit<ADJ, false, NV, kPairBatch / 2>(p, static_cast<uint32_t>(local), lane, stage);
+            }
         }
     } else if (PART == 2 && type == 1) {
         SingleParams p{};
@@ -2319,16 +2528,16 @@ __device__ void batch_unit(const BatchItemDev& it, int type, int64_t local, int 
         p.n_bits = it.n_bits;
         p.particle_cut = it.particle_cut;
         p.ckeys = it.ckeys;
-        p.vals = it.svals;
-        p.starts = it.sstarts;
+        p.mvals = it.smvals;
+        p.glist = it.sglist;
+        p.bins = it.sbins;
         p.counts = it.scounts;
         p.in = it.in;
         p.out = it.out;
         p.in2 = it.in2;
         p.out2 = it.out2;
-        const int64_t groups = it.scounts[1];
-        if (local * 64 < groups && it.scounts[2] == 0) {
-            single_chunk<W, ADJ, NV, 4, true>(p, groups, local * 64, lane);
+        if (it.scounts[2] == 0) {
+            single_unit<W, ADJ, NV, 4>(p, static_cast<uint32_t>(local), lane, stage);
         }
     } else if (PART == 2 && type == 2) {
         diag_rows<W, ADJ, NV>(it, local * 64, lane);
@@ -2353,7 +2562,8 @@ __global__ __launch_bounds__(kBlock, 4) void batch_kernel(const BatchItemDev* __
     const int lane = threadIdx.x & 63;
     const int64_t wave = xcd_wave();
     const int64_t nwaves = (static_cast<int64_t>(gridDim.x) * kBlock) >> 6;
-    __shared__ __align__(16) char stage[kPairStageBytes];
+    __shared__ Stage<NV> stages[kWavesPerBlock];
+    Stage<NV>& stage = stages[threadIdx.x >> 6];
     const int slots = 3 * n_items;
     const int64_t first = PART == 2 ? offsets[n_items] : 0;
     const int64_t last = PART == 1 ? offsets[n_items] : total;
@@ -2371,7 +2581,7 @@ __global__ __launch_bounds__(kBlock, 4) void batch_kernel(const BatchItemDev* __
         const int type = lo / n_items;
         const BatchItemDev& it = items[lo - type * n_items];
         const int64_t local = u - offsets[lo];
-        if (it.n_words == 1) {
+        if (PART == 1 || it.n_words == 1) {  // the pair units take any width
             batch_unit<1, ADJ, NV, PART>(it, type, local, lane, stage);
         } else {
             batch_unit<2, ADJ, NV, PART>(it, type, local, lane, stage);
@@ -2452,6 +2662,38 @@ size_t cores_bytes(int n_qubytes, int64_t n, int max_occupied, int order) {
     return cores_layout(cv, n_qubytes, n, max_occupied, order, nullptr, nullptr, nullptr) == QMB_OK ? cv.off : 0;
 }
 
+namespace {
+
+int cores_build_small(const qmb_targets* targets, int order, void* scratch, qmb_cores* c, hipStream_t stream) {
+    Carver sc{static_cast<char*>(scratch), 0};
+    const size_t cap = static_cast<size_t>(c->capacity);
+    c->mvals = sc.take<uint64_t>(cap);
+    c->glist = sc.take<uint64_t>(cap);
+    c->key_bits = kKeyBits;
+    auto* glist = reinterpret_cast<uint2*>(c->glist);
+    auto go = [&](auto kernel) -> int {
+        QMB_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        static_cast<int>(sizeof(SmallLds))));
+        kernel<<<1, kSmallThreads, sizeof(SmallLds), stream>>>(targets->keys, targets->cols, static_cast<int>(c->n), 8 * c->n_qubytes,
+                                                               c->per_config, c->keys, c->vals, c->starts, c->counts,
+                                                               static_cast<CoreBins*>(c->bins), c->mvals, glist, glist + cap / 2);
+        QMB_CHECK_LAUNCH();
+        return QMB_OK;
+    };
+    switch (c->n_words * 2 + (order - 1)) {
+        case 2: return go(&cores_small_kernel<1, 1>);
+        case 3: return go(&cores_small_kernel<1, 2>);
+        case 4: return go(&cores_small_kernel<2, 1>);
+        case 5: return go(&cores_small_kernel<2, 2>);
+        case 6: return go(&cores_small_kernel<3, 1>);
+        case 7: return go(&cores_small_kernel<3, 2>);
+        case 8: return go(&cores_small_kernel<4, 1>);
+        default: return go(&cores_small_kernel<4, 2>);
+    }
+}
+
+}  // namespace
+
 int cores_build(const qmb_targets* targets, int max_occupied, int order, void* buffer, size_t bytes, qmb_cores* out,
                 hipStream_t stream) {
     if (!targets) {
@@ -2466,19 +2708,25 @@ int cores_build(const qmb_targets* targets, int max_occupied, int order, void* b
         return set_error(QMB_ERR_WORKSPACE, "core index buffer too small: need %zu bytes, have %zu", cv.off, bytes);
     }
     c.bytes = bytes;
-    zero_counts_kernel<<<1, 64, 0, stream>>>(c.counts);
-    QMB_CHECK_LAUNCH();
-    if (c.capacity > 0) {
+    if (c.capacity == 0) {
+        cores_init_kernel<<<1, 64, 0, stream>>>(c.counts, 0, nullptr);
+        QMB_CHECK_LAUNCH();
+    } else if (c.capacity <= kSmallCores) {
+        QMB_TRY(cores_build_small(targets, order, scratch, &c, stream));
+    } else {
         const size_t cap = static_cast<size_t>(c.capacity);
         Carver sc{static_cast<char*>(scratch), 0};
         // a u64 per entry: the emitted keys (u32) or, packed, the emitted entries
         uint64_t* entries_in = sc.take<uint64_t>(cap);
         uint32_t* keys_in = reinterpret_cast<uint32_t*>(entries_in);
         uint64_t* vals_in = sc.take<uint64_t>(cap);
-        uint32_t* flag = sc.take<uint32_t>(cap);
+        uint8_t* flag = sc.take<uint8_t>(cap);
         const int64_t chunks = flag_chunks(c.capacity);
         uint32_t* chunk_heads = sc.take<uint32_t>(static_cast<size_t>(chunks));
         uint32_t* chunk_off = sc.take<uint32_t>(static_cast<size_t>(chunks));
+        const int64_t nblk = bin_blocks(c.capacity);
+        uint32_t* bin_hist = sc.take<uint32_t>(static_cast<size_t>(kBinRows * nblk + 1));
+        uint32_t* bin_scan = sc.take<uint32_t>(static_cast<size_t>(kBinRows * nblk + 1));
         const int n_bits = 8 * c.n_qubytes;
         uint32_t* inv = sc.take<uint32_t>(static_cast<size_t>(n_bits) * n_bits / 2);
         size_t tmp_bytes = scratch_bytes > sc.off + 512 ? scratch_bytes - sc.off - 512 : 0;
@@ -2493,6 +2741,9 @@ int cores_build(const qmb_targets* targets, int max_occupied, int order, void* b
                                               packed ? static_cast<void*>(entries_in) : static_cast<void*>(vals_in), c.counts);
         };
         const int shape = c.n_words * 2 + (order - 1);
+        cores_init_kernel<<<blocks_for(static_cast<int64_t>(n_bits) * n_bits), kBlock, 0, stream>>>(c.counts, n_bits,
+                                                                                                  packed && order == 2 ? inv : nullptr);
+        QMB_CHECK_LAUNCH();
         if (packed) {
             switch (shape) {
                 case 2: emit(&core_emit_kernel<1, 1, true>); break;
@@ -2521,13 +2772,8 @@ int cores_build(const qmb_targets* targets, int max_occupied, int order, void* b
         if (packed) {
             QMB_HIP_TRY(rocprim::radix_sort_keys(tmp, need, entries_in, vals_in, static_cast<unsigned>(cap), kPackedBits,
                                                  kPackedBits + kKeyBits, stream));
-            if (order == 2) {
-                pair_inverse_kernel<<<blocks_for(static_cast<int64_t>(n_bits) * n_bits), kBlock, 0, stream>>>(n_bits, inv);
-                QMB_CHECK_LAUNCH();
-            }
             auto unpack = [&](auto kernel) {
-                kernel<<<blocks_for(c.capacity, kBlock * kFlagUnroll), kBlock, 0, stream>>>(vals_in, c.capacity, flag, chunk_heads, sub_bits,
-                                                                                         inv, targets->keys, c.keys, c.vals, c.counts);
+                kernel<<<blocks_for(c.capacity, kBlock * kFlagUnroll), kBlock, 0, stream>>>(vals_in, c.capacity, flag, chunk_heads, sub_bits,                                                                                         inv, targets->keys, c.keys, c.vals, c.counts);
             };
             switch (shape) {
                 case 2: unpack(&core_flag_unpack_kernel<1, 1>); break;
@@ -2558,17 +2804,78 @@ int cores_build(const qmb_targets* targets, int max_occupied, int order, void* b
             }
         }
         QMB_CHECK_LAUNCH();
-        need = tmp_bytes;
-        QMB_HIP_TRY(rocprim::exclusive_scan(tmp, need, chunk_heads, chunk_off, 0u, static_cast<size_t>(chunks), rocprim::plus<uint32_t>(),
-                                            stream));
+        if (chunks <= kBlockScanMax) {
+            block_scan_kernel<<<1, kBlock, 0, stream>>>(chunk_heads, chunk_off, chunks);
+            QMB_CHECK_LAUNCH();
+        } else {
+            need = tmp_bytes;
+            QMB_HIP_TRY(rocprim::exclusive_scan(tmp, need, chunk_heads, chunk_off, 0u, static_cast<size_t>(chunks),
+                                                rocprim::plus<uint32_t>(), stream));
+        }
         // one wave per flag chunk, as the flag kernel
         core_start_kernel<<<blocks_for(c.capacity, kBlock * kFlagUnroll), kBlock, 0, stream>>>(flag, chunk_off, c.starts, c.counts);
         c.key_bits = kKeyBits;
+        QMB_CHECK_LAUNCH();
+        // the binned entries and the group list take the place of the sort's buffers, which are no
+        // longer read: at most cap / 2 list slots (a slot stands for two or more entries), and as many
+        // noted mixed groups behind them
+        c.mvals = entries_in;
+        c.glist = vals_in;
+        auto* bins = static_cast<CoreBins*>(c.bins);
+        const bool one_block = kBinRows * nblk + 1 <= kBlockScanMax;
+        bin_count_kernel<<<static_cast<unsigned>(nblk), kBlock, 0, stream>>>(c.starts, c.counts, nblk, bin_groups(c.capacity), bin_hist);
+        QMB_CHECK_LAUNCH();
+        if (!one_block) {
+            need = tmp_bytes;
+            QMB_HIP_TRY(rocprim::exclusive_scan(tmp, need, bin_hist, bin_scan, 0u, static_cast<size_t>(kBinRows * nblk + 1),
+                                                rocprim::plus<uint32_t>(), stream));
+        }
+        bin_table_kernel<<<1, kBlock, 0, stream>>>(one_block ? bin_hist : nullptr, bin_scan, nblk, order, bins);
+        QMB_CHECK_LAUNCH();
+        auto* glist = reinterpret_cast<uint2*>(c.glist);
+        auto* msplit = glist + cap / 2;
+        auto scatter = [&](auto kernel) {
+            kernel<<<static_cast<unsigned>(nblk), kBlock, 0, stream>>>(c.starts, c.counts, flag, c.vals, targets->keys, bin_scan, nblk,
+                                                                       bin_groups(c.capacity), n_bits, bins, c.mvals, glist, msplit);
+        };
+        switch (shape) {
+            case 2: scatter(&bin_scatter_kernel<1, 1>); break;
+            case 3: scatter(&bin_scatter_kernel<1, 2>); break;
+            case 4: scatter(&bin_scatter_kernel<2, 1>); break;
+            case 5: scatter(&bin_scatter_kernel<2, 2>); break;
+            case 6: scatter(&bin_scatter_kernel<3, 1>); break;
+            case 7: scatter(&bin_scatter_kernel<3, 2>); break;
+            case 8: scatter(&bin_scatter_kernel<4, 1>); break;
+            default: scatter(&bin_scatter_kernel<4, 2>); break;
+        }
         QMB_CHECK_LAUNCH();
     }
     *out = c;
     return QMB_OK;
 }
+
+namespace {
+
+// Persistent waves of a group kernel: enough to fill every CU several times over, never more than the
+// entries can need (small sets: a wave per 32 entries).
+unsigned group_grid(int64_t capacity) {
+    const int64_t want = capacity / (32 * kWavesPerBlock) + 1;
+    return static_cast<unsigned>(want < 4096 ? want : 4096);
+}
+
+template <int NV>
+int launch_pairs(const PairParams& p, int64_t capacity, int mode, hipStream_t stream) {
+    const unsigned grid = group_grid(capacity);
+    if (p.coef_re != nullptr) {
+        mode == 1 ? pair_kernel<true, true, NV><<<grid, kBlock, 0, stream>>>(p) : pair_kernel<false, true, NV><<<grid, kBlock, 0, stream>>>(p);
+    } else {
+        mode == 1 ? pair_kernel<true, false, NV><<<grid, kBlock, 0, stream>>>(p) : pair_kernel<false, false, NV><<<grid, kBlock, 0, stream>>>(p);
+    }
+    QMB_CHECK_LAUNCH();
+    return QMB_OK;
+}
+
+}  // namespace
 
 int apply_pairs(const qmb_pairs* pairs, const qmb_cores* cores, const qmb_targets* targets, const double* in, double* out,
                 int mode, hipStream_t stream) {
@@ -2591,29 +2898,17 @@ int apply_pairs(const qmb_pairs* pairs, const qmb_cores* cores, const qmb_target
     p.coef = reinterpret_cast<const double2*>(pairs->coef);
     p.coef_re = pairs->real ? pairs->coef_re : nullptr;
     p.n_pairs = pairs->n_pairs;
-    p.n_bits = pairs->n_bits;
     p.particle_cut = pairs->particle_cut;
-    p.ckeys = targets->keys;
-    p.vals = cores->vals;
-    p.starts = cores->starts;
+    p.mvals = cores->mvals;
+    p.glist = reinterpret_cast<const uint2*>(cores->glist);
+    p.bins = static_cast<const CoreBins*>(cores->bins);
     p.counts = cores->counts;
     p.in = reinterpret_cast<const double2*>(in);
     p.out = reinterpret_cast<double2*>(out);
-    // persistent waves: enough to fill every CU several times over, never more than the groups need
-    const int64_t want = (cores->capacity + 64 * 4 - 1) / (64 * 4);
-    const unsigned grid = static_cast<unsigned>(want < 4096 ? (want < 1 ? 1 : want) : 4096);
-    auto go = [&](auto kernel) -> int {
-        kernel<<<grid, kBlock, 0, stream>>>(p);
-        QMB_CHECK_LAUNCH();
-        return QMB_OK;
-    };
-    if (cores->n_words == 1) {
-        return mode == 1 ? go(&pair_kernel<1, true>) : go(&pair_kernel<1, false>);
+    if (cores->n_words > 2) {
+        return set_error(QMB_ERR_UNSUPPORTED, "pair path supports n_qubytes <= %d", kMaxPairBytes);
     }
-    if (cores->n_words == 2) {
-        return mode == 1 ? go(&pair_kernel<2, true>) : go(&pair_kernel<2, false>);
-    }
-    return set_error(QMB_ERR_UNSUPPORTED, "pair path supports n_qubytes <= %d", kMaxPairBytes);
+    return launch_pairs<1>(p, cores->capacity, mode, stream);
 }
 
 size_t singles_bytes(int n_qubytes) {
@@ -2674,13 +2969,13 @@ int apply_singles(const qmb_singles* singles, const qmb_cores* cores, const qmb_
     p.n_bits = singles->n_bits;
     p.particle_cut = singles->particle_cut;
     p.ckeys = targets->keys;
-    p.vals = cores->vals;
-    p.starts = cores->starts;
+    p.mvals = cores->mvals;
+    p.glist = reinterpret_cast<const uint2*>(cores->glist);
+    p.bins = static_cast<const CoreBins*>(cores->bins);
     p.counts = cores->counts;
     p.in = reinterpret_cast<const double2*>(in);
     p.out = reinterpret_cast<double2*>(out);
-    const int64_t want = (cores->capacity + 64 * 4 - 1) / (64 * 4);
-    const unsigned grid = static_cast<unsigned>(want < 4096 ? (want < 1 ? 1 : want) : 4096);
+    const unsigned grid = group_grid(cores->capacity);
     auto go = [&](auto kernel) -> int {
         kernel<<<grid, kBlock, 0, stream>>>(p);
         QMB_CHECK_LAUNCH();
@@ -2948,15 +3243,15 @@ int apply_structured_dual(const qmb_pairs* pairs, const qmb_singles* singles, co
         p.n_bits = singles->n_bits;
         p.particle_cut = singles->particle_cut;
         p.ckeys = targets->keys;
-        p.vals = cores1->vals;
-        p.starts = cores1->starts;
+        p.mvals = cores1->mvals;
+        p.glist = reinterpret_cast<const uint2*>(cores1->glist);
+        p.bins = static_cast<const CoreBins*>(cores1->bins);
         p.counts = cores1->counts;
         p.in = vi;
         p.out = vo;
         p.in2 = vi2;
         p.out2 = vo2;
-        const int64_t want = (cores1->capacity + 64 * 4 - 1) / (64 * 4);
-        const unsigned grid = static_cast<unsigned>(want < 4096 ? (want < 1 ? 1 : want) : 4096);
+        const unsigned grid = group_grid(cores1->capacity);
         if (W == 1) {
             mode == 1 ? single_kernel<1, true, 2><<<grid, kBlock, 0, stream>>>(p) : single_kernel<1, false, 2><<<grid, kBlock, 0, stream>>>(p);
         } else {
@@ -2969,24 +3264,16 @@ int apply_structured_dual(const qmb_pairs* pairs, const qmb_singles* singles, co
         p.coef = reinterpret_cast<const double2*>(pairs->coef);
         p.coef_re = pairs->real ? pairs->coef_re : nullptr;
         p.n_pairs = pairs->n_pairs;
-        p.n_bits = pairs->n_bits;
         p.particle_cut = pairs->particle_cut;
-        p.ckeys = targets->keys;
-        p.vals = cores2->vals;
-        p.starts = cores2->starts;
+        p.mvals = cores2->mvals;
+        p.glist = reinterpret_cast<const uint2*>(cores2->glist);
+        p.bins = static_cast<const CoreBins*>(cores2->bins);
         p.counts = cores2->counts;
         p.in = vi;
         p.out = vo;
         p.in2 = vi2;
         p.out2 = vo2;
-        const int64_t want = (cores2->capacity + 64 * 4 - 1) / (64 * 4);
-        const unsigned grid = static_cast<unsigned>(want < 4096 ? (want < 1 ? 1 : want) : 4096);
-        if (W == 1) {
-            mode == 1 ? pair_kernel<1, true, 2><<<grid, kBlock, 0, stream>>>(p) : pair_kernel<1, false, 2><<<grid, kBlock, 0, stream>>>(p);
-        } else {
-            mode == 1 ? pair_kernel<2, true, 2><<<grid, kBlock, 0, stream>>>(p) : pair_kernel<2, false, 2><<<grid, kBlock, 0, stream>>>(p);
-        }
-        QMB_CHECK_LAUNCH();
+        QMB_TRY(launch_pairs<2>(p, cores2->capacity, mode, stream));
     }
     return QMB_OK;
 }
@@ -3023,6 +3310,7 @@ int batch_plan(const qmb_batch_item* items, int n_items, void* buffer, size_t by
     std::vector<BatchItemDev> dev(static_cast<size_t>(n_items));
     int dual = 0;
     std::vector<int64_t> units(3 * static_cast<size_t>(n_items), 0);
+    std::vector<uint32_t> device_units(2 * static_cast<size_t>(n_items), 0u);  // units of the core indexes' bins
     for (int k = 0; k < n_items; ++k) {
         const qmb_batch_item& x = items[k];
         if (!x.pairs || !x.targets) {
@@ -3051,10 +3339,10 @@ int batch_plan(const qmb_batch_item* items, int n_items, void* buffer, size_t by
             d.pcoef = reinterpret_cast<const double2*>(x.pairs->coef);
             d.pcoef_re = x.pairs->real ? x.pairs->coef_re : nullptr;
             d.n_pairs = x.pairs->n_pairs;
-            d.pvals = x.cores2->vals;
-            d.pstarts = x.cores2->starts;
+            d.pmvals = x.cores2->mvals;
+            d.pglist = reinterpret_cast<const uint2*>(x.cores2->glist);
+            d.pbins = static_cast<const CoreBins*>(x.cores2->bins);
             d.pcounts = x.cores2->counts;
-            units[k] = (x.cores2->capacity + 63) / 64;
         }
         if (x.singles) {
             d.has_singles = 1;
@@ -3062,10 +3350,10 @@ int batch_plan(const qmb_batch_item* items, int n_items, void* buffer, size_t by
             d.skd = reinterpret_cast<const double2*>(x.singles->kd);
             d.sa_re = x.singles->real ? x.singles->a_re : nullptr;
             d.skd_re = x.singles->real ? x.singles->kd_re : nullptr;
-            d.svals = x.cores1->vals;
-            d.sstarts = x.cores1->starts;
+            d.smvals = x.cores1->mvals;
+            d.sglist = reinterpret_cast<const uint2*>(x.cores1->glist);
+            d.sbins = static_cast<const CoreBins*>(x.cores1->bins);
             d.scounts = x.cores1->counts;
-            units[n_items + k] = (x.cores1->capacity + 63) / 64;
         }
         units[2 * n_items + k] = (tg.n + 63) / 64;
         d.in = reinterpret_cast<const double2*>(x.in);
@@ -3078,6 +3366,19 @@ int batch_plan(const qmb_batch_item* items, int n_items, void* buffer, size_t by
         }
         dual = two;
         dev[static_cast<size_t>(k)] = d;
+    }
+    for (int k = 0; k < n_items; ++k) {
+        const BatchItemDev& d = dev[static_cast<size_t>(k)];
+        if (items[k].cores2->capacity > 0) {
+            QMB_HIP_TRY(hipMemcpyAsync(&device_units[k], &d.pbins->unit_start[kBins], sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
+        }
+        if (items[k].singles && items[k].cores1->capacity > 0) {
+            QMB_HIP_TRY(hipMemcpyAsync(&device_units[n_items + k], &d.sbins->unit_start[kBins], sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
+        }
+    }
+    QMB_HIP_TRY(hipStreamSynchronize(stream));
+    for (size_t q = 0; q < device_units.size(); ++q) {
+        units[q] = static_cast<int64_t>(device_units[q]);
     }
     std::vector<int64_t> offsets(units.size() + 1, 0);
     for (size_t q = 0; q < units.size(); ++q) {

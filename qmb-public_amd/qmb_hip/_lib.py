@@ -124,6 +124,9 @@ class QmbCores(ctypes.Structure):
         ("vals", _vp),
         ("starts", _vp),
         ("counts", _vp),
+        ("mvals", _vp),
+        ("glist", _vp),
+        ("bins", _vp),
     ]
 
 

@@ -338,3 +338,48 @@ def test_merged_core_groups(cuda_device: torch.device, name: str, pc: int, case_
     scale = np.abs(ref).sum(axis=1) + np.abs(c).sum(axis=1).max() * np.abs(psi).sum()
     assert np.all(np.abs(got_a - ref).max(axis=1) <= 1e-12 * scale), (name, bits)
 
+
+
+@pytest.mark.parametrize("bits", [0, 4])
+@pytest.mark.parametrize("n", [1, 2, 60, 182, 183, 1000, 3000])
+def test_core_index_builds_around_the_one_block_limit(cuda_device: torch.device, n: int, bits: int) -> None:
+    """Sets of 10 electrons (45 entries a row) on both sides of the 8192 entries that one block indexes
+    (182 rows: 8190) and of the radix sort's lower limit (1000 rows: 45,000; 3000: 135,000), with the
+    set's hash and with 4-bit hash columns (nearly every group mixed): the sorted index equals one
+    made on the host, and both modes equal the oracle and the enumeration."""
+    s, k, c = sorted_terms(*sy.molecular_terms(10, 31))
+    cfg = sy.sector_configs(10, 5, 5, n, 32)
+    cfg_t = _dev(cfg, cuda_device)
+    terms = pp.PreparedTerms(_dev(s, cuda_device), _dev(k, cuda_device), _dev(c, cuda_device), 3, 1)
+    targets = pp.PreparedTargets(cfg_t, 3, distinct=True)
+    if bits:
+        _build_cores_with_narrow_hash(targets, bits, 90 + bits)
+    occupied = np.nonzero(np.unpackbits(cfg, axis=1, bitorder="little"))[1].reshape(n, 10)
+    for order in (2, 1):
+        vals, starts, counts = _core_index(targets, order)
+        per = 45 if order == 2 else 10
+        assert counts.tolist()[:3] == [n * per, len(starts) - 1, 0]
+        removed = [(a, b) for b in range(10) for a in range(b)] if order == 2 else [(a,) for a in range(10)]
+        cores: dict[tuple[int, ...], set[int]] = {}
+        for row, sites in enumerate(occupied.tolist()):
+            for pick in removed:
+                value = (row << 16) | (sites[pick[-1]] << 8 | sites[pick[0]] if order == 2 else sites[pick[0]])
+                cores.setdefault(tuple(x for i, x in enumerate(sites) if i not in pick), set()).add(value)
+        st = (starts & 0x7FFFFFFF).astype(np.int64)
+        groups = [set(vals[a:b].tolist()) for a, b in zip(st[:-1], st[1:])]
+        assert sum(len(g) for g in groups) == n * per
+        where = {v: g for g, members in enumerate(groups) for v in members}
+        held = [set() for _ in groups]  # the cores of each group
+        for core, members in cores.items():
+            (g,) = {where[v] for v in members}
+            held[g].add(core)
+        assert [len(h) > 1 for h in held] == (starts[:-1] >> 31).astype(bool).tolist()
+    psi, g = sy.random_psi(n, 33), sy.random_psi(n, 34)
+    want, asum, _ = orc.apply_within(1, cfg, psi, cfg, s, k, c)
+    vec = torch.view_as_real(_dev(psi, cuda_device)).contiguous()
+    got = pp.apply(terms, targets, cfg_t, vec, pp.MODE_FORWARD, symmetric=pp.SYMMETRIC_OFF, pairs=True).cpu().numpy()
+    assert np.all(np.abs(got[:, 0] + 1j * got[:, 1] - want) <= 1e-12 * asum + 1e-300)
+    gvec = torch.view_as_real(_dev(g, cuda_device)).contiguous()
+    ref, rsum, _ = orc.apply_within(1, cfg, g, cfg, s, k, c)  # the table is Hermitian
+    got = pp.apply(terms, targets, cfg_t, gvec, pp.MODE_ADJOINT, symmetric=pp.SYMMETRIC_OFF, pairs=True).cpu().numpy()
+    assert np.all(np.abs(got[:, 0] + 1j * got[:, 1] - ref) <= 1e-12 * rsum + 1e-300)
