@@ -196,7 +196,8 @@ typedef struct qmb_targets {
     uint64_t* table;   /* [capacity] (index << 32 | fingerprint) or ~0 */
     uint64_t* filter;  /* [filter_words] */
     uint64_t* cols;    /* [256] hash column per site: H(config) = XOR of cols over occupied sites */
-    int64_t* duplicates; /* device: number of rows equal to an earlier row */
+    int64_t* duplicates; /* device: {number of rows equal to an earlier row (by _index), the most occupied sites
+                            of a row (by _keys)} */
 } qmb_targets;
 
 int qmb_targets_workspace_size(int n_qubytes, int64_t n, size_t* bytes);

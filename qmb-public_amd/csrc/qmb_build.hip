@@ -140,37 +140,64 @@ __global__ void orig_records_kernel(const int16_t* __restrict__ site, const uint
 }
 
 // ------------------------------------------------------------------------------ targets ------
+// The key words, and *occupied raised to the most occupied sites of a row.  A grid-stride pass over at
+// most kKeysBlocks blocks with one atomic each: with a block per 256 rows every wave in flight raised
+// the same counter (250,000 rows: 30 us, of which 25 for that).
+constexpr unsigned kKeysBlocks = 1024;
+
 template <int W>
-__global__ void keys_kernel(const uint8_t* __restrict__ configs, int64_t n, int nq, uint64_t* __restrict__ keys) {
-    int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (i >= n) {
-        return;
-    }
-    const uint8_t* row = configs + i * nq;
-    uint64_t w[W];
-#pragma unroll
-    for (int k = 0; k < W; ++k) {
-        w[k] = 0;
-    }
-    for (int b = 0; b < nq; ++b) {
-        const uint64_t byte = row[b];
+__global__ __launch_bounds__(kBlock) void keys_kernel(const uint8_t* __restrict__ configs, int64_t n, int nq, uint64_t* __restrict__ keys,
+                                                      int64_t* __restrict__ occupied) {
+    __shared__ int s_occ[kBlock / 64];
+    int most = 0;
+    for (int64_t i = blockIdx.x * static_cast<int64_t>(kBlock) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * kBlock) {
+        const uint8_t* row = configs + i * nq;
+        uint64_t w[W];
 #pragma unroll
         for (int k = 0; k < W; ++k) {
-            if (k == (b >> 3)) {
-                w[k] |= byte << (8 * (b & 7));
+            w[k] = 0;
+        }
+        for (int b = 0; b < nq; ++b) {
+            const uint64_t byte = row[b];
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+                if (k == (b >> 3)) {
+                    w[k] |= byte << (8 * (b & 7));
+                }
             }
         }
-    }
+        int occ = 0;
 #pragma unroll
-    for (int k = 0; k < W; ++k) {
-        keys[i * W + k] = w[k];
+        for (int k = 0; k < W; ++k) {
+            keys[i * W + k] = w[k];
+            occ += __popcll(w[k]);
+        }
+        most = occ > most ? occ : most;
+    }
+    for (int d = 32; d > 0; d >>= 1) {
+        const int o = __shfl_xor(most, d);
+        most = o > most ? o : most;
+    }
+    if ((threadIdx.x & 63) == 0) {
+        s_occ[threadIdx.x >> 6] = most;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int v = 1; v < kBlock / 64; ++v) {
+            most = s_occ[v] > most ? s_occ[v] : most;
+        }
+        atomicMax(reinterpret_cast<unsigned long long*>(occupied), static_cast<unsigned long long>(most));
     }
 }
 
-__global__ void hash_columns_kernel(uint64_t* __restrict__ cols, int n) {
+// The hash columns, and occupied = 0 for the key kernel after it.
+__global__ void hash_columns_kernel(uint64_t* __restrict__ cols, int n, int64_t* __restrict__ occupied) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b < n) {
         cols[b] = hash_column(b);
+    }
+    if (b == 0 && occupied != nullptr) {
+        *occupied = 0;
     }
 }
 
@@ -249,20 +276,21 @@ __global__ void gather_be_kernel(const uint64_t* __restrict__ keys, const uint32
 }
 
 template <int W>
-int keys_launch(const uint8_t* configs, int64_t n, int nq, uint64_t* keys, hipStream_t stream) {
+int keys_launch(const uint8_t* configs, int64_t n, int nq, uint64_t* keys, int64_t* occupied, hipStream_t stream) {
     if (n > 0) {
-        keys_kernel<W><<<blocks_for(n), kBlock, 0, stream>>>(configs, n, nq, keys);
+        const unsigned blocks = blocks_for(n);
+        keys_kernel<W><<<blocks < kKeysBlocks ? blocks : kKeysBlocks, kBlock, 0, stream>>>(configs, n, nq, keys, occupied);
         QMB_CHECK_LAUNCH();
     }
     return QMB_OK;
 }
 
-int keys_dispatch(int W, const uint8_t* configs, int64_t n, int nq, uint64_t* keys, hipStream_t stream) {
+int keys_dispatch(int W, const uint8_t* configs, int64_t n, int nq, uint64_t* keys, int64_t* occupied, hipStream_t stream) {
     switch (W) {
-        case 1: return keys_launch<1>(configs, n, nq, keys, stream);
-        case 2: return keys_launch<2>(configs, n, nq, keys, stream);
-        case 3: return keys_launch<3>(configs, n, nq, keys, stream);
-        default: return keys_launch<4>(configs, n, nq, keys, stream);
+        case 1: return keys_launch<1>(configs, n, nq, keys, occupied, stream);
+        case 2: return keys_launch<2>(configs, n, nq, keys, occupied, stream);
+        case 3: return keys_launch<3>(configs, n, nq, keys, occupied, stream);
+        default: return keys_launch<4>(configs, n, nq, keys, occupied, stream);
     }
 }
 
@@ -456,7 +484,7 @@ int targets_layout(Carver& cv, int n_qubytes, int64_t n, qmb_targets* out) {
     t.table = cv.take<uint64_t>(t.capacity);
     t.filter = cv.take<uint64_t>(t.filter_words);
     t.cols = cv.take<uint64_t>(64 * kMaxWords);
-    t.duplicates = cv.take<int64_t>(1);
+    t.duplicates = cv.take<int64_t>(2);
     t.bytes = cv.off;
     if (out) {
         *out = t;
@@ -473,9 +501,9 @@ int targets_build_keys(int n_qubytes, const uint8_t* configs, int64_t n, void* b
         return set_error(QMB_ERR_WORKSPACE, "target buffer too small: need %zu bytes, have %zu", cv.off, bytes);
     }
     t.bytes = bytes;
-    QMB_TRY(keys_dispatch(t.n_words, configs, n, n_qubytes, t.keys, stream));
-    hash_columns_kernel<<<1, 64 * kMaxWords, 0, stream>>>(t.cols, 64 * kMaxWords);
+    hash_columns_kernel<<<1, 64 * kMaxWords, 0, stream>>>(t.cols, 64 * kMaxWords, t.duplicates + 1);
     QMB_CHECK_LAUNCH();
+    QMB_TRY(keys_dispatch(t.n_words, configs, n, n_qubytes, t.keys, t.duplicates + 1, stream));
     *out = t;
     return QMB_OK;
 }
@@ -506,6 +534,7 @@ size_t sort_configs_scratch_bytes(int n_words, int64_t n) {
     cv.take<uint64_t>(N);            // word in
     cv.take<uint64_t>(N);            // word out
     cv.take<uint32_t>(N);            // perm in
+    cv.take<int64_t>(1);             // most occupied row (unused)
     cv.take_bytes(sort_bytes);
     return cv.off + 256;
 }
@@ -522,13 +551,15 @@ int sort_configs(int n_qubytes, const uint8_t* configs, int64_t n, uint64_t* key
     uint64_t* win = cv.take<uint64_t>(N);
     uint64_t* wout = cv.take<uint64_t>(N);
     uint32_t* pin = cv.take<uint32_t>(N);
+    int64_t* occupied = cv.take<int64_t>(1);
     size_t sort_bytes = 0;
     (void)rocprim::radix_sort_pairs(nullptr, sort_bytes, win, wout, pin, perm, static_cast<unsigned>(N));
     void* tmp = cv.take_bytes(sort_bytes);
     if (cv.off > scratch_bytes) {
         return set_error(QMB_ERR_WORKSPACE, "sort scratch too small: need %zu, have %zu", cv.off, scratch_bytes);
     }
-    QMB_TRY(keys_dispatch(W, configs, n, n_qubytes, raw, stream));
+    QMB_TRY(launch_fill_u64(reinterpret_cast<uint64_t*>(occupied), 0ull, 1, stream));
+    QMB_TRY(keys_dispatch(W, configs, n, n_qubytes, raw, occupied, stream));
     iota_kernel<<<blocks_for(n), kBlock, 0, stream>>>(perm, n);
     QMB_CHECK_LAUNCH();
     // LSD over words: least significant word (last) first; each pass is a stable radix sort.

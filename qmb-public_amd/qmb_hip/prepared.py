@@ -246,9 +246,17 @@ class PreparedTargets:
     def duplicates(self) -> int:
         """Rows equal to an earlier row (synchronises once)."""
         if self._duplicates is None:
-            offset = int(self.desc.duplicates) - self.buffer.data_ptr()
-            self._duplicates = int(self.buffer[offset:offset + 8].view(torch.int64).item())
+            duplicates, occupied = self._counters(self.desc)
+            self._duplicates = duplicates
+            if self._max_occupied is None:
+                self._max_occupied = occupied  # in the same read-back
         return self._duplicates
+
+    def _counters(self, desc: _lib.QmbTargets) -> tuple[int, int]:
+        """(rows equal to an earlier row, valid once indexed; the most occupied sites of a row)."""
+        offset = int(desc.duplicates) - self.buffer.data_ptr()
+        duplicates, occupied = self.buffer[offset:offset + 16].view(torch.int64).tolist()
+        return int(duplicates), int(occupied)
 
     def indexes(self, configs: torch.Tensor) -> bool:
         """True when `configs` is the very tensor this index was built over."""
@@ -257,11 +265,7 @@ class PreparedTargets:
     def max_occupied(self) -> int:
         """Largest number of occupied sites in a row (synchronises unless given at construction)."""
         if self._max_occupied is None:
-            if self.n == 0:
-                self._max_occupied = 0
-            else:
-                table = torch.tensor([bin(v).count("1") for v in range(256)], dtype=torch.int32, device=self.device)
-                self._max_occupied = int(table[self.configs.long()].sum(dim=1).max().item())
+            self._max_occupied = self._counters(self.keys_desc)[1]
         return self._max_occupied
 
     def has_cores(self, order: int) -> bool:
