@@ -83,8 +83,16 @@ __device__ __forceinline__ int64_t lookup(const uint64_t* __restrict__ table, ui
 //                            before the barrier that precedes the first post(); acc is the tile's
 //                            LDS accumulator row per config (double2[C]);
 //   tile_end(i0, nc, acc)    every thread, after the barrier that follows the last post();
-//   direct_end(i, valid)     the direct enumeration's thread for config i, after its last post().
+//   direct_end(i, valid)     the direct enumeration's thread for config i, after its last post();
+//   kPruned, tile_bound(i0), drop(t, bound)
+//                            kPruned: within a bucket the terms come in an order in which drop(t, bound)
+//                            stays true once it is, and a dropped term's connections from the tile's
+//                            rows are not wanted.  Each bucket is then cut at its first dropped term, and
+//                            a bucket without terms left costs nothing (find_relative).
 struct ActionHooks {
+    static constexpr bool kPruned = false;
+    __device__ __forceinline__ double tile_bound(int64_t) const { return 0.0; }
+    __device__ __forceinline__ bool drop(uint32_t, double) const { return false; }
     __device__ __forceinline__ void tile_begin(int64_t, int, double2*) {}
     __device__ __forceinline__ void tile_end(int64_t, int, double2*) {}
     __device__ __forceinline__ void direct_end(int64_t, bool) {}
@@ -291,6 +299,7 @@ template <int W, typename Action>
 __device__ void enumerate_tile(const EnumSource& p, const HashIndex& ix, int64_t tile, int tile_log2, int g, int groups, uint64_t* smem,
                                Action& act) {
     __shared__ int s_count;
+    __shared__ uint32_t s_cut[Action::kPruned ? kEnumBlock : 1];
     const int C = 1 << tile_log2;
     const int CW = C >> 6;
     const EnumLds L = carve_lds<W>(smem, tile_log2, p.n_bits);
@@ -344,9 +353,34 @@ __device__ void enumerate_tile(const EnumSource& p, const HashIndex& ix, int64_t
 
     const int64_t single_end = 1 + p.n_bits;
     const int64_t residual = p.n_buckets - 1;
-    for (int64_t b = g; b < p.n_buckets; b += groups) {
+    const double bound = Action::kPruned ? act.tile_bound(i0) : 0.0;
+    int nth = 0;  // of this group's buckets; the cuts of kEnumBlock of them are in s_cut at a time
+    for (int64_t b = g; b < p.n_buckets; b += groups, ++nth) {
         const uint32_t ts = p.bucket_start[b];
-        const uint32_t te = p.bucket_start[b + 1];
+        uint32_t te = p.bucket_start[b + 1];
+        if (Action::kPruned) {
+            if (nth % kEnumBlock == 0) {
+                // a thread per bucket: its first dropped term by bisection
+                __syncthreads();
+                const int64_t mine = b + static_cast<int64_t>(tid) * groups;
+                uint32_t lo = 0, hi = 0;
+                if (mine < p.n_buckets) {
+                    lo = p.bucket_start[mine];
+                    hi = p.bucket_start[mine + 1];
+                    while (lo < hi) {
+                        const uint32_t mid = (lo + hi) >> 1;
+                        if (act.drop(mid, bound)) {
+                            hi = mid;
+                        } else {
+                            lo = mid + 1;
+                        }
+                    }
+                }
+                s_cut[tid] = lo;
+                __syncthreads();
+            }
+            te = s_cut[nth % kEnumBlock];
+        }
         if (ts == te) {
             continue;  // uniform across the workgroup
         }

@@ -5,23 +5,24 @@
 // on the GPU by per-node spin locks with racy pre-reads (qmb/_hamiltonian_cuda.cu:276-427); then it
 // drops zero weights and returns the distinct configs sorted by bytes (:537-545).
 //
-// Here the K largest contributions are found without locks.  Positive doubles order like their bit
-// patterns, so the K-th largest weight is located digit by digit (12-bit digits of the weight bits):
-// every pass re-runs the enumeration and histograms the next digit of the entries still tied with
-// the threshold, and a single-thread kernel picks the digit at which the running count reaches K.
-// Once the tied class fits the candidate buffer, one more pass collects every entry strictly above
-// the threshold prefix and the tied candidates; the candidates are ordered by (weight desc, config
-// asc) and the first K - above are kept.  All control lives in device memory, so the whole call is
-// enqueued without host synchronisation.
+// Here the K largest contributions are found without locks, and without looking at most of them.  A
+// contribution's weight is at most (|coef| |psi|)^2, so the rows are first put in descending |psi| and
+// the terms of every bucket in descending |coef|: the contributions that can reach a weight are then a
+// prefix of every bucket's terms for a prefix of the rows, and nothing else is enumerated.  (At 52 spin
+// orbitals and 1M rows, K = 100,000, enumerating and weighing all 2.9e10 connections took 64 ms of a
+// 73.9 ms call; the whole call takes 4.6 ms this way, 1.9 of them in the digit passes and 1.7 in the
+// collecting pass.  At 20 spin orbitals and 10,000 rows, K = 1000: 1.76 -> 0.62 ms.)
 //
-// Large selections first try a sampled threshold, which needs one full pass instead of three: the
-// contributions of an evenly spaced sample of n_s rows (with their exclusion lookups) are sorted,
-// and the sample weights at ranks f K -+ 6 sqrt(f K) (f = n_s / n_i) bracket the K-th weight of the
-// whole set with overwhelming probability.  One pass then collects every entry above the upper
-// bound and every entry between the bounds as candidates.  The result is exact when fewer than K
-// entries lie above and at least K lie above the lower bound, which the device checks; otherwise
-// the state is reset and the digit-by-digit passes run as before.  Either way the candidates are
-// finished by the same sort, so ties resolve identically.
+// Positive doubles order like their bit patterns, so the K-th largest weight is located digit by digit
+// (12-bit digits of the weight bits): every pass histograms the next digit of the entries tied with the
+// threshold so far, and a one-block kernel picks the digit at which the running count reaches K.  The
+// first digit's pass needs a lower bound to be a prefix: it starts from the power of four whose
+// products |coef| |psi| (counted from exponent histograms of the two) number some 64 K, and is repeated
+// at 16 times as many while it finds fewer than K entries (most connections do not exist or are
+// excluded).  Once the tied class fits the candidate buffer, one more pass collects every entry strictly
+// above the threshold prefix and the tied candidates; the candidates are ordered by (weight desc,
+// config asc) and the first K - above are kept.  All control lives in device memory, so the whole call
+// is enqueued without host synchronisation; passes that are not needed return at once.
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 
@@ -43,24 +44,40 @@ inline unsigned blocks_for(int64_t n, int block = 256) {
     return static_cast<unsigned>(b < 1 ? 1 : b);
 }
 
+constexpr int kTries = 6;  // lower bounds of the first digit's pass; the last is the least weight
+
 struct FrState {
     int64_t k_rem;
     uint64_t prefix;
     int32_t level;
-    int32_t shift;
+    int32_t tries;  // bounds tried at level 0
     int32_t done;
-    int32_t all;
+    int32_t reserved;
     unsigned long long n_above;
     unsigned long long n_cand;
     int64_t cand_needed;
-    uint64_t lo;   // collect: candidates are lo <= w < hi, entries with w >= hi are selected outright
-    uint64_t hi;
-    unsigned long long n_sample;
-    int32_t fast_try;   // the sampled bounds are set
-    int32_t collected;  // a collect pass produced the final selection
-    int32_t failed;     // the sampled attempt did not bracket the K-th weight
-    int32_t reserved;
+    uint64_t lo;     // entries with w < lo are not wanted; collect: candidates are lo <= w < hi,
+    uint64_t hi;     // entries with w >= hi are selected outright
+    double reach;    // |coef| |psi| of an entry with w >= lo is not below this
+    int64_t active;  // rows that can reach it: a prefix
+    uint64_t bound[kTries];
 };
+
+// Reach of the weight with these bits: no product |coef| |psi| below it gives that weight.  The computed
+// weight is within a few roundings of (|coef| |psi|)^2, except at the ends of the range: a product whose
+// square overflows (or is NaN) is at least about the root of the largest finite weight, and each square
+// of a denormal weight may be rounded up to it.
+__device__ __forceinline__ double reach_of(uint64_t lo) {
+    constexpr uint64_t kLargest = 0x7fefffffffffffffull;
+    const double root = sqrt(__longlong_as_double(static_cast<long long>(lo < kLargest ? lo : kLargest)));
+    return root * (lo < (64ull << 52) ? 0.5 : 1.0 - 1e-9);
+}
+
+// Rows and terms are ordered by the high word of the bits of |psi| and |coef| (20 bits of mantissa), so
+// a later one is at most this factor above an earlier one.  NaN orders first and drops nothing.
+constexpr double kOrderSlack = 1.0 + 2e-6;
+
+__device__ __forceinline__ bool below_reach(double a, double b, double reach) { return a * b < reach; }
 
 struct FrParams {
     EnumSource src;
@@ -72,13 +89,12 @@ struct FrParams {
     const uint64_t* xfilter;
     uint64_t xfmask;
     const uint64_t* xcols;
+    const double* aw;  // |coef| per term, descending within each bucket (times kOrderSlack)
     FrState* state;
     unsigned long long* hist;
     uint64_t* sel_c;   // [K][W] selected configs ("above" entries, then the kept candidates)
     uint64_t* cand_w;  // [cap]
     uint64_t* cand_c;  // [cap][W]
-    uint64_t* sample_w;  // [sample_cap] weights of the sampled rows' contributions
-    int64_t sample_cap;
     int64_t k;
     int64_t cand_cap;
     int tile_log2;
@@ -95,19 +111,29 @@ __device__ __forceinline__ uint64_t weight_bits(const double2 cf, const double2 
     return static_cast<uint64_t>(__double_as_longlong(w));
 }
 
-template <int W>
-struct HistAction : ActionHooks {
+// The pruning both passes share: terms whose |coef| with the tile's largest |psi| stays below the reach.
+struct PrunedHooks : ActionHooks {
+    static constexpr bool kPruned = true;
     const FrParams& p;
+    double reach;
+    __device__ explicit PrunedHooks(const FrParams& pp) : p(pp), reach(pp.state->reach) {}
+    __device__ __forceinline__ double tile_bound(int64_t i0) const { return hypot(p.psi[i0].x, p.psi[i0].y) * kOrderSlack; }
+    __device__ __forceinline__ bool drop(uint32_t t, double bound) const { return below_reach(p.aw[t], bound, reach); }
+};
+
+template <int W>
+struct HistAction : PrunedHooks {
     uint32_t* hist;
     uint64_t prefix;
+    uint64_t lo;
     int shift;
     int width;
     __device__ HistAction(const FrParams& pp, uint32_t* h, uint64_t pre_, int sh, int wd)
-        : p(pp), hist(h), prefix(pre_), shift(sh), width(wd) {}
+        : PrunedHooks(pp), hist(h), prefix(pre_), lo(pp.state->lo), shift(sh), width(wd) {}
     // Only entries still tied with the threshold prefix need the (costly) exclusion lookup.
     __device__ __forceinline__ bool pre(int64_t i, uint32_t t, const Cfg<W>&, int, uint64_t, uint64_t) {
         const uint64_t w = weight_bits(p.coefs[t], p.psi[i]);
-        return w != 0 && (w >> (shift + width)) == prefix;
+        return w >= lo && (w >> (shift + width)) == prefix;
     }
     __device__ __forceinline__ void post(int64_t i, uint32_t t, const Cfg<W>&, int, int64_t j, bool) {
         if (j >= 0) {
@@ -118,53 +144,13 @@ struct HistAction : ActionHooks {
     }
 };
 
-// Appends to a device counter from the active lanes with one atomic per wave: returns this lane's slot.
-__device__ __forceinline__ unsigned long long wave_append(unsigned long long* counter) {
-    const uint64_t active = __ballot(1);
-    const int leader = __ffsll(static_cast<long long>(active)) - 1;
-    const int lane = static_cast<int>(threadIdx.x & 63);
-    unsigned long long base = 0;
-    if (lane == leader) {
-        base = atomicAdd(counter, static_cast<unsigned long long>(__popcll(active)));
-    }
-    base = __shfl(base, leader);
-    return base + static_cast<unsigned long long>(__popcll(active & ((1ull << lane) - 1ull)));
-}
-
-__device__ __forceinline__ bool sample_full(const FrParams& p) {
-    return *reinterpret_cast<const volatile unsigned long long*>(&p.state->n_sample) > static_cast<unsigned long long>(p.sample_cap);
-}
-
-// The sampled rows' contributions: every nonzero weight whose target is not excluded.  Threads
-// that start after the buffer has overflowed (the attempt is then abandoned) skip their lookups.
 template <int W>
-struct SampleAction : ActionHooks {
-    const FrParams& p;
-    bool full;
-    __device__ explicit SampleAction(const FrParams& pp) : p(pp), full(sample_full(pp)) {}
-    __device__ __forceinline__ bool pre(int64_t i, uint32_t t, const Cfg<W>&, int, uint64_t, uint64_t) {
-        return !full && weight_bits(p.coefs[t], p.psi[i]) != 0;
-    }
-    __device__ __forceinline__ void post(int64_t i, uint32_t t, const Cfg<W>&, int, int64_t j, bool) {
-        if (j >= 0) {
-            return;  // excluded
-        }
-        const unsigned long long s = wave_append(&p.state->n_sample);
-        if (s < static_cast<unsigned long long>(p.sample_cap)) {
-            p.sample_w[s] = weight_bits(p.coefs[t], p.psi[i]);
-        }
-    }
-};
-
-template <int W>
-struct CollectAction : ActionHooks {
-    const FrParams& p;
+struct CollectAction : PrunedHooks {
     uint64_t lo;
     uint64_t hi;
-    __device__ CollectAction(const FrParams& pp, uint64_t lo_, uint64_t hi_) : p(pp), lo(lo_), hi(hi_) {}
+    __device__ explicit CollectAction(const FrParams& pp) : PrunedHooks(pp), lo(pp.state->lo), hi(pp.state->hi) {}
     __device__ __forceinline__ bool pre(int64_t i, uint32_t t, const Cfg<W>&, int, uint64_t, uint64_t) {
-        const uint64_t w = weight_bits(p.coefs[t], p.psi[i]);
-        return w != 0 && w >= lo;
+        return weight_bits(p.coefs[t], p.psi[i]) >= lo;
     }
     __device__ __forceinline__ void post(int64_t i, uint32_t t, const Cfg<W>& o, int, int64_t j, bool) {
         if (j >= 0) {
@@ -192,13 +178,24 @@ struct CollectAction : ActionHooks {
     }
 };
 
+// The connections of the rows that can reach the bound, the (tile, bucket group) units dealt over the
+// grid's work-groups.
 template <int W, typename Action>
 __device__ __forceinline__ void fr_enumerate(const FrParams& p, uint64_t* smem, Action& act) {
     const HashIndex ix{p.xtable, p.xkeys, p.xmask, p.xfilter, p.xfmask, p.xcols, false};
+    EnumSource src = p.src;
+    src.n_i = p.state->active;
     if (p.direct) {
-        enumerate_direct<W>(p.src, ix, blockIdx.x, *reinterpret_cast<DirectLds<W>*>(smem), act);
+        const int64_t blocks = (src.n_i + kEnumBlock - 1) / kEnumBlock;
+        for (int64_t b = blockIdx.x; b < blocks; b += gridDim.x) {
+            enumerate_direct<W>(src, ix, b, *reinterpret_cast<DirectLds<W>*>(smem), act);
+        }
     } else {
-        enumerate_tile<W>(p.src, ix, blockIdx.x / p.groups, p.tile_log2, blockIdx.x % p.groups, p.groups, smem, act);
+        const int64_t units = ((src.n_i + (1ll << p.tile_log2) - 1) >> p.tile_log2) * p.groups;
+        for (int64_t u = blockIdx.x; u < units; u += gridDim.x) {
+            enumerate_tile<W>(src, ix, u / p.groups, p.tile_log2, static_cast<int>(u % p.groups), p.groups, smem, act);
+            __syncthreads();  // the next unit reuses the tile's LDS
+        }
     }
 }
 
@@ -227,158 +224,304 @@ __global__ __launch_bounds__(kEnumBlock) void fr_hist_kernel(FrParams p) {
     }
 }
 
-// phase 0: the sampled attempt (runs when its bounds are set); phase 1: the digit-by-digit result
-// (runs unless the sampled attempt already produced the selection).
 template <int W>
-__global__ __launch_bounds__(kEnumBlock) void fr_collect_kernel(FrParams p, int phase) {
+__global__ __launch_bounds__(kEnumBlock) void fr_collect_kernel(FrParams p) {
     extern __shared__ uint64_t smem[];
-    if (p.state->collected || (phase == 0 && !p.state->fast_try)) {
-        return;  // uniform: every thread reads the same flags
-    }
-    CollectAction<W> act(p, p.state->lo, p.state->hi);
+    CollectAction<W> act(p);
     fr_enumerate<W>(p, smem, act);
 }
 
-template <int W>
-__global__ __launch_bounds__(kEnumBlock) void fr_sample_kernel(FrParams p) {
-    extern __shared__ uint64_t smem[];
-    SampleAction<W> act(p);
-    fr_enumerate<W>(p, smem, act);
-}
-
-// Bounds from the sorted (descending) sample weights; single thread.
-__global__ void fr_bounds_kernel(FrState* st, const uint64_t* __restrict__ sorted, int64_t sample_cap, double fraction, int64_t k) {
-    if (threadIdx.x != 0) {
-        return;
-    }
-    st->fast_try = 0;
-    if (st->n_sample > static_cast<unsigned long long>(sample_cap)) {
-        return;  // the sample overflowed its buffer: take the exact passes
-    }
-    const int64_t count = static_cast<int64_t>(st->n_sample);
-    const double e = fraction * static_cast<double>(k);
-    const double sd = sqrt(e);
-    const int64_t k_hi = static_cast<int64_t>(floor(e - 6.0 * sd)) - 1;
-    const int64_t k_lo = static_cast<int64_t>(ceil(e + 6.0 * sd)) + 1;
-    st->hi = k_hi < 0 ? ~0ull : (k_hi < count ? sorted[k_hi] + 1ull : 1ull);
-    st->lo = k_lo < count ? sorted[k_lo] : 1ull;
-    if (st->lo < 1ull) {
-        st->lo = 1ull;
-    }
-    if (st->hi < st->lo) {
-        st->hi = st->lo;
-    }
-    st->fast_try = 1;
-}
-
-// Accepts the sampled attempt when the bounds bracket the K-th weight, else resets for the exact
-// passes; single thread.
-__global__ void fr_verify_kernel(FrState* st, int64_t k, int64_t cand_cap) {
-    if (threadIdx.x != 0 || !st->fast_try) {
-        return;
-    }
-    const unsigned long long kk = static_cast<unsigned long long>(k);
-    // lo = 1 collects every nonzero entry, so fewer than K of them is a complete selection too
-    const bool reached = st->n_above + st->n_cand >= kk || st->lo <= 1ull;
-    if (st->n_above < kk && reached && st->n_cand <= static_cast<unsigned long long>(cand_cap)) {
-        st->collected = 1;
-        st->done = 1;
-        st->cand_needed = static_cast<int64_t>(kk - st->n_above);
-    } else {
-        st->failed = 1;
-        st->n_above = 0;
-        st->n_cand = 0;
-    }
-}
-
-// After a failed sampled attempt the candidate buffer must start empty again.
-__global__ void fr_clear_failed_kernel(const FrState* __restrict__ st, uint64_t* __restrict__ cand_w, int64_t cap) {
+// Sort keys of the rows: the high word of |psi|'s bits.
+__global__ void fr_row_keys_kernel(const double2* __restrict__ psi, int64_t n, uint32_t* __restrict__ keys, uint32_t* __restrict__ idx) {
     const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (i < cap && st->failed) {
-        cand_w[i] = 0ull;
+    if (i < n) {
+        keys[i] = static_cast<uint32_t>(static_cast<uint64_t>(__double_as_longlong(hypot(psi[i].x, psi[i].y))) >> 32);
+        idx[i] = static_cast<uint32_t>(i);
     }
 }
 
-// Every sample-th row of configs_i and psi_i, compacted.
-__global__ void fr_gather_sample_kernel(const uint8_t* __restrict__ configs, const double2* __restrict__ psi, int64_t n_i, int nq,
-                                        int64_t n_s, uint8_t* __restrict__ sample_configs, double2* __restrict__ sample_psi) {
-    const int64_t j = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (j >= n_s) {
-        return;
+__global__ void fr_row_gather_kernel(const uint32_t* __restrict__ order, const uint8_t* __restrict__ configs, const double2* __restrict__ psi,
+                                     int64_t n, int nq, uint8_t* __restrict__ out_configs, double2* __restrict__ out_psi) {
+    const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+    if (i < n) {
+        const int64_t r = order[i];
+        for (int b = 0; b < nq; ++b) {
+            out_configs[i * nq + b] = configs[r * nq + b];
+        }
+        out_psi[i] = psi[r];
     }
-    const int64_t r = j * n_i / n_s;
-    for (int b = 0; b < nq; ++b) {
-        sample_configs[j * nq + b] = configs[r * nq + b];
-    }
-    sample_psi[j] = psi[r];
 }
 
-__global__ void fr_init_kernel(FrState* st, unsigned long long* hist, int64_t k) {
+// Sort keys of the terms (in bucket order): bucket, then descending |coef|.  Terms that never succeed
+// stay behind the last bucket.
+__global__ void fr_term_keys_kernel(const double2* __restrict__ coefs, const uint32_t* __restrict__ bucket_start, int64_t n_buckets,
+                                    int64_t n_terms, uint64_t* __restrict__ keys, uint32_t* __restrict__ idx) {
+    const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+    if (t < n_terms) {
+        int64_t lo = 0, hi = n_buckets;  // last bucket starting at or before t
+        while (lo < hi) {
+            const int64_t mid = (lo + hi + 1) >> 1;
+            if (bucket_start[mid] <= t) {
+                lo = mid;
+            } else {
+                hi = mid - 1;
+            }
+        }
+        const uint64_t bits = static_cast<uint64_t>(__double_as_longlong(hypot(coefs[t].x, coefs[t].y)));
+        keys[t] = (static_cast<uint64_t>(lo) << 32) | static_cast<uint32_t>(~(bits >> 32));
+        idx[t] = static_cast<uint32_t>(t);
+    }
+}
+
+__global__ void fr_term_gather_kernel(const uint32_t* __restrict__ order, const uint64_t* __restrict__ recs, const double2* __restrict__ coefs,
+                                      int64_t n_terms, uint64_t* __restrict__ out_recs, double2* __restrict__ out_coefs,
+                                      double* __restrict__ aw) {
+    const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+    if (t < n_terms) {
+        const uint32_t o = order[t];
+        const double2 c = coefs[o];
+        out_recs[t] = recs[o];
+        out_coefs[t] = c;
+        aw[t] = hypot(c.x, c.y) * kOrderSlack;
+    }
+}
+
+// The exponent histogram of |v| and the largest |v| (as its bits: NaN above everything).
+struct FrExponents {
+    uint32_t count[2048];
+    unsigned long long most;
+};
+
+__global__ __launch_bounds__(256) void fr_exponents_kernel(const double2* __restrict__ v, int64_t n, FrExponents* __restrict__ exps) {
+    __shared__ uint32_t s_exp[2048];
+    unsigned long long most = 0ull;
+    for (int b = threadIdx.x; b < 2048; b += 256) {
+        s_exp[b] = 0u;
+    }
+    __syncthreads();
+    for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += gridDim.x * 256ll) {
+        const unsigned long long a = static_cast<unsigned long long>(__double_as_longlong(hypot(v[i].x, v[i].y)));
+        atomicAdd(&s_exp[(a >> 52) & 0x7ffu], 1u);
+        most = a > most ? a : most;
+    }
+    for (int d = 32; d > 0; d >>= 1) {
+        const unsigned long long o = __shfl_xor(most, d);
+        most = o > most ? o : most;
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicMax(&exps->most, most);
+    }
+    __syncthreads();
+    for (int b = threadIdx.x; b < 2048; b += 256) {
+        if (s_exp[b] != 0u) {
+            atomicAdd(&exps->count[b], s_exp[b]);
+        }
+    }
+}
+
+// exps: of the rows, then of the terms.
+__global__ void fr_init_kernel(FrState* st, unsigned long long* hist, FrExponents* exps, int64_t k) {
     for (int b = threadIdx.x; b < kHistBins; b += blockDim.x) {
         hist[b] = 0;
+        exps[b >> 11].count[b & 2047] = 0;
     }
     if (threadIdx.x == 0) {
+        exps[0].most = 0;
+        exps[1].most = 0;
+        *st = FrState{};
         st->k_rem = k;
-        st->prefix = 0;
-        st->level = 0;
-        st->shift = 0;
-        st->done = 0;
-        st->all = 0;
-        st->n_above = 0;
-        st->n_cand = 0;
-        st->cand_needed = 0;
         st->lo = 1;
         st->hi = 1;
-        st->n_sample = 0;
-        st->fast_try = 0;
-        st->collected = 0;
-        st->failed = 0;
-        st->reserved = 0;
     }
 }
 
-// Chooses the threshold digit of the current level (single thread; 4096 bins).
-__global__ void fr_select_kernel(FrState* st, unsigned long long* hist, int64_t cand_cap) {
-    if (threadIdx.x != 0 || st->done) {
-        return;
+// Rows (in descending |psi|) that can reach `reach` with the largest |coef|.
+__device__ int64_t fr_active(const double2* __restrict__ psi, int64_t n, double amax, double reach) {
+    int64_t lo = 0, hi = n;
+    while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (below_reach(amax, hypot(psi[mid].x, psi[mid].y) * kOrderSlack, reach)) {
+            hi = mid;
+        } else {
+            lo = mid + 1;
+        }
+    }
+    return lo;
+}
+
+__device__ void fr_set_lo(FrState* st, uint64_t lo, const double2* __restrict__ psi, int64_t n, double amax) {
+    st->lo = lo < 1ull ? 1ull : lo;
+    st->reach = reach_of(st->lo);
+    st->active = fr_active(psi, n, amax, st->reach);
+}
+
+__device__ __forceinline__ double fr_amax(const FrExponents* exps) {
+    return __longlong_as_double(static_cast<long long>(exps[1].most)) * kOrderSlack;
+}
+
+// The bounds of the first digit's pass: the products |psi| |coef| whose exponents sum to e or more number
+// N(e), from the histograms (zeros and denormals count as the least, non-finite values as the largest
+// exponent); bound q is the weight of a product 2^e for the largest e with N(e) >= 64 K 16^q, the last one
+// the least weight.  One block.
+__global__ __launch_bounds__(1024) void fr_plan_kernel(FrState* st, const double2* __restrict__ psi, int64_t n,
+                                                       const FrExponents* __restrict__ exps, int64_t k) {
+    __shared__ unsigned long long s_pairs[4096];  // by exponent sum
+    __shared__ uint32_t s_rows[2048];
+    __shared__ uint32_t s_list[2048];  // exponents that some coefficient has
+    __shared__ unsigned long long s_wave[16];
+    __shared__ int s_count, s_e[kTries];
+    for (int e = threadIdx.x; e < 4096; e += 1024) {
+        s_pairs[e] = 0ull;
+    }
+    if (threadIdx.x == 0) {
+        s_count = 0;
+    }
+    if (threadIdx.x < kTries) {
+        s_e[threadIdx.x] = -1;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < 2048; e += 1024) {
+        s_rows[e] = exps[0].count[e];
+        if (exps[1].count[e] != 0u) {
+            s_list[atomicAdd(&s_count, 1)] = static_cast<uint32_t>(e);
+        }
+    }
+    __syncthreads();
+    for (int l = 0; l < s_count; ++l) {
+        const uint32_t a = s_list[l];
+        const unsigned long long na = exps[1].count[a];
+        for (int b = threadIdx.x; b < 2048; b += 1024) {
+            if (s_rows[b] != 0u) {
+                atomicAdd(&s_pairs[a + b], na * s_rows[b]);
+            }
+        }
+    }
+    __syncthreads();
+    // N(e) from the top, four sums a thread
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    unsigned long long v[4], sum = 0ull;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        v[q] = s_pairs[4095 - 4 * static_cast<int>(threadIdx.x) - q];
+        sum += v[q];
+    }
+    unsigned long long incl = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+        const unsigned long long o = __shfl_up(incl, d);
+        incl += lane >= d ? o : 0ull;
+    }
+    if (lane == 63) {
+        s_wave[wave] = incl;
+    }
+    __syncthreads();
+    unsigned long long cum = incl - sum;
+    for (int w = 0; w < wave; ++w) {
+        cum += s_wave[w];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        unsigned long long want = 64ull * static_cast<unsigned long long>(k);
+        for (int t = 0; t < kTries - 1; ++t, want *= 16ull) {
+            if (cum < want && cum + v[q] >= want) {
+                s_e[t] = 4095 - 4 * static_cast<int>(threadIdx.x) - q;
+            }
+        }
+        cum += v[q];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int q = 0, last = -1;
+        for (int t = 0; t < kTries - 1; ++t) {
+            if (s_e[t] >= 0 && s_e[t] != last) {
+                // biased exponents summing to e: products from 2^(e - 2046), weights from 2^(2 e - 4092)
+                last = s_e[t];
+                const int biased = 2 * last - 4092 + 1023;
+                st->bound[q++] = biased >= 2046 ? 2046ull << 52 : (biased > 0 ? static_cast<uint64_t>(biased) << 52 : 1ull);
+            }
+        }
+        for (; q < kTries; ++q) {
+            st->bound[q] = 1ull;
+        }
+        fr_set_lo(st, st->bound[0], psi, n, fr_amax(exps));
+    }
+}
+
+// Chooses the threshold digit of the current level (one block; 4096 bins, four a thread, from the top).
+__global__ __launch_bounds__(1024) void fr_select_kernel(FrState* st, unsigned long long* hist, const double2* __restrict__ psi, int64_t n,
+                                                         const FrExponents* __restrict__ exps, int64_t cand_cap) {
+    __shared__ unsigned long long s_wave[16];
+    __shared__ unsigned long long s_cum, s_in;
+    __shared__ int s_digit;
+    if (st->done) {
+        return;  // uniform: every thread reads the same flag
     }
     const int level = st->level;
     const int width = fr_width(level);
     const int bins = 1 << width;
-    unsigned long long total = 0;
-    for (int b = 0; b < bins; ++b) {
-        total += hist[b];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    unsigned long long v[4], sum = 0ull;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int b = bins - 1 - (4 * static_cast<int>(threadIdx.x) + q);
+        v[q] = b >= 0 ? hist[b] : 0ull;
+        sum += v[q];
+        if (b >= 0) {
+            hist[b] = 0ull;
+        }
+    }
+    unsigned long long incl = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+        const unsigned long long o = __shfl_up(incl, d);
+        incl += lane >= d ? o : 0ull;
+    }
+    if (lane == 63) {
+        s_wave[wave] = incl;
+    }
+    if (threadIdx.x == 0) {
+        s_digit = -1;
+    }
+    __syncthreads();
+    unsigned long long total = 0ull, cum = incl - sum;
+    for (int w = 0; w < 16; ++w) {
+        total += s_wave[w];
+        cum += w < wave ? s_wave[w] : 0ull;
     }
     const unsigned long long need = static_cast<unsigned long long>(st->k_rem);
-    if (level == 0 && total <= need) {
-        st->all = 1;
-        st->done = 1;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        if (cum < need && cum + v[q] >= need) {
+            s_digit = bins - 1 - (4 * static_cast<int>(threadIdx.x) + q);
+            s_cum = cum;
+            s_in = v[q];
+        }
+        cum += v[q];
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) {
+        return;
+    }
+    const double amax = fr_amax(exps);
+    if (level == 0 && total <= need && st->lo > 1ull) {
+        // fewer than K above the bound: the next one (K of them exactly: the same selection, found again)
+        fr_set_lo(st, st->bound[++st->tries], psi, n, amax);
+    } else if (level == 0 && total <= need) {
+        st->done = 1;  // every nonzero entry is selected outright
         st->cand_needed = 0;
-        st->lo = 1;  // every nonzero entry is selected outright
         st->hi = 1;
     } else {
-        unsigned long long cum = 0;
-        int d = bins - 1;
-        for (; d > 0; --d) {
-            if (cum + hist[d] >= need) {
-                break;
-            }
-            cum += hist[d];
-        }
-        st->k_rem = static_cast<int64_t>(need - cum);
-        st->prefix = (st->prefix << width) | static_cast<uint64_t>(d);
-        st->shift = fr_shift(level);
-        if (hist[d] <= static_cast<unsigned long long>(cand_cap) || level == kLevels - 1) {
+        const uint64_t d = static_cast<uint64_t>(s_digit);
+        st->k_rem = static_cast<int64_t>(need - s_cum);
+        st->prefix = (st->prefix << width) | d;
+        const int shift = fr_shift(level);
+        const uint64_t tied = st->prefix << shift;  // the tied class and everything above it
+        fr_set_lo(st, level == 0 && tied < st->lo ? st->lo : tied, psi, n, amax);
+        if (s_in <= static_cast<unsigned long long>(cand_cap) || level == kLevels - 1) {
             st->done = 1;
             st->cand_needed = st->k_rem;
-            st->lo = st->prefix << st->shift;         // the tied class
-            st->hi = (st->prefix + 1ull) << st->shift;  // everything above it
+            st->hi = (st->prefix + 1ull) << shift;
         } else {
             st->level = level + 1;
         }
-    }
-    for (int b = 0; b < bins; ++b) {
-        hist[b] = 0;
     }
 }
 
@@ -483,41 +626,29 @@ __global__ void fr_scatter_kernel(const uint32_t* __restrict__ perm, int64_t n, 
     }
 }
 
+// Entries tied on the digits so far are collected as candidates up to this many, and narrowed by another
+// digit's pass above it: the candidates are sorted twice in full (1M of them: 1.7 ms), a pass over what
+// is left of the connections costs less.
 int64_t cand_capacity(int64_t k) {
-    int64_t cap = 2 * k;
-    return cap < (1 << 20) ? (1 << 20) : cap;
-}
-
-// The sampled attempt: n_s rows (0 = no attempt) with f K >= 64 sampled ranks, and a weight
-// buffer of at most 2^25 entries (n_s n_terms bounds the contributions of the sample).  At most
-// 4096 rows are sampled, so an attempt whose sample overflows the buffer wastes little.
-struct FrSamplePlan {
-    int64_t n_s;
-    int64_t cap;
-};
-
-FrSamplePlan fr_sample_plan(int64_t n_i, int64_t k, int64_t n_terms) {
-    FrSamplePlan sp{0, 0};
-    if (n_i < 4096 || k <= 0 || n_terms <= 0) {
-        return sp;
-    }
-    int64_t n_s = (64 * n_i + k - 1) / k;
-    n_s = n_s < 512 ? 512 : n_s;
-    if (n_s > n_i / 4 || n_s > 4096) {
-        return sp;  // a sample this large saves little over the exact passes
-    }
-    const int64_t limit = int64_t{1} << 25;
-    sp.n_s = n_s;
-    sp.cap = n_s > limit / n_terms ? limit : n_s * n_terms;
-    return sp;
+    const int64_t cap = 2 * k;
+    return cap < (1 << 16) ? (1 << 16) : cap;
 }
 
 struct FrScratch {
-    FrSamplePlan plan;
-    uint8_t* sample_configs;
-    double2* sample_psi;
-    uint64_t* sample_w;
-    uint64_t* sample_alt;
+    uint8_t* configs;  // rows in descending |psi|
+    double2* psi;
+    uint32_t* row_key_a;
+    uint32_t* row_key_b;
+    uint32_t* row_a;
+    uint32_t* row_b;
+    uint64_t* recs;  // terms in descending |coef| within each bucket
+    double2* coefs;
+    double* aw;
+    uint64_t* term_key_a;
+    uint64_t* term_key_b;
+    uint32_t* term_a;
+    uint32_t* term_b;
+    FrExponents* exps;
     FrState* state;
     unsigned long long* hist;
     uint64_t* sel_c;
@@ -537,11 +668,21 @@ FrScratch fr_layout(Carver& cv, int W, int n_qubytes, int64_t n_i, int64_t k, in
     const int64_t cap = cand_capacity(k);
     const size_t M = static_cast<size_t>(cap > k ? cap : k);
     FrScratch s{};
-    s.plan = fr_sample_plan(n_i, k, n_terms);
-    s.sample_configs = cv.take<uint8_t>(static_cast<size_t>(s.plan.n_s) * n_qubytes);
-    s.sample_psi = cv.take<double2>(static_cast<size_t>(s.plan.n_s));
-    s.sample_w = cv.take<uint64_t>(static_cast<size_t>(s.plan.cap));
-    s.sample_alt = cv.take<uint64_t>(static_cast<size_t>(s.plan.cap));
+    const size_t N = static_cast<size_t>(n_i > 0 ? n_i : 1), T = static_cast<size_t>(n_terms > 0 ? n_terms : 1);
+    s.configs = cv.take<uint8_t>(N * static_cast<size_t>(n_qubytes));
+    s.psi = cv.take<double2>(N);
+    s.row_key_a = cv.take<uint32_t>(N);
+    s.row_key_b = cv.take<uint32_t>(N);
+    s.row_a = cv.take<uint32_t>(N);
+    s.row_b = cv.take<uint32_t>(N);
+    s.recs = cv.take<uint64_t>(T);
+    s.coefs = cv.take<double2>(T);
+    s.aw = cv.take<double>(T);
+    s.term_key_a = cv.take<uint64_t>(T);
+    s.term_key_b = cv.take<uint64_t>(T);
+    s.term_a = cv.take<uint32_t>(T);
+    s.term_b = cv.take<uint32_t>(T);
+    s.exps = cv.take<FrExponents>(2);
     s.state = cv.take<FrState>(1);
     s.hist = cv.take<unsigned long long>(kHistBins);
     s.sel_c = cv.take<uint64_t>(static_cast<size_t>(k) * W);
@@ -553,16 +694,16 @@ FrScratch fr_layout(Carver& cv, int W, int n_qubytes, int64_t n_i, int64_t k, in
     s.key_b = cv.take<uint64_t>(M);
     s.flag = cv.take<uint32_t>(static_cast<size_t>(k));
     s.pos = cv.take<uint32_t>(static_cast<size_t>(k));
-    size_t sort_bytes = 0, sort_desc_bytes = 0, scan_bytes = 0, sample_bytes = 0;
+    size_t sort_bytes = 0, sort_desc_bytes = 0, scan_bytes = 0, row_bytes = 0, term_bytes = 0;
     (void)rocprim::radix_sort_pairs(nullptr, sort_bytes, s.key_a, s.key_b, s.perm_a, s.perm_b, static_cast<unsigned>(M));
     (void)rocprim::radix_sort_pairs_desc(nullptr, sort_desc_bytes, s.key_a, s.key_b, s.perm_a, s.perm_b, static_cast<unsigned>(M));
     (void)rocprim::exclusive_scan(nullptr, scan_bytes, s.flag, s.pos, 0u, static_cast<size_t>(k), rocprim::plus<uint32_t>());
-    if (s.plan.n_s > 0) {
-        (void)rocprim::radix_sort_keys_desc(nullptr, sample_bytes, s.sample_w, s.sample_alt, static_cast<unsigned>(s.plan.cap));
-    }
+    (void)rocprim::radix_sort_pairs_desc(nullptr, row_bytes, s.row_key_a, s.row_key_b, s.row_a, s.row_b, N);
+    (void)rocprim::radix_sort_pairs(nullptr, term_bytes, s.term_key_a, s.term_key_b, s.term_a, s.term_b, T);
     size_t t = sort_bytes > sort_desc_bytes ? sort_bytes : sort_desc_bytes;
     t = t > scan_bytes ? t : scan_bytes;
-    t = t > sample_bytes ? t : sample_bytes;
+    t = t > row_bytes ? t : row_bytes;
+    t = t > term_bytes ? t : term_bytes;
     s.tmp = cv.take_bytes(t);
     s.tmp_bytes = t;
     return s;
@@ -592,11 +733,19 @@ int find_relative_impl(const qmb_terms* terms, const qmb_targets* exclude, const
         return set_error(QMB_ERR_WORKSPACE, "find_relative scratch too small: need %zu, have %zu", cv.off, scratch_bytes);
     }
     const int64_t cap = cand_capacity(k);
-    const LaunchShape ls = resolve_launch(nullptr, W, n_i, terms->n_terms);
+    LaunchShape ls = resolve_launch(nullptr, W, n_i, terms->n_terms);
+    if (!ls.direct) {
+        // small units: what is enumerated lies in the first tiles' rows and the buckets' first terms
+        ls.tile_log2 = 6;
+        ls.groups = 16;
+    }
+    const int64_t T = terms->n_terms;
     FrParams p{};
-    p.src = make_source(terms, configs_i, n_i);
-    p.psi = reinterpret_cast<const double2*>(psi_i);
-    p.coefs = reinterpret_cast<const double2*>(terms->coefs);
+    p.src = make_source(terms, s.configs, n_i);
+    p.src.recs = s.recs;
+    p.psi = s.psi;
+    p.coefs = s.coefs;
+    p.aw = s.aw;
     p.xkeys = exclude->keys;
     p.xtable = exclude->table;
     p.xmask = exclude->capacity - 1;
@@ -608,66 +757,57 @@ int find_relative_impl(const qmb_terms* terms, const qmb_targets* exclude, const
     p.sel_c = s.sel_c;
     p.cand_w = s.cand_w;
     p.cand_c = s.cand_c;
-    p.sample_w = s.sample_w;
-    p.sample_cap = s.plan.cap;
     p.k = k;
     p.cand_cap = cap;
     p.tile_log2 = ls.tile_log2;
     p.groups = ls.groups;
     p.direct = ls.direct ? 1 : 0;
     const int64_t tiles = (n_i + (1ll << ls.tile_log2) - 1) >> ls.tile_log2;
-    const int64_t grid = n_i <= 0 ? 0 : (ls.direct ? (n_i + kEnumBlock - 1) / kEnumBlock : tiles * ls.groups);
+    const int64_t units = n_i <= 0 ? 0 : (ls.direct ? (n_i + kEnumBlock - 1) / kEnumBlock : tiles * ls.groups);
+    const unsigned grid = static_cast<unsigned>(units < 4096 ? units : 4096);
     const size_t lds = ls.direct ? direct_lds_bytes(W) : enum_lds_bytes_of(W, terms->n_bits, ls.tile_log2);
 
-    fr_init_kernel<<<1, 256, 0, stream>>>(s.state, s.hist, k);
+    fr_init_kernel<<<1, 256, 0, stream>>>(s.state, s.hist, s.exps, k);
     QMB_CHECK_LAUNCH();
     QMB_TRY(launch_fill_u64(s.cand_w, 0ull, cap, stream));
-    if (grid > 0 && terms->n_terms > 0) {
+    if (grid > 0 && T > 0) {
         QMB_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&fr_hist_kernel<W>),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
         QMB_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&fr_collect_kernel<W>),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-        if (s.plan.n_s > 0) {
-            // the sampled attempt: sample contributions, bounds, one collect pass, check
-            const int64_t n_s = s.plan.n_s;
-            fr_gather_sample_kernel<<<blocks_for(n_s), 256, 0, stream>>>(configs_i, p.psi, n_i, terms->n_qubytes, n_s, s.sample_configs,
-                                                                         s.sample_psi);
+        const auto* psi = reinterpret_cast<const double2*>(psi_i);
+        const auto* coefs = reinterpret_cast<const double2*>(terms->coefs);
+        fr_row_keys_kernel<<<blocks_for(n_i), 256, 0, stream>>>(psi, n_i, s.row_key_a, s.row_a);
+        QMB_CHECK_LAUNCH();
+        size_t need = s.tmp_bytes;
+        QMB_HIP_TRY(rocprim::radix_sort_pairs_desc(s.tmp, need, s.row_key_a, s.row_key_b, s.row_a, s.row_b, static_cast<size_t>(n_i), 0, 32,
+                                                   stream));
+        fr_row_gather_kernel<<<blocks_for(n_i), 256, 0, stream>>>(s.row_b, configs_i, psi, n_i, terms->n_qubytes, s.configs, s.psi);
+        QMB_CHECK_LAUNCH();
+        fr_term_keys_kernel<<<blocks_for(T), 256, 0, stream>>>(coefs, terms->bucket_start, terms->n_buckets, T, s.term_key_a, s.term_a);
+        QMB_CHECK_LAUNCH();
+        int bits = 33;
+        while ((int64_t{1} << (bits - 32)) <= terms->n_buckets) {
+            ++bits;
+        }
+        need = s.tmp_bytes;
+        QMB_HIP_TRY(rocprim::radix_sort_pairs(s.tmp, need, s.term_key_a, s.term_key_b, s.term_a, s.term_b, static_cast<size_t>(T), 0,
+                                              static_cast<unsigned>(bits), stream));
+        fr_term_gather_kernel<<<blocks_for(T), 256, 0, stream>>>(s.term_b, terms->recs, coefs, T, s.recs, s.coefs, s.aw);
+        QMB_CHECK_LAUNCH();
+        fr_exponents_kernel<<<blocks_for(n_i) < 512u ? blocks_for(n_i) : 512u, 256, 0, stream>>>(psi, n_i, s.exps);
+        QMB_CHECK_LAUNCH();
+        fr_exponents_kernel<<<blocks_for(T) < 512u ? blocks_for(T) : 512u, 256, 0, stream>>>(coefs, T, s.exps + 1);
+        QMB_CHECK_LAUNCH();
+        fr_plan_kernel<<<1, 1024, 0, stream>>>(s.state, s.psi, n_i, s.exps, k);
+        QMB_CHECK_LAUNCH();
+        for (int pass = 0; pass < kTries - 1 + kLevels; ++pass) {
+            fr_hist_kernel<W><<<grid, kEnumBlock, lds, stream>>>(p);
             QMB_CHECK_LAUNCH();
-            QMB_TRY(launch_fill_u64(s.sample_w, 0ull, s.plan.cap, stream));
-            FrParams ps = p;
-            ps.src = make_source(terms, s.sample_configs, n_s);
-            ps.psi = s.sample_psi;
-            const LaunchShape lss = resolve_launch(nullptr, W, n_s, terms->n_terms);
-            const int64_t tiles_s = (n_s + (1ll << lss.tile_log2) - 1) >> lss.tile_log2;
-            const int64_t grid_s = lss.direct ? (n_s + kEnumBlock - 1) / kEnumBlock : tiles_s * lss.groups;
-            const size_t lds_s = lss.direct ? direct_lds_bytes(W) : enum_lds_bytes_of(W, terms->n_bits, lss.tile_log2);
-            ps.tile_log2 = lss.tile_log2;
-            ps.groups = lss.groups;
-            ps.direct = lss.direct ? 1 : 0;
-            QMB_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&fr_sample_kernel<W>),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_s > lds ? lds_s : lds)));
-            fr_sample_kernel<W><<<static_cast<unsigned>(grid_s), kEnumBlock, lds_s, stream>>>(ps);
-            QMB_CHECK_LAUNCH();
-            size_t need_s = s.tmp_bytes;
-            QMB_HIP_TRY(rocprim::radix_sort_keys_desc(s.tmp, need_s, s.sample_w, s.sample_alt, static_cast<unsigned>(s.plan.cap), 0, 64,
-                                                      stream));
-            fr_bounds_kernel<<<1, 64, 0, stream>>>(s.state, s.sample_alt, s.plan.cap,
-                                                   static_cast<double>(n_s) / static_cast<double>(n_i), k);
-            QMB_CHECK_LAUNCH();
-            fr_collect_kernel<W><<<static_cast<unsigned>(grid), kEnumBlock, lds, stream>>>(p, 0);
-            QMB_CHECK_LAUNCH();
-            fr_verify_kernel<<<1, 64, 0, stream>>>(s.state, k, cap);
-            QMB_CHECK_LAUNCH();
-            fr_clear_failed_kernel<<<blocks_for(cap), 256, 0, stream>>>(s.state, s.cand_w, cap);
+            fr_select_kernel<<<1, 1024, 0, stream>>>(s.state, s.hist, s.psi, n_i, s.exps, cap);
             QMB_CHECK_LAUNCH();
         }
-        for (int level = 0; level < kLevels; ++level) {
-            fr_hist_kernel<W><<<static_cast<unsigned>(grid), kEnumBlock, lds, stream>>>(p);
-            QMB_CHECK_LAUNCH();
-            fr_select_kernel<<<1, 64, 0, stream>>>(s.state, s.hist, cap);
-            QMB_CHECK_LAUNCH();
-        }
-        fr_collect_kernel<W><<<static_cast<unsigned>(grid), kEnumBlock, lds, stream>>>(p, 1);
+        fr_collect_kernel<W><<<grid, kEnumBlock, lds, stream>>>(p);
         QMB_CHECK_LAUNCH();
     }
     // Candidates: order by (weight desc, config asc), keep the first cand_needed.

@@ -102,6 +102,53 @@ def test_find_relative_distinct_exclude_set(cuda_device: torch.device) -> None:
     _assert_same_selection("distinct-exclude", 1, cfg, psi, exclude, s, k, c, got, want, kth)
 
 
+def _spread_psi(kind: str, n: int) -> np.ndarray:
+    """Amplitudes that rank rows very unevenly: a decay over 12 decades, many exact zeros, magnitudes whose
+    weights underflow to denormals and zero or overflow to infinity, or one heavy row."""
+    rng = np.random.default_rng(71)
+    psi = rng.normal(size=n) + 1j * rng.normal(size=n)
+    if kind == "decay":
+        return psi * 10.0 ** rng.uniform(-12, 0, size=n)
+    if kind == "zeros":
+        return np.where(rng.random(n) < 0.9, 0.0, psi)
+    if kind == "range":
+        return psi * 10.0 ** rng.uniform(-170, 155, size=n)
+    psi *= 1e-9
+    psi[n // 3] = 1.0
+    return psi
+
+
+@pytest.mark.parametrize("k_sel", [1, 40, 3000, 500_000])
+@pytest.mark.parametrize("kind", ["decay", "zeros", "range", "heavy-row"])
+@pytest.mark.parametrize("name", ["molecular", "molecular-unsorted", "two-words", "hubbard", "hubbard-300-terms"])
+def test_find_relative_selects_what_the_host_operator_does(cuda_device: torch.device, name: str, kind: str, k_sel: int) -> None:
+    """The pruned passes against the host operator (every connection weighed, the same rule on ties: weight
+    descending, then config ascending), row for row: both enumerations (above and up to 4096 terms), term
+    tables in any order, row counts that leave a ragged tile, and K below, inside and above the number of
+    connections outside the set."""
+    pc = 1
+    if name.startswith("molecular"):
+        s, k, c = sorted_terms(*sy.molecular_terms(8, 72))
+        cfg = sy.sector_configs(8, 3, 3, 333, 73)
+    elif name == "two-words":
+        s, k, c = sorted_terms(*sy.random_terms(70, 6000, 74))
+        cfg = sy.sort_unique_configs(np.random.default_rng(75).integers(0, 256, size=(129, 9), dtype=np.uint8) & np.array([255] * 8 + [63], np.uint8))
+    else:
+        m = 4 if name == "hubbard" else 50
+        s, k, c = (x.numpy() for x in sy.terms_from_dict(sy.hubbard_dict(m, 1, 1.0, 4.0)))
+        cfg = sy.sector_configs(4, 2, 2, 30, 76) if m == 4 else sy.hubbard_chain_configs(50, 1200, 77, n_seed_configs=64)
+    if name == "molecular-unsorted":
+        order = np.random.default_rng(78).permutation(len(s))
+        s, k, c = s[order], k[order], c[order]
+    psi = _spread_psi(kind, len(cfg))
+    ns = ops.load(cfg.shape[1], pc)
+    host = [torch.from_numpy(np.ascontiguousarray(x)) for x in (cfg, psi.view(np.float64).reshape(-1, 2), s, k, c)]
+    want = ns.find_relative(host[0], host[1], k_sel, host[2], host[3], host[4], host[0])
+    dev = [t.to(cuda_device) for t in host]
+    got = ns.find_relative(dev[0], dev[1], k_sel, dev[2], dev[3], dev[4], dev[0]).cpu()
+    assert torch.equal(got, want), (name, kind, k_sel, got.shape, want.shape)
+
+
 DIAG_CASES = [
     ("molecular-20so", 1, lambda: sorted_terms(*sy.molecular_terms(10, 1001)), lambda: sy.sector_configs(10, 5, 5, 2000, 21)),
     ("random-ops", 1, lambda: tuple(x.numpy() for x in sy.random_terms(12, 500, 22)),
