@@ -338,8 +338,9 @@ typedef struct qmb_cores {
     uint64_t* mvals;   /* their entries bin by bin: row | slot << 32 | sign << 63 (slot: pair_slot of the removed
                           pair, order 1 the removed site; sign: parity of the core's sites in [site0, site1),
                           order 1 below site0) */
-    uint64_t* glist;   /* groups of more than 32 entries and the groups of the mixed groups' cores, as two u32
-                          each: first entry in mvals, size (0: an unused slot) */
+    uint64_t* glist;   /* 64 rows each of the groups of more than 32 entries and of the groups of the mixed
+                          groups' cores, as two u32: first entry in mvals, size | tile << 16 (0: an unused
+                          slot; from 2^16 entries on all rows: size | 2^31) */
     void* bins;        /* device table of the bins */
 } qmb_cores;
 

@@ -767,6 +767,20 @@ __device__ __forceinline__ int group_bin(uint32_t size, bool mixed) {
     return kExactBins + (k < kBigBins ? k : kBigBins - 1);
 }
 
+// A group above 64 entries is listed once per 64 of its rows: a wave each, with all its entries.  (With
+// one wave for a whole group the few hundred groups of 130 to 700 entries were the kernel's tail: 200,000
+// two-word configs 5.0 -> 4.5 ms, a batch of 12 sets of 50,000 4.1 -> 3.7 ms.)  A list element is
+// {first entry, size | tile << 16}; from 2^16 entries on (only with repeated configs) it is
+// {first entry, size | kWholeGroup}, for one wave.
+constexpr uint32_t kTiledMax = 0xffffu;
+constexpr uint32_t kWholeGroup = 0x80000000u;
+__device__ __forceinline__ uint32_t group_tiles(uint32_t size) { return size <= kTiledMax ? (size + 63u) / 64u : 1u; }
+__device__ __forceinline__ uint2 listed_tile(uint32_t first, uint32_t size, uint32_t tile) {
+    return make_uint2(first, size <= kTiledMax ? size | (tile << 16) : size | kWholeGroup);
+}
+// Elements a group of bin b adds to the bin's count.
+__device__ __forceinline__ uint32_t bin_items(int b, uint32_t size) { return b >= kExactBins && b < kSplitBin ? group_tiles(size) : 1u; }
+
 // A work unit of a bin of size g: this many passes of 64 lanes (64 / g groups each), so that a unit of
 // small groups is worth its decoding and keeps a few gathers in flight.
 __host__ __device__ __forceinline__ int unit_passes(int g, int order) {
@@ -855,7 +869,8 @@ __global__ __launch_bounds__(kBlock) void bin_count_kernel(const uint32_t* __res
             const uint32_t s = starts[g];
             const uint32_t size = (starts[g + 1] & kGroupStart) - (s & kGroupStart);
             if (size >= 2u) {
-                atomicAdd(&s_bin[group_bin(size, (s & kGroupMixed) != 0u)], (1ull << 32) | size);
+                const int b = group_bin(size, (s & kGroupMixed) != 0u);
+                atomicAdd(&s_bin[b], (static_cast<unsigned long long>(bin_items(b, size)) << 32) | size);
             }
         }
     }
@@ -869,7 +884,7 @@ __global__ __launch_bounds__(kBlock) void bin_count_kernel(const uint32_t* __res
 }
 
 // Splits the mixed group m (group, place in mvals) by core, by one wave: each core's entries go to the group's place in
-// mvals, in the order of their first entries, and take the next of the group's list slots; an entry
+// mvals, in the order of their first entries, and take the next size / 2 of the group's list slots; an entry
 // alone with its core has no partner and is dropped.  The slots of a group placed `a` entries into the
 // bin are [a / 2, (a + size) / 2): disjoint, and at least floor(size / 2) of them.  The rest are empty.
 template <int W, int ORDER>
@@ -938,10 +953,14 @@ __device__ void split_group(const uint32_t* __restrict__ starts, const uint64_t*
                 n += static_cast<uint32_t>(__popcll(mask));
             }
             if (n >= 2u) {
-                if (lane == 0) {
-                    glist[slot] = make_uint2(out, n);
+                // its tiles, apart so that no two are one unit's (a tile has at least kSplitSlots slots)
+                const uint32_t apart = n / 2u / group_tiles(n);
+                for (uint32_t k = lane; k < n / 2u; k += 64) {
+                    const uint32_t tile = k / apart;
+                    const bool here = k % apart == 0u && tile < group_tiles(n);
+                    glist[slot + k] = here ? listed_tile(out, n, tile) : make_uint2(0u, 0u);
                 }
-                ++slot;
+                slot += n / 2u;
                 out += n;
             }
         }
@@ -985,7 +1004,7 @@ __global__ __launch_bounds__(kBlock) void bin_scatter_kernel(const uint32_t* __r
         uint32_t move = kStay;
         if (size >= 2u) {
             const int b = group_bin(size, (s & kGroupMixed) != 0u);
-            const unsigned long long r = atomicAdd(&s_rank[b], (1ull << 32) | size);
+            const unsigned long long r = atomicAdd(&s_rank[b], (static_cast<unsigned long long>(bin_items(b, size)) << 32) | size);
             const uint32_t rank = s_group0[b] + static_cast<uint32_t>(r >> 32);
             if (b < kExactBins) {
                 move = bins->entry_base[b] + rank * size - first;
@@ -994,7 +1013,9 @@ __global__ __launch_bounds__(kBlock) void bin_scatter_kernel(const uint32_t* __r
                 if (b == kSplitBin) {
                     msplit[rank] = make_uint2(static_cast<uint32_t>(g0) + static_cast<uint32_t>(t), at);
                 } else {
-                    glist[bins->list_base[b] + rank] = make_uint2(at, size);
+                    for (uint32_t k = 0; k < group_tiles(size); ++k) {
+                        glist[bins->list_base[b] + rank + k] = listed_tile(at, size, k);
+                    }
                     move = at - first;
                 }
             }
@@ -1211,7 +1232,8 @@ __global__ __launch_bounds__(kSmallThreads) void cores_small_kernel(const uint64
         starts[q] = first | (mixed ? kGroupMixed : 0u);
         const uint32_t size = q < n_groups ? L.start[q + 1] - first : 0u;
         if (size >= 2u) {
-            atomicAdd(&L.rank[group_bin(size, mixed)], (1ull << 32) | size);
+            const int b = group_bin(size, mixed);
+            atomicAdd(&L.rank[b], (static_cast<unsigned long long>(bin_items(b, size)) << 32) | size);
         }
     }
     __syncthreads();
@@ -1228,7 +1250,7 @@ __global__ __launch_bounds__(kSmallThreads) void cores_small_kernel(const uint64
         uint32_t move = kSmallStay;
         if (size >= 2u) {
             const int b = group_bin(size, L.mixed[q] != 0);
-            const unsigned long long r = atomicAdd(&L.rank[b], (1ull << 32) | size);
+            const unsigned long long r = atomicAdd(&L.rank[b], (static_cast<unsigned long long>(bin_items(b, size)) << 32) | size);
             const uint32_t rank = static_cast<uint32_t>(r >> 32);
             move = bins->entry_base[b] + static_cast<uint32_t>(r);
             if (b == kSplitBin) {
@@ -1236,7 +1258,9 @@ __global__ __launch_bounds__(kSmallThreads) void cores_small_kernel(const uint64
                 atomicAdd(&L.n_mixed, 1u);
                 move = kSmallStay;
             } else if (b >= kExactBins) {
-                glist[bins->list_base[b] + rank] = make_uint2(move, size);
+                for (uint32_t k = 0; k < group_tiles(size); ++k) {
+                    glist[bins->list_base[b] + rank + k] = listed_tile(move, size, k);
+                }
             }
         }
         L.move[q] = static_cast<uint16_t>(move);
@@ -1575,13 +1599,13 @@ __device__ __forceinline__ void pair_rows(const PairParams& p, int g, uint32_t e
     add_rows<NV>(p, st, 0, lane, act, e, re, im);
 }
 
-// One group of any size from mvals[s]: 64 rows at a time against its entries, 64 staged
-// at a time.
+// Rows [first, last) of one group of any size from mvals[s]: 64 rows at a time against its entries, 64
+// staged at a time.
 template <bool ADJ, bool REAL, int NV, int B>
-__device__ __forceinline__ void pair_big(const PairParams& p, uint32_t s, uint32_t size, int lane, Stage<NV>& st) {
+__device__ __forceinline__ void pair_big(const PairParams& p, uint32_t s, uint32_t size, uint32_t first, uint32_t last, int lane, Stage<NV>& st) {
     const bool fermi = p.particle_cut == 1;
     const auto wide = [&](const Entry& e) { return e.slot * static_cast<uint32_t>(p.n_pairs); };
-    for (uint32_t a0 = 0; a0 < size; a0 += 64) {
+    for (uint32_t a0 = first; a0 < last; a0 += 64) {
         const bool act = a0 + lane < size;
         const Entry e = binned_entry(act ? p.mvals[s + a0 + lane] : 0ull, fermi);
         const uint32_t mine = ADJ ? wide(e) : e.slot;
@@ -1608,13 +1632,18 @@ __device__ __forceinline__ int unit_bin(const CoreBins* bins, uint32_t u, int la
     return kBins - 1 - pos;
 }
 
-// The groups of a listed unit: one group of a bin above 32 entries, or kSplitSlots slots of the split
-// bin, most of them empty.  f(first entry, size) runs for each, wave-uniform.
+// The rows of a listed unit: one list element of a bin above 32 entries, or kSplitSlots of the split
+// bin, most of them empty.  f(first entry, size, first row, end of the rows) runs for each, wave-uniform.
 template <typename P, typename F>
 __device__ __forceinline__ void for_listed(const P& p, int bin, uint32_t local, int lane, F&& f) {
+    const auto tile = [&](uint32_t s, uint32_t y) {
+        const bool whole = (y & kWholeGroup) != 0u;
+        const uint32_t size = whole ? y & ~kWholeGroup : y & kTiledMax;
+        f(s, size, whole ? 0u : (y >> 16) * 64u, whole ? size : (y >> 16) * 64u + 1u);
+    };
     if (bin != kSplitBin) {
         const uint2 group = p.glist[p.bins->list_base[bin] + local];
-        f(group.x, group.y);
+        tile(group.x, group.y);
         return;
     }
     const uint32_t slot = local * kSplitSlots + static_cast<uint32_t>(lane);
@@ -1624,7 +1653,7 @@ __device__ __forceinline__ void for_listed(const P& p, int bin, uint32_t local, 
     while (full) {
         const int l = __builtin_ctzll(full);
         full &= full - 1;
-        f(__builtin_amdgcn_readlane(mine.x, l), __builtin_amdgcn_readlane(mine.y, l));
+        tile(__builtin_amdgcn_readlane(mine.x, l), __builtin_amdgcn_readlane(mine.y, l));
     }
 }
 
@@ -1654,7 +1683,9 @@ __device__ __forceinline__ void pair_unit(const PairParams& p, uint32_t u, int l
         }
         return;
     }
-    for_listed(p, bin, local, lane, [&](uint32_t s, uint32_t size) { pair_big<ADJ, REAL, NV, B>(p, s, size, lane, st); });
+    for_listed(p, bin, local, lane, [&](uint32_t s, uint32_t size, uint32_t first, uint32_t last) {
+        pair_big<ADJ, REAL, NV, B>(p, s, size, first, last, lane, st);
+    });
 }
 
 __device__ __forceinline__ void mark_overflow(double2* out) {
@@ -1873,14 +1904,14 @@ __device__ __forceinline__ void single_rows(const SingleParams& p, int g, uint32
     add_rows<NV>(p, st, 0, lane, act, e, re, im);
 }
 
-// One group of any size from mvals[s], lane = row.
+// Rows [first, last) of one group of any size from mvals[s], lane = row.
 template <int W, bool ADJ, int NV, int CH>
-__device__ void single_group(const SingleParams& p, uint32_t s, uint32_t size, int lane, Stage<NV>& st) {
+__device__ void single_group(const SingleParams& p, uint32_t s, uint32_t size, uint32_t first, uint32_t last, int lane, Stage<NV>& st) {
     const bool fermi = p.particle_cut == 1;
-    const Entry first = binned_entry(p.mvals[s], fermi);
-    Cfg<W> core = load_key<W>(p.ckeys, static_cast<int64_t>(first.row));
-    flip_site<W>(core, static_cast<int>(first.slot));
-    for (uint32_t a0 = 0; a0 < size; a0 += 64) {
+    const Entry head = binned_entry(p.mvals[s], fermi);
+    Cfg<W> core = load_key<W>(p.ckeys, static_cast<int64_t>(head.row));
+    flip_site<W>(core, static_cast<int>(head.slot));
+    for (uint32_t a0 = first; a0 < last; a0 += 64) {
         const bool act = a0 + lane < size;
         const Entry e = binned_entry(p.mvals[s + (act ? a0 + lane : 0u)], fermi);
         const int r = static_cast<int>(e.slot);
@@ -1920,7 +1951,9 @@ __device__ __forceinline__ void single_unit(const SingleParams& p, uint32_t u, i
         }
         return;
     }
-    for_listed(p, bin, local, lane, [&](uint32_t s, uint32_t size) { single_group<W, ADJ, NV, CH>(p, s, size, lane, st); });
+    for_listed(p, bin, local, lane, [&](uint32_t s, uint32_t size, uint32_t first, uint32_t last) {
+        single_group<W, ADJ, NV, CH>(p, s, size, first, last, lane, st);
+    });
 }
 
 template <int W, bool ADJ, int NV = 1>

@@ -383,3 +383,42 @@ def test_core_index_builds_around_the_one_block_limit(cuda_device: torch.device,
     ref, rsum, _ = orc.apply_within(1, cfg, g, cfg, s, k, c)  # the table is Hermitian
     got = pp.apply(terms, targets, cfg_t, gvec, pp.MODE_ADJOINT, symmetric=pp.SYMMETRIC_OFF, pairs=True).cpu().numpy()
     assert np.all(np.abs(got[:, 0] + 1j * got[:, 1] - ref) <= 1e-12 * rsum + 1e-300)
+
+
+@pytest.mark.parametrize("bits", [0, 4])
+@pytest.mark.parametrize("order,size", [(2, 63), (2, 64), (2, 65), (2, 128), (2, 129), (2, 256), (1, 63), (1, 64), (1, 65), (1, 127)])
+def test_groups_around_the_row_tiles(cuda_device: torch.device, order: int, size: int, bits: int) -> None:
+    """Core groups on both sides of multiples of the 64 rows one wave takes, alone under their key and
+    (4-bit hash columns) mixed with others: `size` site pairs of opposite parity beside each of 20
+    spectators (order 2), or `size` sites beside one occupied site (order 1)."""
+    if order == 2:
+        nq = 9
+        pairs = [(a, b) for a in range(0, 32, 2) for b in range(1, 32, 2)][:size]
+        occupied = [(a, b, s) for a, b in pairs for s in range(40, 60)]
+        table = _pair_heavy_table(np.arange(32), 6000, 7)
+    else:
+        nq = 16
+        occupied = [(0, x) for x in range(1, size + 1)]
+        table = _pair_heavy_table(np.arange(0, 128), 12000, 8)
+    rows = np.zeros((len(occupied), 8 * nq), dtype=np.uint8)
+    for row, sites in zip(rows, occupied):
+        row[list(sites)] = 1
+    cfg = sy.sort_unique_configs(np.packbits(rows, axis=1, bitorder="little"))
+    n = len(cfg)
+    s, k, c = table
+    cfg_t = _dev(cfg, cuda_device)
+    terms = pp.PreparedTerms(_dev(s, cuda_device), _dev(k, cuda_device), _dev(c, cuda_device), nq, 1)
+    targets = pp.PreparedTargets(cfg_t, nq, distinct=True)
+    if bits:
+        _build_cores_with_narrow_hash(targets, bits, 50 + bits)
+    _, starts, _ = _core_index(targets, order)
+    st = (starts & 0x7FFFFFFF).astype(np.int64)
+    assert np.diff(st).max() >= size
+    psi = sy.random_psi(n, 33)
+    vec = torch.view_as_real(_dev(psi, cuda_device)).contiguous()
+    want, asum, _ = orc.apply_within(1, cfg, psi, cfg, s, k, c)
+    got = pp.apply(terms, targets, cfg_t, vec, pp.MODE_FORWARD, symmetric=pp.SYMMETRIC_OFF, pairs=True).cpu().numpy()
+    assert np.all(np.abs(got[:, 0] + 1j * got[:, 1] - want) <= 1e-12 * asum + 1e-300)
+    plain = pp.apply(terms, targets, cfg_t, vec, pp.MODE_ADJOINT, symmetric=pp.SYMMETRIC_OFF, pairs=False).cpu().numpy()
+    got = pp.apply(terms, targets, cfg_t, vec, pp.MODE_ADJOINT, symmetric=pp.SYMMETRIC_OFF, pairs=True).cpu().numpy()
+    assert np.abs(got - plain).max() <= 1e-12 * (np.abs(c).sum() * np.abs(psi).max())
