@@ -769,7 +769,7 @@ __device__ __forceinline__ int group_bin(uint32_t size, bool mixed) {
 
 // A group above 64 entries is listed once per 64 of its rows: a wave each, with all its entries.  (With
 // one wave for a whole group the few hundred groups of 130 to 700 entries were the kernel's tail: 200,000
-// two-word configs 5.0 -> 4.5 ms, a batch of 12 sets of 50,000 4.1 -> 3.7 ms.)  A list element is
+// two-word configs 5.0 -> 4.5 ms, a batch of 12 sets 4.1 -> 3.7 ms.)  A list element is
 // {first entry, size | tile << 16}; from 2^16 entries on (only with repeated configs) it is
 // {first entry, size | kWholeGroup}, for one wave.
 constexpr uint32_t kTiledMax = 0xffffu;

@@ -245,15 +245,30 @@ __global__ void __launch_bounds__(kSamplerThreads)
 // Fused one-hidden-layer site networks (float32).  A site network maps the 0/1 prefix bits x to
 // W2 silu(W1 x + b1) + b2; with binary inputs W1 x is the sum of the W1 columns of the set bits,
 // so the first layer is a handful of vector adds per row instead of a dense product, and the
-// hidden activations never leave registers.  A work-group of 16 waves owns 1024 rows; per site it
-// stages the site's weights in LDS (W1 as [k][h], so a bit's column is one contiguous row) and
-// every wave walks its 64 rows one at a time with all 64 lanes across the hidden units (lane l
-// holds units l, l + 64, ...: consecutive lanes read consecutive LDS words), then reduces the four
-// outputs across the wave.  Each lane keeps its own
-// row's logits, so the masks, normalisation and the rest run row-parallel afterwards.
+// hidden activations never leave registers.  A work-group of 16 waves stages a site's weights in LDS
+// and every wave walks its rows one at a time with all 64 lanes across the hidden units (lane l
+// holds units l, l + 64, ...).  The outputs of four rows are summed over the lanes together, each step
+// of the sum halving the values a lane holds: row by row these sums were a fifth of the instructions.
+// Each lane keeps its own row's logits, so the masks, normalisation and the rest run row-parallel
+// afterwards.
+//
+// The vector unit bounds it: per row and site of width 512 and seven set bits, 448 adds, 512 SiLUs
+// (five instructions each, two of them transcendental) and 2048 multiply-adds over 64 lanes.  1M rows
+// of 26 sites took 11.1 ms with a sum of four outputs per row, 9.1 with the sums of four rows together,
+// 8.6 with four units to an LDS read and the bias as the first add's operand; the vector unit then
+// issues all the time.  (The first layer on the matrix unit, 16 rows x 16 units x 4 inputs an
+// instruction, gives the same bits but 11.9 ms: the float32 matrix and vector instructions took turns,
+// and only a quarter of the inputs are set.)
+//
+// Every sum keeps one fixed order whatever the launch (a unique draw compares perturbed values, so a
+// last bit may change which configs it keeps): a hidden unit adds its bias and then the set inputs in
+// ascending order; unit u of the second layer belongs to lane u % 64, which adds its units in
+// ascending order; the 64 lanes are added as a butterfly inside each 16 and then the four 16s in order.
 // ---------------------------------------------------------------------------------------------
 constexpr int kFusedWaves = 16;
 constexpr int kFusedThreads = 64 * kFusedWaves;
+constexpr int kFusedTile = 16;     // rows whose outputs reach their lanes together
+constexpr int kFusedMaxTiles = 4;  // of a wave: a lane holds one row
 
 __device__ __forceinline__ uint64_t wave_read64(uint64_t v, int lane) {
     const uint32_t lo = __builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(v)), lane);
@@ -261,27 +276,42 @@ __device__ __forceinline__ uint64_t wave_read64(uint64_t v, int lane) {
     return (static_cast<uint64_t>(hi) << 32) | lo;
 }
 
-// DPP lane exchange within rows of 16 lanes (quad_perm, row_half_mirror, row_mirror controls).
-template <int CTRL>
-__device__ __forceinline__ float dpp(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+// DPP lane exchange within rows of 16 lanes: `old` in the banks (four lanes) that MASK leaves out.
+template <int CTRL, int MASK = 0xF>
+__device__ __forceinline__ float dpp(float v, float old = 0.f) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL, 0xF, MASK, false));
+}
+constexpr int kDppXor1 = 0xB1;    // quad_perm [1,0,3,2]
+constexpr int kDppXor2 = 0x4E;    // quad_perm [2,3,0,1]
+constexpr int kDppPlus4 = 0x104;  // row_shl 4: from lane + 4
+constexpr int kDppMinus4 = 0x114; // row_shr 4: from lane - 4
+constexpr int kDppXor8 = 0x128;   // row_ror 8
+
+// Sums over each 16 lanes of 16 values at once, as a butterfly (lane ^ 1, 2, 4, 8): lane l receives the
+// sum of p[l / 4 % 4][l % 4].  A lane passes on the half it does not keep.
+__device__ __forceinline__ float row_sums(const float (&p)[4][4], int lane) {
+    const bool b0 = (lane & 1) != 0, b1 = (lane & 2) != 0, b2 = (lane & 4) != 0, b3 = (lane & 8) != 0;
+    float s[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const float q0 = (b0 ? p[v][1] : p[v][0]) + dpp<kDppXor1>(b0 ? p[v][0] : p[v][1]);
+        const float q1 = (b0 ? p[v][3] : p[v][2]) + dpp<kDppXor1>(b0 ? p[v][2] : p[v][3]);
+        s[v] = (b1 ? q1 : q0) + dpp<kDppXor2>(b1 ? q0 : q1);
+    }
+    const float t0 = (b2 ? s[1] : s[0]) + dpp<kDppMinus4, 0xA>(s[1], dpp<kDppPlus4, 0x5>(s[0]));
+    const float t1 = (b2 ? s[3] : s[2]) + dpp<kDppMinus4, 0xA>(s[3], dpp<kDppPlus4, 0x5>(s[2]));
+    return (b3 ? t1 : t0) + dpp<kDppXor8, 0xC>(t1, dpp<kDppXor8, 0x3>(t0));
 }
 
-// Sum over the wave, the same value in every lane: a butterfly inside each row of 16 lanes on the
-// DPP network, then the four row sums read as scalars and added in row order.
-__device__ __forceinline__ float wave_sum(float v) {
-    v += dpp<0xB1>(v);   // quad_perm [1,0,3,2]
-    v += dpp<0x4E>(v);   // quad_perm [2,3,0,1]
-    v += dpp<0x141>(v);  // row_half_mirror
-    v += dpp<0x140>(v);  // row_mirror
-    const float r0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
-    const float r1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16));
-    const float r2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
-    const float r3 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
-    return ((r0 + r1) + r2) + r3;
-}
+// The hidden units of a lane in one or two LDS reads.
+template <int HPL>
+struct UnitVec {
+    static constexpr int V = HPL < 4 ? HPL : 4;
+    typedef float type __attribute__((ext_vector_type(V)));
+};
 
-// LDS image of one site network: w1 [k_rows][H], b1 [H], w2 [n_out][H], b2 [n_out].
+// LDS image of one site network: w1 [k_rows][H], b1 [H], w2 [n_out][H], b2 [n_out].  A column of w1 (all
+// units of an input) is stored in lane order, up to four units of a lane together.
 struct SiteLds {
     float* w1;
     float* b1;
@@ -298,15 +328,19 @@ __device__ __forceinline__ SiteLds site_lds(float* base, int k_max, int hidden) 
     return s;
 }
 
+template <int HPL>
 __device__ __forceinline__ void stage_site(const SiteLds& s, const float* w1, int k_rows, const float* b1, const float* w2, const float* b2,
-                                           int n_out, int hidden) {
-    for (int t = threadIdx.x; t < k_rows * hidden; t += blockDim.x) {
-        s.w1[t] = w1[t];
+                                           int n_out) {
+    constexpr int H = 64 * HPL;
+    constexpr int V = UnitVec<HPL>::V;
+    for (int t = threadIdx.x; t < k_rows * H; t += blockDim.x) {
+        const int u = t % H;
+        s.w1[t - u + u / (64 * V) * (64 * V) + u % 64 * V + u / 64 % V] = w1[t];
     }
-    for (int t = threadIdx.x; t < hidden; t += blockDim.x) {
+    for (int t = threadIdx.x; t < H; t += blockDim.x) {
         s.b1[t] = b1[t];
     }
-    for (int t = threadIdx.x; t < n_out * hidden; t += blockDim.x) {
+    for (int t = threadIdx.x; t < n_out * H; t += blockDim.x) {
         s.w2[t] = w2[t];
     }
     if (threadIdx.x < n_out) {
@@ -323,14 +357,15 @@ struct SiteRegs {
 };
 
 template <int HPL>
-__device__ __forceinline__ SiteRegs<HPL> site_regs(const SiteLds& s, int hidden, int n_out, int lane) {
+__device__ __forceinline__ SiteRegs<HPL> site_regs(const SiteLds& s, int n_out, int lane) {
+    constexpr int H = 64 * HPL;
     SiteRegs<HPL> r;
 #pragma unroll
     for (int j = 0; j < HPL; ++j) {
         r.b1[j] = s.b1[lane + 64 * j];
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            r.w2[c][j] = c < n_out ? s.w2[c * hidden + lane + 64 * j] : 0.f;
+            r.w2[c][j] = c < n_out ? s.w2[c * H + lane + 64 * j] : 0.f;
         }
     }
 #pragma unroll
@@ -340,40 +375,61 @@ __device__ __forceinline__ SiteRegs<HPL> site_regs(const SiteLds& s, int hidden,
     return r;
 }
 
-// The n_out outputs of a site network on one row (bits s0/s1, wave-uniform, already cut to the
-// network's inputs), summed across the wave; every lane receives them.
+// The lane's share of the outputs of a site network on one row (bits s0/s1, wave-uniform, already cut
+// to the network's inputs).
 template <int HPL>
-__device__ __forceinline__ void site_row(const SiteLds& s, const SiteRegs<HPL>& g, int hidden, int n_out, uint64_t s0, uint64_t s1, int lane,
-                                         float out[4]) {
+__device__ __forceinline__ void site_row(const SiteLds& s, const SiteRegs<HPL>& g, uint64_t s0, uint64_t s1, int lane, float (&part)[4]) {
+    using Vec = typename UnitVec<HPL>::type;
+    constexpr int V = UnitVec<HPL>::V;
+    constexpr int N = HPL / V;
+    const Vec* w1 = reinterpret_cast<const Vec*>(s.w1) + lane;
     float acc[HPL];
+    const auto add = [&](int k, const float (&to)[HPL]) {
+        Vec col[N];
 #pragma unroll
-    for (int j = 0; j < HPL; ++j) {
-        acc[j] = g.b1[j];
-    }
-    for (int half = 0; half < 2; ++half) {
-        uint64_t m = half ? s1 : s0;
-        while (m) {
-            const int k = 64 * half + __builtin_ctzll(m);
-            m &= m - 1;
-            const float* col = s.w1 + static_cast<size_t>(k) * hidden + lane;
+        for (int q = 0; q < N; ++q) {
+            col[q] = w1[(k * N + q) * 64];
+        }
 #pragma unroll
-            for (int j = 0; j < HPL; ++j) {
-                acc[j] += col[64 * j];
+        for (int j = 0; j < HPL; ++j) {
+            if constexpr (V == 1) {
+                acc[j] = to[j] + col[j][0];
+            } else {
+                acc[j] = to[j] + col[j / V][j % V];
             }
         }
+    };
+    if (s0 != 0ull) {
+        add(__builtin_ctzll(s0), g.b1);
+        s0 &= s0 - 1;
+    } else if (s1 != 0ull) {
+        add(64 + __builtin_ctzll(s1), g.b1);
+        s1 &= s1 - 1;
+    } else {
+#pragma unroll
+        for (int j = 0; j < HPL; ++j) {
+            acc[j] = g.b1[j];
+        }
     }
-    float part[4] = {0.f, 0.f, 0.f, 0.f};
+    while (s0 != 0ull) {
+        add(__builtin_ctzll(s0), acc);
+        s0 &= s0 - 1;
+    }
+    while (s1 != 0ull) {
+        add(64 + __builtin_ctzll(s1), acc);
+        s1 &= s1 - 1;
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        part[c] = 0.f;
+    }
 #pragma unroll
     for (int j = 0; j < HPL; ++j) {
         const float h = acc[j] * __builtin_amdgcn_rcpf(1.0f + __expf(-acc[j]));  // SiLU
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            part[c] += h * g.w2[c][j];
+            part[c] = __fmaf_rn(h, g.w2[c][j], part[c]);
         }
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        out[c] = c < n_out ? wave_sum(part[c]) + g.b2[c] : 0.f;
     }
 }
 
@@ -386,20 +442,52 @@ __device__ __forceinline__ void cut_bits(uint64_t& s0, uint64_t& s1, int n_bits)
     }
 }
 
+// The outputs of a staged site network on the wave's rows (rows_here of them, lane = row, bits b0/b1).
+template <int HPL>
+__device__ __forceinline__ void site_rows(const SiteLds& s, int n_out, int k_rows, int rows_here, uint64_t b0, uint64_t b1, int lane,
+                                          float (&mine)[4]) {
+    const SiteRegs<HPL> g = site_regs<HPL>(s, n_out, lane);
+    const int from = 16 * ((lane & 15) >> 2) + 4 * (lane & 3);  // the lanes that receive a row's outputs
+    for (int t = 0; kFusedTile * t < rows_here; ++t) {
+        float out = 0.f;
+        for (int q = 0; q < 4; ++q) {  // rows past rows_here are computed as empty ones
+            float part[4][4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int r = kFusedTile * t + 4 * q + v;
+                uint64_t s0 = wave_read64(b0, r), s1 = wave_read64(b1, r);
+                cut_bits(s0, s1, k_rows);
+                site_row<HPL>(s, g, s0, s1, lane, part[v]);
+            }
+            const float sum = row_sums(part, lane);
+            const float r0 = __shfl(sum, lane & 15), r1 = __shfl(sum, 16 + (lane & 15));
+            const float r2 = __shfl(sum, 32 + (lane & 15)), r3 = __shfl(sum, 48 + (lane & 15));
+            out = lane >> 4 == q ? ((r0 + r1) + r2) + r3 : out;
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float v = __shfl(out, from + c);
+            mine[c] = lane >> 4 == t ? v + g.b2[c] : mine[c];
+        }
+    }
+}
+
 // Forward of the whole network: log-amplitude (double) and phase per config.
 template <int HPL>
 __global__ void __launch_bounds__(kFusedThreads)
-    network_fused_kernel(int64_t n, int n_sites, int spin_up, int spin_down, const uint8_t* __restrict__ configs, int n_qubytes,
+    network_fused_kernel(int64_t n, int tiles, int n_sites, int spin_up, int spin_down, const uint8_t* __restrict__ configs, int n_qubytes,
                          const int64_t* __restrict__ ordering_reversed, const float* __restrict__ w1, const float* __restrict__ b1,
                          const float* __restrict__ w2, const float* __restrict__ b2, const float* __restrict__ wp1,
                          const float* __restrict__ bp1, const float* __restrict__ wp2, const float* __restrict__ bp2,
                          double* __restrict__ amplitude, float* __restrict__ phase) {
-    extern __shared__ float lds[];
+    extern __shared__ __attribute__((aligned(16))) float lds[];
     constexpr int H = 64 * HPL;
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int64_t row = static_cast<int64_t>(blockIdx.x) * kFusedThreads + threadIdx.x;
-    const bool valid = row < n;
+    const int64_t wave_row0 = (static_cast<int64_t>(blockIdx.x) * kFusedWaves + (threadIdx.x >> 6)) * (kFusedTile * tiles);
+    const int64_t left = n - wave_row0;
+    const int rows_here = static_cast<int>(left < 0 ? 0 : (left > kFusedTile * tiles ? kFusedTile * tiles : left));
+    const int64_t row = wave_row0 + lane;
+    const bool valid = lane < rows_here;
     // the own row's bits in sampling order
     uint64_t b0 = 0, b1w = 0;
     if (valid) {
@@ -421,8 +509,6 @@ __global__ void __launch_bounds__(kFusedThreads)
             }
         }
     }
-    const int64_t wave_row0 = static_cast<int64_t>(blockIdx.x) * kFusedThreads + 64 * wave;
-    const int rows_here = static_cast<int>(n - wave_row0 < 0 ? 0 : (n - wave_row0 > 64 ? 64 : n - wave_row0));
     const SiteLds s = site_lds(lds, 2 * n_sites, H);
     double total = 0.0;
     int up = 0, down = 0;
@@ -432,26 +518,14 @@ __global__ void __launch_bounds__(kFusedThreads)
         const int n_out = is_phase ? 1 : 4;
         __syncthreads();
         if (is_phase) {
-            stage_site(s, wp1, k_rows, bp1, wp2, bp2, 1, H);
+            stage_site<HPL>(s, wp1, k_rows, bp1, wp2, bp2, 1);
         } else {
-            stage_site(s, w1 + static_cast<size_t>(site) * (site - 1) * H, k_rows, b1 + static_cast<size_t>(site) * H,
-                       w2 + static_cast<size_t>(site) * 4 * H, b2 + 4 * site, 4, H);
+            stage_site<HPL>(s, w1 + static_cast<size_t>(site) * (site - 1) * H, k_rows, b1 + static_cast<size_t>(site) * H,
+                            w2 + static_cast<size_t>(site) * 4 * H, b2 + 4 * site, 4);
         }
         __syncthreads();
-        const SiteRegs<HPL> g = site_regs<HPL>(s, H, n_out, lane);
         float mine[4] = {0.f, 0.f, 0.f, 0.f};
-        for (int r = 0; r < rows_here; ++r) {
-            uint64_t s0 = wave_read64(b0, r), s1 = wave_read64(b1w, r);
-            cut_bits(s0, s1, k_rows);
-            float out[4];
-            site_row<HPL>(s, g, H, n_out, s0, s1, lane, out);
-            if (lane == r) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    mine[c] = out[c];
-                }
-            }
-        }
+        site_rows<HPL>(s, n_out, k_rows, rows_here, b0, b1w, lane, mine);
         if (!valid) {
             continue;
         }
@@ -479,42 +553,30 @@ __global__ void __launch_bounds__(kFusedThreads)
 // Gumbel-perturbed values, as children_kernel computes them from given logits.
 template <int HPL>
 __global__ void __launch_bounds__(kFusedThreads)
-    sampler_fused_kernel(int64_t n, int site, int n_sites, int spin_up, int spin_down, const uint64_t* __restrict__ prefix, int words,
+    sampler_fused_kernel(int64_t n, int tiles, int site, int n_sites, int spin_up, int spin_down, const uint64_t* __restrict__ prefix, int words,
                          const float* __restrict__ w1, const float* __restrict__ b1, const float* __restrict__ w2,
                          const float* __restrict__ b2, const float* __restrict__ unperturbed, const float* __restrict__ perturbed,
                          const float* __restrict__ uniform, uint64_t seed, float* __restrict__ child_unperturbed,
                          float* __restrict__ child_perturbed) {
-    extern __shared__ float lds[];
+    extern __shared__ __attribute__((aligned(16))) float lds[];
     constexpr int H = 64 * HPL;
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int64_t row = static_cast<int64_t>(blockIdx.x) * kFusedThreads + threadIdx.x;
-    const bool valid = row < n;
+    const int64_t wave_row0 = (static_cast<int64_t>(blockIdx.x) * kFusedWaves + (threadIdx.x >> 6)) * (kFusedTile * tiles);
+    const int64_t left = n - wave_row0;
+    const int rows_here = static_cast<int>(left < 0 ? 0 : (left > kFusedTile * tiles ? kFusedTile * tiles : left));
+    const int64_t row = wave_row0 + lane;
+    const bool valid = lane < rows_here;
     uint64_t b0 = 0, b1w = 0;
     if (valid) {
         b0 = prefix[row * words];
         b1w = words > 1 ? prefix[row * words + 1] : 0ull;
     }
-    const int64_t wave_row0 = static_cast<int64_t>(blockIdx.x) * kFusedThreads + 64 * wave;
-    const int rows_here = static_cast<int>(n - wave_row0 < 0 ? 0 : (n - wave_row0 > 64 ? 64 : n - wave_row0));
     const SiteLds s = site_lds(lds, 2 * site, H);
-    stage_site(s, w1 + static_cast<size_t>(site) * (site - 1) * H, 2 * site, b1 + static_cast<size_t>(site) * H,
-               w2 + static_cast<size_t>(site) * 4 * H, b2 + 4 * site, 4, H);
+    stage_site<HPL>(s, w1 + static_cast<size_t>(site) * (site - 1) * H, 2 * site, b1 + static_cast<size_t>(site) * H,
+                    w2 + static_cast<size_t>(site) * 4 * H, b2 + 4 * site, 4);
     __syncthreads();
-    const SiteRegs<HPL> g = site_regs<HPL>(s, H, 4, lane);
     float mine[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int r = 0; r < rows_here; ++r) {
-        uint64_t s0 = wave_read64(b0, r), s1 = wave_read64(b1w, r);
-        cut_bits(s0, s1, 2 * site);
-        float out[4];
-        site_row<HPL>(s, g, H, 4, s0, s1, lane, out);
-        if (lane == r) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                mine[c] = out[c];
-            }
-        }
-    }
+    site_rows<HPL>(s, 4, 2 * site, rows_here, b0, b1w, lane, mine);
     if (!valid) {
         return;
     }
@@ -558,6 +620,25 @@ int by_hidden(int hidden, F&& f) {
 }
 
 size_t fused_lds_bytes(int k_max, int hidden) { return (static_cast<size_t>(k_max) * hidden + 5 * static_cast<size_t>(hidden) + 4) * sizeof(float); }
+
+// Work-groups, and tiles of 16 rows a wave.  A work-group's weights fill most of a CU's LDS, so the
+// work-groups run 256 at a time: the tiles that leave the fewest rows' time in those rounds, and of
+// these the most (each work-group stages the weights).  100,000 rows in 98 work-groups of 1024: 3.2 ms
+// for the 26-site forward and 3.5 for the 26 sampling steps of width 512; in 196 of 512: 1.4 and 1.4.
+unsigned fused_grid(int64_t n, int* tiles) {
+    int64_t least = 0, grid = 0;
+    for (int t = kFusedMaxTiles; t >= 1; --t) {
+        const int64_t rows = static_cast<int64_t>(kFusedWaves) * kFusedTile * t;
+        const int64_t blocks = (n + rows - 1) / rows;
+        const int64_t rounds = (blocks + 255) / 256 * t;
+        if (grid == 0 || rounds < least) {
+            least = rounds;
+            grid = blocks;
+            *tiles = t;
+        }
+    }
+    return static_cast<unsigned>(grid);
+}
 
 constexpr size_t kFusedMaxLds = 160 * 1024;
 
@@ -610,12 +691,13 @@ int network_forward_fused(int64_t n, int n_sites, int hidden, int spin_up, int s
         return set_error(QMB_ERR_ARGUMENT, "null pointer argument");
     }
     const size_t lds = fused_lds_bytes(2 * n_sites, hidden);
-    const unsigned grid = static_cast<unsigned>((n + kFusedThreads - 1) / kFusedThreads);
+    int tiles = 0;
+    const unsigned grid = fused_grid(n, &tiles);
     return by_hidden(hidden, [&](auto hc) -> int {
         constexpr int HPL = decltype(hc)::value;
         QMB_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&network_fused_kernel<HPL>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                         static_cast<int>(lds)));
-        network_fused_kernel<HPL><<<grid, kFusedThreads, lds, stream>>>(n, n_sites, spin_up, spin_down, configs, n_qubytes, ordering_reversed,
+        network_fused_kernel<HPL><<<grid, kFusedThreads, lds, stream>>>(n, tiles, n_sites, spin_up, spin_down, configs, n_qubytes, ordering_reversed,
                                                                        w1, b1, w2, b2, wp1, bp1, wp2, bp2, amplitude, phase);
         QMB_CHECK_LAUNCH();
         return QMB_OK;
@@ -640,12 +722,13 @@ int sampler_step_fused(int64_t n, int site, int n_sites, int hidden, int spin_up
         return set_error(QMB_ERR_ARGUMENT, "null pointer argument");
     }
     const size_t lds = fused_lds_bytes(2 * site, hidden);
-    const unsigned grid = static_cast<unsigned>((n + kFusedThreads - 1) / kFusedThreads);
+    int tiles = 0;
+    const unsigned grid = fused_grid(n, &tiles);
     return by_hidden(hidden, [&](auto hc) -> int {
         constexpr int HPL = decltype(hc)::value;
         QMB_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&sampler_fused_kernel<HPL>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                         static_cast<int>(fused_lds_bytes(2 * n_sites, hidden))));
-        sampler_fused_kernel<HPL><<<grid, kFusedThreads, lds, stream>>>(n, site, n_sites, spin_up, spin_down, prefix, words, w1, b1, w2, b2,
+        sampler_fused_kernel<HPL><<<grid, kFusedThreads, lds, stream>>>(n, tiles, site, n_sites, spin_up, spin_down, prefix, words, w1, b1, w2, b2,
                                                                        unperturbed, perturbed, uniform, seed, child_unperturbed,
                                                                        child_perturbed);
         QMB_CHECK_LAUNCH();

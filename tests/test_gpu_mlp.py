@@ -250,3 +250,36 @@ def test_fused_sampler_matches_reference_algorithm(cuda_device: torch.device, ba
     with torch.no_grad():
         want = _ref_generate(net, batch, uniforms)
     assert torch.equal(configs, want)
+
+
+@pytest.mark.parametrize("sites,hidden", [(1, 64), (3, 128), (26, 512), (33, 256), (37, 512), (64, 64)])
+def test_fused_rows_are_independent_of_the_launch(cuda_device: torch.device, sites: int, hidden: int) -> None:
+    """A row's value is the same bits whatever the number of rows beside it (tiles of 16 rows, 1 to 4 a
+    wave, 256 work-groups a round), and whatever the weights of the inputs it does not set."""
+    up = (sites + 1) // 2
+    net = _net(sites, up, sites // 2, (hidden,), 1, torch.float32, cuda_device, seed=sites)
+    rng = np.random.default_rng(sites)
+    n = {1: 260_000, 3: 190_000, 64: 70_000}.get(sites, 5000)  # 4, 3 and 2 tiles a wave, else 1
+    bits = np.zeros((n, sites, 2), dtype=np.uint8)
+    for spin, count in ((0, up), (1, sites // 2)):
+        rank = rng.random((n, sites)).argsort(axis=1)
+        bits[:, :, spin] = rank < count
+    x = torch.from_numpy(np.packbits(bits.reshape(n, 2 * sites), axis=1, bitorder="little")).to(cuda_device)
+    with torch.no_grad():
+        for p in net.parameters():
+            p.mul_(0.3)
+        assert net._fused_ok()  # pylint: disable=protected-access
+        want = torch.view_as_real(net(x)).view(torch.int64)
+        for rows in (1, 15, 16, 17, 255, 256, 257, 513, 1025):
+            got = torch.view_as_real(net(x[-rows:])).view(torch.int64)
+            assert torch.equal(got, want[-rows:]), rows
+        k = 2 * (sites // 2)  # an input: the up bit of the middle site
+        for m in [*net.amplitude, net.phase]:
+            for p in m.parameters():
+                if p.dim() == 2 and p.shape[0] == hidden and p.shape[1] > k:
+                    p[:, k] = torch.inf
+        unset = torch.from_numpy(bits[:, sites // 2, 0] == 0).to(cuda_device)
+        got = torch.view_as_real(net(x)).view(torch.int64)
+        assert torch.equal(got[unset], want[unset])
+        if sites > 1:
+            assert bool(unset.any())
