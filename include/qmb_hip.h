@@ -269,7 +269,7 @@ typedef struct qmb_pairs {
     double* coef_re;   /* [n_pairs * n_pairs] real parts, filled by qmb_pairs_set_real */
     double* diag;      /* [1 + n_bits + n_pairs][2] */
     int64_t* counts;   /* device: {pair-excitation terms, diagonal terms, entries with a nonzero imaginary
-                          part (after qmb_pairs_set_real), 0} */
+                          part and entries that are not finite (both after qmb_pairs_set_real)} */
 } qmb_pairs;
 
 int qmb_pairs_workspace_size(int n_qubytes, size_t* bytes);

@@ -194,7 +194,8 @@ int pairs_layout(Carver& cv, int n_qubytes, qmb_pairs* out) {
     return QMB_OK;
 }
 
-// Real parts of the merged coefficients; counts[2] += entries with a nonzero imaginary part.
+// Real parts of the merged coefficients; counts[2] += entries with a nonzero imaginary part, counts[3] +=
+// entries that are not finite.
 __global__ void pairs_real_kernel(const double2* __restrict__ coef, int64_t n, double* __restrict__ re, int64_t* __restrict__ counts) {
     const int64_t k = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
     if (k >= n) {
@@ -204,6 +205,9 @@ __global__ void pairs_real_kernel(const double2* __restrict__ coef, int64_t n, d
     re[k] = v.x;
     if (v.y != 0.0) {
         atomicAdd(reinterpret_cast<unsigned long long*>(&counts[2]), 1ull);
+    }
+    if (!(fabs(v.x) < INFINITY)) {
+        atomicAdd(reinterpret_cast<unsigned long long*>(&counts[3]), 1ull);
     }
 }
 
@@ -1382,6 +1386,8 @@ struct PairParams {
     double2* out;
     const double2* in2;  // second input/output of a two-vector pass (NV = 2), else null
     double2* out2;
+    const int64_t* table_counts;  // qmb_pairs.counts
+    int dense;                    // the bins above 32 entries are pair_dense_kernel's
 };
 
 // The lanes' entries as the rows of a group read them, in this wave's LDS: the amplitude with the
@@ -1693,6 +1699,32 @@ __device__ __forceinline__ void mark_overflow(double2* out) {
     out[0] = make_double2(__longlong_as_double(0x7ff8000000000000ll), __longlong_as_double(0x7ff8000000000000ll));
 }
 
+constexpr int kDenseFirst = kExactBins + 2;  // groups above 64 entries, see pair_dense_kernel
+constexpr int kDenseGroups = 8;
+constexpr uint32_t kDensePanels = 128;
+
+// List elements of a group of the bin, at least.
+__device__ __forceinline__ uint32_t least_tiles(int bin) {
+    const int k = bin - kExactBins;
+    return k < 2 ? 1u : (k < 4 ? 2u : static_cast<uint32_t>(k) - 1u);
+}
+
+// The list elements of a panel of eight groups, and the bin's panels.
+__device__ __forceinline__ uint32_t panel_window(int bin) { return kDenseGroups * least_tiles(bin); }
+__device__ __forceinline__ uint32_t bin_panels(const CoreBins* bins, int bin) { return (bins->groups[bin] + panel_window(bin) - 1u) / panel_window(bin); }
+
+// Whether the groups above 64 entries go to pair_dense_kernel: a panel takes one CU 20 to 50 us, so that
+// a few panels end as a tail (12,000 rows of 52 spin orbitals: 48 us, 100 with their 17 panels; 100,000 rows of
+// 40 take 267 us, 286 with 171 panels, which an index of kDenseMin entries no longer notices).
+__device__ __forceinline__ bool dense_bins(const CoreBins* bins) {
+    uint32_t panels = 0;
+#pragma unroll
+    for (int bin = kDenseFirst; bin < kSplitBin; ++bin) {
+        panels += bin_panels(bins, bin);
+    }
+    return panels >= kDensePanels;
+}
+
 // Persistent waves over the units of the bins.  Every wave leaves when the units are done.
 template <bool ADJ, bool REAL, int NV>
 __global__ __launch_bounds__(kBlock) void pair_kernel(PairParams p) {
@@ -1706,9 +1738,239 @@ __global__ __launch_bounds__(kBlock) void pair_kernel(PairParams p) {
         }
         return;
     }
-    const uint32_t units = p.bins->unit_start[kBins];
-    for (uint32_t u = wave; u < units; u += nwaves) {
+    // the largest bins stand right after the split bin
+    const uint32_t skip_at = p.bins->unit_start[1];
+    const uint32_t skip = p.dense && dense_bins(p.bins) ? p.bins->unit_start[1 + kSplitBin - kDenseFirst] - skip_at : 0u;
+    const uint32_t units = p.bins->unit_start[kBins] - skip;
+    for (uint32_t i = wave; i < units; i += nwaves) {
+        const uint32_t u = i < skip_at ? i : i + skip;
         pair_unit<ADJ, REAL, NV, NV == 1 ? kPairBatch : kPairBatch / 2>(p, u, lane, stages[threadIdx.x >> 6]);
+    }
+}
+
+// The groups above 32 entries of a real table, eight at a time as a dense product on the matrix unit.
+// A panel is eight groups that follow each other in a bin; its slots are the U pair slots that any of
+// them has, and with S the table at these slots and B the [U][16] amplitudes (eight groups, real and imaginary
+// part, zero where a group has no such entry) the panel's contributions are S^T B (ADJ: S B).  The
+// group kernel gathers one coefficient per pair of entries, a cache line each, and that bounds it;
+// here a coefficient is read once for eight groups, in rows.  1M rows of 52 spin orbitals: forward 4.68 ->
+// 4.32 ms, adjoint (whose gathers fall in as many rows as lanes) 7.87 -> 5.92; 200,000 rows of 76:
+// 3.94 -> 3.27 and 5.44 -> 4.87 (most of its panels are walked; the waves of a work-group then share the rows
+// of the table).  The time of a dense panel is half products, half the steps around them.
+// A panel is dense where its pairs of entries pay for the products of the slots that a group lacks:
+// from kDenseGain pairs per matrix instruction (16 x 16 x 4, eight groups' 512 pairs at most; a local
+// energy step of 200,000 sampled rows of 76 spin orbitals: 9.1 ms from 20, 9.2 from 32, 11.1 without panels), U within
+// the LDS, and a finite table (a zero amplitude times infinity would reach other groups' rows).  The
+// other panels are walked as in pair_kernel.
+// Matrix operands: lane l holds S of row slot l % 16 and column slot l / 16 of four, and B of that column slot
+// at l % 16; results v = 0..3 are row slot 4 v + l / 16 at l % 16, so that neighbouring lanes add the
+// two components of one output row.
+constexpr int kDenseThreads = 1024;
+constexpr int kDenseWaves = kDenseThreads / 64;
+constexpr int kDenseStep = 32;        // column slots whose coefficients are in flight
+constexpr int kDenseGain = 20;
+constexpr int kDenseSlots = 8192;     // pair slots of 16 bytes of sites: 8128
+constexpr int kDenseWindow = 64;      // list elements of a panel, at most
+constexpr int kDenseUnion = 960;      // U that fits the LDS
+// Entries of the index from which panels are made, forward with / without and adjoint with / without, us:
+//   9.1M (52 spin orbitals, 100,000 rows)  317 / 261     432 / 408
+//  18.2M (52, 200,000)                     583 / 562     823 / 903
+//  23.0M (60, 150,000)                     696 / 625     980 / 976
+//  36.4M (52, 400,000)                    1297 / 1347   1807 / 2192
+//  61.2M (60, 400,000)                    1717 / 1900   2265 / 2491
+constexpr int64_t kDenseMin = 1 << 25;
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+struct DenseLds {
+    double b[kDenseUnion * 16];
+    uint32_t rows[kDenseUnion * kDenseGroups];  // row | sign << 31 of a slot in a group, ~0: none
+    uint32_t slots[kDenseUnion];
+    uint64_t bits[kDenseSlots / 64];
+    uint32_t before[kDenseSlots / 64];  // used slots before the word
+    uint2 groups[kDenseWindow];         // first entry, size
+    uint32_t n_groups;
+    uint32_t used;
+};
+
+template <bool ADJ, int NV>
+__global__ __launch_bounds__(kDenseThreads) void pair_dense_kernel(PairParams p) {
+    extern __shared__ uint64_t smem[];
+    static_assert(kDenseUnion % kDenseStep == 0 && sizeof(DenseLds) <= 160 * 1024 && sizeof(Stage<NV>) * kDenseWaves <= sizeof(DenseLds::b), "LDS");
+    DenseLds& L = *reinterpret_cast<DenseLds*>(smem);
+    if (p.counts[2] != 0 || !dense_bins(p.bins)) {
+        return;  // pair_kernel marks the overflow, or walks all bins
+    }
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool fermi = p.particle_cut == 1;
+    const bool finite = p.table_counts[3] == 0;
+    const uint32_t np = static_cast<uint32_t>(p.n_pairs);
+    const auto place = [&](uint32_t slot) {
+        return L.before[slot >> 6] + static_cast<uint32_t>(__popcll(L.bits[slot >> 6] & ((1ull << (slot & 63u)) - 1ull)));
+    };
+    for (uint32_t panel = blockIdx.x;; panel += gridDim.x) {
+        uint32_t local = panel, window = 0;
+        int bin = kSplitBin - 1;
+        for (; bin >= kDenseFirst; --bin) {
+            window = panel_window(bin);
+            const uint32_t here = bin_panels(p.bins, bin);
+            if (local < here) {
+                break;
+            }
+            local -= here;
+        }
+        if (bin < kDenseFirst) {
+            return;  // the whole work-group
+        }
+        __syncthreads();  // the previous panel's LDS is done with
+        if (tid < kDenseSlots / 64) {
+            L.bits[tid] = 0ull;
+        }
+        if (wave == 0) {
+            // the groups that start in the panel's list elements (at most eight, save whole ones)
+            const uint32_t at = local * window + static_cast<uint32_t>(lane);
+            const bool in = lane < static_cast<int>(window) && at < p.bins->groups[bin];
+            const uint2 item = in ? p.glist[p.bins->list_base[bin] + at] : make_uint2(0u, 0u);
+            const bool whole = (item.y & kWholeGroup) != 0u;
+            const bool start = in && (whole || (item.y >> 16) == 0u);
+            const uint64_t starts = __ballot(start);
+            if (start) {
+                L.groups[__popcll(starts & ((1ull << lane) - 1ull))] = make_uint2(item.x, whole ? item.y & ~kWholeGroup : item.y & kTiledMax);
+            }
+            if (lane == 0) {
+                L.n_groups = static_cast<uint32_t>(__popcll(starts));
+            }
+        }
+        __syncthreads();
+        const uint32_t n_groups = L.n_groups;
+        const int own_group = wave % kDenseGroups;  // two waves to a group
+        const uint32_t own_first = static_cast<uint32_t>(wave / kDenseGroups * 64 + lane);
+        const uint2 own = static_cast<uint32_t>(own_group) < n_groups ? L.groups[own_group] : make_uint2(0u, 0u);
+        bool dense = finite && n_groups <= kDenseGroups;
+        uint64_t pairs = 0;
+        for (uint32_t g = 0; g < n_groups; ++g) {
+            pairs += static_cast<uint64_t>(L.groups[g].y) * L.groups[g].y;
+            dense = dense && L.groups[g].y <= kDenseUnion;
+        }
+        if (dense) {
+            for (uint32_t e = own_first; e < own.y; e += 64 * kDenseWaves / kDenseGroups) {
+                const uint32_t slot = binned_entry(p.mvals[own.x + e], fermi).slot;
+                atomicOr(reinterpret_cast<unsigned long long*>(&L.bits[slot >> 6]), 1ull << (slot & 63u));
+            }
+            __syncthreads();
+            if (wave == 0) {
+                const uint32_t c0 = static_cast<uint32_t>(__popcll(L.bits[2 * lane])), c1 = static_cast<uint32_t>(__popcll(L.bits[2 * lane + 1]));
+                uint32_t incl = c0 + c1;
+#pragma unroll
+                for (int d = 1; d < 64; d <<= 1) {
+                    const uint32_t o = __shfl_up(incl, d);
+                    incl += lane >= d ? o : 0u;
+                }
+                L.before[2 * lane] = incl - c0 - c1;
+                L.before[2 * lane + 1] = incl - c1;
+                if (lane == 63) {
+                    L.used = incl;
+                }
+            }
+            __syncthreads();
+            const uint64_t tiles = (L.used + 15u) / 16u;
+            dense = L.used <= kDenseUnion && pairs >= kDenseGain * tiles * tiles * 4u;
+        }
+        if (!dense) {
+            __syncthreads();
+            Stage<NV>& st = reinterpret_cast<Stage<NV>*>(L.b)[wave];
+            uint32_t item = 0;
+            for (uint32_t g = 0; g < n_groups; ++g) {
+                const uint2 group = L.groups[g];
+                const bool whole = group.y > kTiledMax;
+                for (uint32_t t = 0; t < group_tiles(group.y); ++t, ++item) {
+                    if (item % kDenseWaves == static_cast<uint32_t>(wave)) {
+                        pair_big<ADJ, true, NV, kPairBatch>(p, group.x, group.y, 64u * t, whole ? group.y : 64u * t + 1u, lane, st);
+                    }
+                }
+            }
+            continue;
+        }
+        const int used = static_cast<int>(L.used);
+        const int n_rows = (used + 15) / 16 * 16;
+        const int n_cols = (used + kDenseStep - 1) / kDenseStep * kDenseStep;
+        {
+            const int word = tid >> 3, byte = 8 * (tid & 7);  // kDenseThreads = 8 * words
+            const uint64_t bits = L.bits[word];
+            uint32_t m = static_cast<uint32_t>(bits >> byte) & 0xffu;
+            uint32_t at = L.before[word] + static_cast<uint32_t>(__popcll(bits & ((1ull << byte) - 1ull)));
+            while (m) {
+                L.slots[at++] = static_cast<uint32_t>(64 * word + byte + __builtin_ctz(m));
+                m &= m - 1;
+            }
+            if (used + tid < n_cols) {
+                L.slots[used + tid] = 0u;
+            }
+        }
+        for (int t = tid; t < n_rows * kDenseGroups; t += kDenseThreads) {
+            L.rows[t] = ~0u;
+        }
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            for (int t = tid; t < n_cols * 16; t += kDenseThreads) {
+                L.b[t] = 0.0;
+            }
+            __syncthreads();
+            for (uint32_t i = own_first; i < own.y; i += 64 * kDenseWaves / kDenseGroups) {
+                const Entry e = binned_entry(p.mvals[own.x + i], fermi);
+                const uint32_t at = place(e.slot);
+                const double2 x = signed_by((v == 0 ? p.in : p.in2)[e.row], e.sign);
+                L.rows[at * kDenseGroups + own_group] = e.row | (e.sign << 31);
+                L.b[16 * at + 2 * own_group] = x.x;
+                L.b[16 * at + 2 * own_group + 1] = x.y;
+            }
+            __syncthreads();
+            double* out = reinterpret_cast<double*>(v == 0 ? p.out : p.out2);
+            const int quad = lane >> 4, col = lane & 15;
+            for (int r0 = 16 * wave; r0 < n_rows; r0 += 16 * kDenseWaves) {
+                const uint32_t row_slot = L.slots[r0 + col];
+                const auto load = [&](int k) {
+                    const uint32_t slot = L.slots[k + quad];
+                    return p.coef_re[ADJ ? row_slot * np + slot : slot * np + row_slot];
+                };
+                f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+                double next[kDenseStep / 4];
+#pragma unroll
+                for (int q = 0; q < kDenseStep / 4; ++q) {
+                    next[q] = load(4 * q);
+                }
+                for (int k0 = 0; k0 < n_cols; k0 += kDenseStep) {
+                    double a[kDenseStep / 4];
+#pragma unroll
+                    for (int q = 0; q < kDenseStep / 4; ++q) {
+                        a[q] = next[q];
+                    }
+                    if (k0 + kDenseStep < n_cols) {
+#pragma unroll
+                        for (int q = 0; q < kDenseStep / 4; ++q) {
+                            next[q] = load(k0 + kDenseStep + 4 * q);
+                        }
+                    }
+#pragma unroll
+                    for (int q = 0; q < kDenseStep / 4; ++q) {
+                        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], L.b[16 * (k0 + 4 * q + quad) + col], acc, 0, 0, 0);
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t row = L.rows[(r0 + 4 * q + quad) * kDenseGroups + (col >> 1)];
+                    if (row != ~0u && acc[q] != 0.0) {
+                        const double x = (row >> 31) != 0u ? -acc[q] : acc[q];
+                        unsafeAtomicAdd(&out[2 * static_cast<int64_t>(row & 0x7fffffffu) + (lane & 1)], x);
+                    }
+                }
+            }
+            if (v + 1 < NV) {
+                __syncthreads();
+            }
+        }
     }
 }
 
@@ -2897,8 +3159,18 @@ unsigned group_grid(int64_t capacity) {
 }
 
 template <int NV>
-int launch_pairs(const PairParams& p, int64_t capacity, int mode, hipStream_t stream) {
+int launch_pairs(PairParams p, int64_t capacity, int mode, hipStream_t stream) {
     const unsigned grid = group_grid(capacity);
+    if (p.coef_re != nullptr && capacity >= kDenseMin && p.n_pairs <= kDenseSlots) {
+        p.dense = 1;
+        const auto go = [&](auto kernel) -> int {
+            QMB_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(DenseLds)));
+            kernel<<<256, kDenseThreads, sizeof(DenseLds), stream>>>(p);
+            QMB_CHECK_LAUNCH();
+            return QMB_OK;
+        };
+        QMB_TRY(mode == 1 ? go(&pair_dense_kernel<true, NV>) : go(&pair_dense_kernel<false, NV>));
+    }
     if (p.coef_re != nullptr) {
         mode == 1 ? pair_kernel<true, true, NV><<<grid, kBlock, 0, stream>>>(p) : pair_kernel<false, true, NV><<<grid, kBlock, 0, stream>>>(p);
     } else {
@@ -2930,6 +3202,7 @@ int apply_pairs(const qmb_pairs* pairs, const qmb_cores* cores, const qmb_target
     PairParams p{};
     p.coef = reinterpret_cast<const double2*>(pairs->coef);
     p.coef_re = pairs->real ? pairs->coef_re : nullptr;
+    p.table_counts = pairs->counts;
     p.n_pairs = pairs->n_pairs;
     p.particle_cut = pairs->particle_cut;
     p.mvals = cores->mvals;
@@ -3296,6 +3569,7 @@ int apply_structured_dual(const qmb_pairs* pairs, const qmb_singles* singles, co
         PairParams p{};
         p.coef = reinterpret_cast<const double2*>(pairs->coef);
         p.coef_re = pairs->real ? pairs->coef_re : nullptr;
+        p.table_counts = pairs->counts;
         p.n_pairs = pairs->n_pairs;
         p.particle_cut = pairs->particle_cut;
         p.mvals = cores2->mvals;

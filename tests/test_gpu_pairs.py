@@ -422,3 +422,45 @@ def test_groups_around_the_row_tiles(cuda_device: torch.device, order: int, size
     plain = pp.apply(terms, targets, cfg_t, vec, pp.MODE_ADJOINT, symmetric=pp.SYMMETRIC_OFF, pairs=False).cpu().numpy()
     got = pp.apply(terms, targets, cfg_t, vec, pp.MODE_ADJOINT, symmetric=pp.SYMMETRIC_OFF, pairs=True).cpu().numpy()
     assert np.abs(got - plain).max() <= 1e-12 * (np.abs(c).sum() * np.abs(psi).max())
+
+
+@pytest.mark.parametrize("size,shared,finite", [(80, True, True), (80, False, True), (129, True, True), (129, False, True), (80, True, False)])
+def test_panels_of_large_groups(cuda_device: torch.device, size: int, shared: bool, finite: bool) -> None:
+    """An index of over 2^25 entries takes its groups above 64 entries in panels of eight: groups of `size`
+    site pairs beside two of 36 spectators, the same pairs in each (dense products) or random ones
+    (partly walked), and the groups that the spectators make; with an infinite coefficient no panel is dense."""
+    nq, rng = 16, np.random.default_rng(size)
+    grid = [(a, b) for a in range(0, 32, 2) for b in range(1, 32, 2)]
+    combos = [(s, t) for s in range(32, 68) for t in range(32, s)]
+    combos = [combos[q] for q in rng.permutation(len(combos))[: 50_400 // size]]
+    rows = np.zeros((len(combos) * size, 8 * nq), dtype=np.uint8)
+    for k, (s, t) in enumerate(combos):
+        picked = range(size) if shared else rng.permutation(len(grid))[:size]
+        for j, q in enumerate(picked):
+            rows[k * size + j, [*grid[q], s, t]] = 1
+    rows[:, 68:] = 1
+    cfg = sy.sort_unique_configs(np.packbits(rows, axis=1, bitorder="little"))
+    n = len(cfg)
+    assert n == len(rows) and n * (64 * 63 // 2) >= 1 << 25
+    s, k, c = _pair_heavy_table(np.arange(48), 8000, 9)
+    c[:, 1] = 0.0
+    if not finite:
+        s = np.concatenate([s, np.array([[60, 62, 120, 122]], dtype=np.int16)])  # its target pair is held by every row
+        k = np.concatenate([k, np.array([[1, 1, 0, 0]], dtype=np.uint8)])
+        c = np.concatenate([c, np.array([[np.inf, 0.0]])])
+    cfg_t = _dev(cfg, cuda_device)
+    terms = pp.PreparedTerms(_dev(s, cuda_device), _dev(k, cuda_device), _dev(c, cuda_device), nq, 1)
+    targets = pp.PreparedTargets(cfg_t, nq, distinct=True)
+    assert terms.pairs_desc.real == 1
+    _, starts, _ = _core_index(targets, 2)
+    sizes = np.diff((starts & 0x7FFFFFFF).astype(np.int64))[starts[:-1] >> 31 == 0]
+    assert (sizes > 64).sum() >= 8 * 128  # panels enough
+    psi, g = sy.random_psi(n, 33), sy.random_psi(n, 34)
+    vec, gvec = (torch.view_as_real(_dev(x, cuda_device)).contiguous() for x in (psi, g))
+    want, asum, _ = orc.apply_within(1, cfg, psi, cfg, s, k, c)
+    got = pp.apply(terms, targets, cfg_t, vec, pp.MODE_FORWARD, symmetric=pp.SYMMETRIC_OFF, pairs=True).cpu().numpy()
+    assert np.all(np.abs(got[:, 0] + 1j * got[:, 1] - want) <= 1e-12 * asum + 1e-300)
+    bound = 1e-12 * np.abs(c[np.isfinite(c[:, 0])]).sum()
+    plain = pp.apply(terms, targets, cfg_t, gvec, pp.MODE_ADJOINT, symmetric=pp.SYMMETRIC_OFF, pairs=False).cpu().numpy()
+    got = pp.apply(terms, targets, cfg_t, gvec, pp.MODE_ADJOINT, symmetric=pp.SYMMETRIC_OFF, pairs=True).cpu().numpy()
+    assert np.abs(got - plain).max() <= bound * np.abs(g).max()
