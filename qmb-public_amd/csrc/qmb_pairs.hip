@@ -1075,6 +1075,10 @@ __global__ __launch_bounds__(kBlock) void bin_scatter_kernel(const uint32_t* __r
 // size.  The limit is the LDS: 17 bytes an entry and the sort's power of two.  Entries sort by (key,
 // emission index k * n + row), the order the general build's stable sort gives.
 constexpr int kSmallCores = 8192;
+// Up to this many entries one wave takes all units, in order: the sums of so small a set then come out
+// the same in every call (whole units spread over waves add to a row in the order they finish), for
+// about the time that the kernel's launch and the call around it take anyway.
+constexpr int kTinyCores = 512;
 constexpr int kSmallThreads = 1024;
 
 struct SmallLds {
@@ -1248,7 +1252,8 @@ __global__ __launch_bounds__(kSmallThreads) void cores_small_kernel(const uint64
     }
     __threadfence_block();
     __syncthreads();
-    for (int q = tid; q < n_groups; q += kSmallThreads) {
+    const int placers = cap <= kTinyCores ? 64 : kSmallThreads;  // one wave: always the same places
+    for (int q = tid; tid < placers && q < n_groups; q += placers) {
         const uint32_t first = L.start[q];
         const uint32_t size = L.start[q + 1] - first;
         uint32_t move = kSmallStay;
@@ -1730,8 +1735,8 @@ template <bool ADJ, bool REAL, int NV>
 __global__ __launch_bounds__(kBlock) void pair_kernel(PairParams p) {
     __shared__ Stage<NV> stages[kWavesPerBlock];
     const int lane = threadIdx.x & 63;
-    const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6))));
-    const uint32_t nwaves = gridDim.x * kWavesPerBlock;
+    const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>((blockIdx.x * blockDim.x + threadIdx.x) >> 6)));
+    const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
     if (p.counts[2] != 0) {
         if (wave == 0 && lane == 0) {
             mark_overflow(p.out);
@@ -2222,8 +2227,8 @@ template <int W, bool ADJ, int NV = 1>
 __global__ __launch_bounds__(kBlock) void single_kernel(SingleParams p) {
     __shared__ Stage<NV> stages[kWavesPerBlock];
     const int lane = threadIdx.x & 63;
-    const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6))));
-    const uint32_t nwaves = gridDim.x * kWavesPerBlock;
+    const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>((blockIdx.x * blockDim.x + threadIdx.x) >> 6)));
+    const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
     if (p.counts[2] != 0) {
         if (wave == 0 && lane == 0) {
             mark_overflow(p.out);
@@ -3154,9 +3159,10 @@ namespace {
 // Persistent waves of a group kernel: enough to fill every CU several times over, never more than the
 // entries can need (small sets: a wave per 32 entries).
 unsigned group_grid(int64_t capacity) {
-    const int64_t want = capacity / (32 * kWavesPerBlock) + 1;
+    const int64_t want = capacity <= kTinyCores ? 1 : capacity / (32 * kWavesPerBlock) + 1;
     return static_cast<unsigned>(want < 4096 ? want : 4096);
 }
+unsigned group_block(int64_t capacity) { return capacity <= kTinyCores ? 64u : static_cast<unsigned>(kBlock); }
 
 template <int NV>
 int launch_pairs(PairParams p, int64_t capacity, int mode, hipStream_t stream) {
@@ -3172,9 +3178,9 @@ int launch_pairs(PairParams p, int64_t capacity, int mode, hipStream_t stream) {
         QMB_TRY(mode == 1 ? go(&pair_dense_kernel<true, NV>) : go(&pair_dense_kernel<false, NV>));
     }
     if (p.coef_re != nullptr) {
-        mode == 1 ? pair_kernel<true, true, NV><<<grid, kBlock, 0, stream>>>(p) : pair_kernel<false, true, NV><<<grid, kBlock, 0, stream>>>(p);
+        mode == 1 ? pair_kernel<true, true, NV><<<grid, group_block(capacity), 0, stream>>>(p) : pair_kernel<false, true, NV><<<grid, group_block(capacity), 0, stream>>>(p);
     } else {
-        mode == 1 ? pair_kernel<true, false, NV><<<grid, kBlock, 0, stream>>>(p) : pair_kernel<false, false, NV><<<grid, kBlock, 0, stream>>>(p);
+        mode == 1 ? pair_kernel<true, false, NV><<<grid, group_block(capacity), 0, stream>>>(p) : pair_kernel<false, false, NV><<<grid, group_block(capacity), 0, stream>>>(p);
     }
     QMB_CHECK_LAUNCH();
     return QMB_OK;
@@ -3283,7 +3289,7 @@ int apply_singles(const qmb_singles* singles, const qmb_cores* cores, const qmb_
     p.out = reinterpret_cast<double2*>(out);
     const unsigned grid = group_grid(cores->capacity);
     auto go = [&](auto kernel) -> int {
-        kernel<<<grid, kBlock, 0, stream>>>(p);
+        kernel<<<grid, group_block(cores->capacity), 0, stream>>>(p);
         QMB_CHECK_LAUNCH();
         return QMB_OK;
     };
@@ -3559,9 +3565,9 @@ int apply_structured_dual(const qmb_pairs* pairs, const qmb_singles* singles, co
         p.out2 = vo2;
         const unsigned grid = group_grid(cores1->capacity);
         if (W == 1) {
-            mode == 1 ? single_kernel<1, true, 2><<<grid, kBlock, 0, stream>>>(p) : single_kernel<1, false, 2><<<grid, kBlock, 0, stream>>>(p);
+            mode == 1 ? single_kernel<1, true, 2><<<grid, group_block(cores1->capacity), 0, stream>>>(p) : single_kernel<1, false, 2><<<grid, group_block(cores1->capacity), 0, stream>>>(p);
         } else {
-            mode == 1 ? single_kernel<2, true, 2><<<grid, kBlock, 0, stream>>>(p) : single_kernel<2, false, 2><<<grid, kBlock, 0, stream>>>(p);
+            mode == 1 ? single_kernel<2, true, 2><<<grid, group_block(cores1->capacity), 0, stream>>>(p) : single_kernel<2, false, 2><<<grid, group_block(cores1->capacity), 0, stream>>>(p);
         }
         QMB_CHECK_LAUNCH();
     }
