@@ -21,8 +21,10 @@
 // at 16 times as many while it finds fewer than K entries (most connections do not exist or are
 // excluded).  Once the tied class fits the candidate buffer, one more pass collects every entry strictly
 // above the threshold prefix and the tied candidates; the candidates are ordered by (weight desc,
-// config asc) and the first K - above are kept.  All control lives in device memory, so the whole call
-// is enqueued without host synchronisation; passes that are not needed return at once.
+// config asc) and the first K - above are kept.  A class that does not fit although its weight is settled
+// to the last bit (one hopping magnitude and a uniform |psi|, say) is narrowed in the same way by the
+// digits of the config, ascending.  All control lives in device memory, so the whole call is enqueued
+// without host synchronisation; passes that are not needed return at once.
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 
@@ -61,6 +63,12 @@ struct FrState {
     double reach;    // |coef| |psi| of an entry with w >= lo is not below this
     int64_t active;  // rows that can reach it: a prefix
     uint64_t bound[kTries];
+    // Entries of one weight narrowed by config: those with `key & tie_mask` below tie_key are selected
+    // outright, equal to it candidates, above it not wanted (all of them candidates while the mask is 0).
+    uint64_t tie_key[kMaxWords];
+    uint64_t tie_mask[kMaxWords];
+    int32_t ties;  // more entries than the candidate buffer holds are tied on weight and tie_key
+    uint32_t tie_blocks;
 };
 
 // Reach of the weight with these bits: no product |coef| |psi| below it gives that weight.  The computed
@@ -111,6 +119,63 @@ __device__ __forceinline__ uint64_t weight_bits(const double2 cf, const double2 
     return static_cast<uint64_t>(__double_as_longlong(w));
 }
 
+// Digits of a config's key, the config as one big-endian number (word w of it: bytes 8 w to 8 w + 7), so
+// that keys order as configs do.  Digit d is bits [12 d, 12 d + 12) from the top; one may straddle words.
+__host__ __device__ inline int tie_levels(int n_qubytes) { return (8 * n_qubytes + kHistBits - 1) / kHistBits; }
+
+// Adds digit `value` of position d to key.
+template <int W>
+__device__ __forceinline__ void put_digit(uint64_t (&key)[W], int d, uint64_t value) {
+    const int first = kHistBits * d >> 6, r = kHistBits * d & 63;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        if (w == first) {
+            key[w] |= (value << (64 - kHistBits)) >> r;
+        }
+        if (w == first + 1 && r > 64 - kHistBits) {
+            key[w] |= value << (128 - kHistBits - r);
+        }
+    }
+}
+
+template <int W>
+__device__ __forceinline__ uint32_t get_digit(const uint64_t (&key)[W], int d) {
+    const int first = kHistBits * d >> 6, r = kHistBits * d & 63;
+    uint64_t v = 0ull;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        if (w == first) {
+            v |= (key[w] << r) >> (64 - kHistBits);
+        }
+        if (w == first + 1 && r > 64 - kHistBits) {
+            v |= key[w] >> (128 - kHistBits - r);
+        }
+    }
+    return static_cast<uint32_t>(v);
+}
+
+template <int W>
+struct TieRange {
+    uint64_t key[W], mask[W];
+    __device__ __forceinline__ explicit TieRange(const FrState* st) {
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            key[w] = st->tie_key[w];
+            mask[w] = st->tie_mask[w];
+        }
+    }
+    // -1, 0, 1: the config's settled digits below, equal to or above the tied ones.
+    __device__ __forceinline__ int side(const Cfg<W>& c) const {
+        int s = 0;
+#pragma unroll
+        for (int w = W - 1; w >= 0; --w) {
+            const uint64_t k = bswap64(c.w[w]) & mask[w];
+            s = k < key[w] ? -1 : (k > key[w] ? 1 : s);
+        }
+        return s;
+    }
+};
+
 // The pruning both passes share: terms whose |coef| with the tile's largest |psi| stays below the reach.
 struct PrunedHooks : ActionHooks {
     static constexpr bool kPruned = true;
@@ -144,20 +209,47 @@ struct HistAction : PrunedHooks {
     }
 };
 
+// The next config digit of the entries with the settled weight and the settled config digits.
+template <int W>
+struct TieAction : PrunedHooks {
+    uint32_t* hist;
+    uint64_t weight;
+    TieRange<W> range;
+    int digit;
+    __device__ TieAction(const FrParams& pp, uint32_t* h, int d)
+        : PrunedHooks(pp), hist(h), weight(pp.state->prefix), range(pp.state), digit(d) {}
+    __device__ __forceinline__ bool pre(int64_t i, uint32_t t, const Cfg<W>& o, int, uint64_t, uint64_t) {
+        return weight_bits(p.coefs[t], p.psi[i]) == weight && range.side(o) == 0;
+    }
+    __device__ __forceinline__ void post(int64_t, uint32_t, const Cfg<W>& o, int, int64_t j, bool) {
+        if (j >= 0) {
+            return;  // excluded
+        }
+        uint64_t key[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            key[w] = bswap64(o.w[w]);
+        }
+        atomicAdd(&hist[get_digit<W>(key, digit)], 1u);
+    }
+};
+
 template <int W>
 struct CollectAction : PrunedHooks {
     uint64_t lo;
     uint64_t hi;
-    __device__ explicit CollectAction(const FrParams& pp) : PrunedHooks(pp), lo(pp.state->lo), hi(pp.state->hi) {}
-    __device__ __forceinline__ bool pre(int64_t i, uint32_t t, const Cfg<W>&, int, uint64_t, uint64_t) {
-        return weight_bits(p.coefs[t], p.psi[i]) >= lo;
+    TieRange<W> range;
+    __device__ explicit CollectAction(const FrParams& pp) : PrunedHooks(pp), lo(pp.state->lo), hi(pp.state->hi), range(pp.state) {}
+    __device__ __forceinline__ bool pre(int64_t i, uint32_t t, const Cfg<W>& o, int, uint64_t, uint64_t) {
+        const uint64_t w = weight_bits(p.coefs[t], p.psi[i]);
+        return w >= lo && (w >= hi || range.side(o) <= 0);
     }
     __device__ __forceinline__ void post(int64_t i, uint32_t t, const Cfg<W>& o, int, int64_t j, bool) {
         if (j >= 0) {
             return;  // excluded
         }
         const uint64_t w = weight_bits(p.coefs[t], p.psi[i]);
-        if (w >= hi) {
+        if (w >= hi || range.side(o) < 0) {
             const unsigned long long s = atomicAdd(&p.state->n_above, 1ull);
             if (s < static_cast<unsigned long long>(p.k)) {
 #pragma unroll
@@ -229,6 +321,93 @@ __global__ __launch_bounds__(kEnumBlock) void fr_collect_kernel(FrParams p) {
     extern __shared__ uint64_t smem[];
     CollectAction<W> act(p);
     fr_enumerate<W>(p, smem, act);
+}
+
+// Entries of one weight that exceed the candidate buffer, digit d of their configs: every block counts, the
+// last one to finish picks the digit at which the running count from the lowest reaches what is needed
+// (a fence per block, but only where there are such ties; a kernel of its own for the choice would cost
+// every other call a launch a digit: the two to five launches without ties are 3 us of 620).  30,000 rows
+// of a 32-site Hubbard chain with |psi| = 1 and K = 5000 take 1.1 ms.
+template <int W>
+__global__ __launch_bounds__(kEnumBlock) void fr_tie_kernel(FrParams p, int d, int levels) {
+    extern __shared__ uint64_t smem[];
+    __shared__ uint32_t s_hist[kHistBins];
+    __shared__ unsigned long long s_wave[kEnumBlock / 64];
+    __shared__ bool s_last;
+    FrState* st = p.state;
+    if (st->ties == 0) {
+        return;  // uniform: every thread reads the same flag, which only the last block to finish changes
+    }
+    for (int b = threadIdx.x; b < kHistBins; b += kEnumBlock) {
+        s_hist[b] = 0;
+    }
+    __syncthreads();
+    TieAction<W> act(p, s_hist, d);
+    fr_enumerate<W>(p, smem, act);
+    __syncthreads();
+    for (int b = threadIdx.x; b < kHistBins; b += kEnumBlock) {
+        if (s_hist[b]) {
+            atomicAdd(&p.hist[b], static_cast<unsigned long long>(s_hist[b]));
+        }
+    }
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        s_last = atomicAdd(&st->tie_blocks, 1u) == gridDim.x - 1u;
+    }
+    __syncthreads();
+    if (!s_last) {
+        return;
+    }
+    __threadfence();
+    constexpr int kPer = kHistBins / kEnumBlock;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    unsigned long long v[kPer], sum = 0ull;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        unsigned long long* bin = &p.hist[kPer * static_cast<int>(threadIdx.x) + q];
+        v[q] = __hip_atomic_load(bin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *bin = 0ull;
+        sum += v[q];
+    }
+    unsigned long long incl = sum;
+    for (int k = 1; k < 64; k <<= 1) {
+        const unsigned long long o = __shfl_up(incl, k);
+        incl += lane >= k ? o : 0ull;
+    }
+    if (lane == 63) {
+        s_wave[wave] = incl;
+    }
+    __syncthreads();
+    unsigned long long cum = incl - sum;
+    for (int w = 0; w < wave; ++w) {
+        cum += s_wave[w];
+    }
+    const unsigned long long need = static_cast<unsigned long long>(st->cand_needed);
+    __syncthreads();  // every thread has it before one changes it
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        if (cum < need && cum + v[q] >= need) {  // one thread
+            uint64_t key[W], mask[W];
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                key[w] = st->tie_key[w];
+                mask[w] = st->tie_mask[w];
+            }
+            put_digit<W>(key, d, static_cast<uint64_t>(kPer * static_cast<int>(threadIdx.x) + q));
+            put_digit<W>(mask, d, kHistBins - 1);
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                st->tie_key[w] = key[w];
+                st->tie_mask[w] = mask[w];
+            }
+            st->cand_needed = static_cast<int64_t>(need - cum);
+            // past the last digit the entries left are one config's: any of them will do
+            st->ties = v[q] > static_cast<unsigned long long>(p.cand_cap) && d + 1 < levels ? 1 : 0;
+            st->tie_blocks = 0u;
+        }
+        cum += v[q];
+    }
 }
 
 // Sort keys of the rows: the high word of |psi|'s bits.
@@ -519,6 +698,7 @@ __global__ __launch_bounds__(1024) void fr_select_kernel(FrState* st, unsigned l
             st->done = 1;
             st->cand_needed = st->k_rem;
             st->hi = (st->prefix + 1ull) << shift;
+            st->ties = s_in > static_cast<unsigned long long>(cand_cap) ? 1 : 0;
         } else {
             st->level = level + 1;
         }
@@ -626,8 +806,10 @@ __global__ void fr_scatter_kernel(const uint32_t* __restrict__ perm, int64_t n, 
     }
 }
 
+constexpr unsigned kTieGrid = 1024;  // four work-groups a CU: a launch that finds no ties costs 2 us
+
 // Entries tied on the digits so far are collected as candidates up to this many, and narrowed by another
-// digit's pass above it: the candidates are sorted twice in full (1M of them: 1.7 ms), a pass over what
+// digit's pass above it (of the weight, then of the config): the candidates are sorted twice in full (1M of them: 1.7 ms), a pass over what
 // is left of the connections costs less.
 int64_t cand_capacity(int64_t k) {
     const int64_t cap = 2 * k;
@@ -775,6 +957,8 @@ int find_relative_impl(const qmb_terms* terms, const qmb_targets* exclude, const
                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
         QMB_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&fr_collect_kernel<W>),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+        QMB_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&fr_tie_kernel<W>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
         const auto* psi = reinterpret_cast<const double2*>(psi_i);
         const auto* coefs = reinterpret_cast<const double2*>(terms->coefs);
         fr_row_keys_kernel<<<blocks_for(n_i), 256, 0, stream>>>(psi, n_i, s.row_key_a, s.row_a);
@@ -806,6 +990,13 @@ int find_relative_impl(const qmb_terms* terms, const qmb_targets* exclude, const
             QMB_CHECK_LAUNCH();
             fr_select_kernel<<<1, 1024, 0, stream>>>(s.state, s.hist, s.psi, n_i, s.exps, cap);
             QMB_CHECK_LAUNCH();
+        }
+        if (n_i > cap / T) {  // else no class can exceed the buffer
+            const int digits = tie_levels(terms->n_qubytes);
+            for (int d = 0; d < digits; ++d) {
+                fr_tie_kernel<W><<<grid < kTieGrid ? grid : kTieGrid, kEnumBlock, lds, stream>>>(p, d, digits);
+                QMB_CHECK_LAUNCH();
+            }
         }
         fr_collect_kernel<W><<<grid, kEnumBlock, lds, stream>>>(p);
         QMB_CHECK_LAUNCH();

@@ -149,6 +149,38 @@ def test_find_relative_selects_what_the_host_operator_does(cuda_device: torch.de
     assert torch.equal(got, want), (name, kind, k_sel, got.shape, want.shape)
 
 
+@pytest.mark.parametrize("k_sel", [1, 100, 40_000])
+@pytest.mark.parametrize("name,rows", [("hubbard-32", 3000), ("hubbard-32", 45_000), ("hubbard-70", 2000), ("hubbard-100", 1500),
+                                       ("molecular-20", 3000), ("molecular-40", 1000)])
+def test_find_relative_takes_exact_ties_by_config(cuda_device: torch.device, name: str, rows: int, k_sel: int) -> None:
+    """More entries of exactly one weight than any buffer holds (one coefficient size, |psi| = 1 with any
+    sign): those with the lowest configs are taken, so the rows equal the host operator's and a second
+    call's.  One to four words a config, both enumerations, 10^5 to several 10^6 tied entries."""
+    rng = np.random.default_rng(rows)
+    if name.startswith("hubbard"):
+        sites = int(name[8:])
+        s, k, c = (x.numpy() for x in sy.terms_from_dict(sy.hubbard_dict(sites, 1, 1.0, 4.0)))
+        if sites == 32:
+            cfg = sy.hubbard_chain_configs(sites, rows, 78, n_seed_configs=rows // 30)
+        else:
+            bits = np.zeros((rows, (2 * sites + 7) // 8 * 8), dtype=np.uint8)
+            bits[:, : 2 * sites] = rng.random((rows, 2 * sites)) < 0.5
+            cfg = sy.sort_unique_configs(np.packbits(bits, axis=1, bitorder="little"))
+    else:
+        orbitals = int(name[10:]) // 2
+        s, k, c = sorted_terms(*sy.molecular_terms(orbitals, 79))
+        c = np.stack([np.where(c[:, 0] < 0, -1.0, 1.0), np.zeros(len(c))], axis=1)
+        cfg = sy.sector_configs(10, 5, 5, rows, 80) if orbitals == 10 else sy.excitation_configs(orbitals, 6, 6, rows, 80)
+    psi = np.where(rng.random(len(cfg)) < 0.5, -1.0, 1.0) + 0j
+    ns = ops.load(cfg.shape[1], 1)
+    host = [torch.from_numpy(np.ascontiguousarray(x)) for x in (cfg, psi.view(np.float64).reshape(-1, 2), s, k, c)]
+    want = ns.find_relative(host[0], host[1], k_sel, host[2], host[3], host[4], host[0])
+    dev = [t.to(cuda_device) for t in host]
+    for _ in range(2):
+        got = ns.find_relative(dev[0], dev[1], k_sel, dev[2], dev[3], dev[4], dev[0]).cpu()
+        assert torch.equal(got, want), (got.shape, want.shape)
+
+
 DIAG_CASES = [
     ("molecular-20so", 1, lambda: sorted_terms(*sy.molecular_terms(10, 1001)), lambda: sy.sector_configs(10, 5, 5, 2000, 21)),
     ("random-ops", 1, lambda: tuple(x.numpy() for x in sy.random_terms(12, 500, 22)),
