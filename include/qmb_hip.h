@@ -427,10 +427,11 @@ int qmb_apply_structured_dual(const qmb_pairs* pairs, const qmb_singles* singles
 
 /* ---------------- batched persistent launch (no reference counterpart) -------------------------
  * Many instances -- a term table and a config set each, of any sizes -- applied by two persistent
- * kernel launches for all of them: the diagonal, single- and pair-excitation work of every instance
- * is cut into units of a few passes over core groups of one size, or 64 rows; the first launch's waves take the pair units of
- * all instances round-robin, the second's the single and diagonal units.  For many small instances
- * this replaces a few kernels per instance by two launches that fill the GPU; both are capturable
+ * kernel launches for all of them (after a one-block launch that numbers the work where there is much of
+ * it): the diagonal, single- and pair-excitation work of every instance is cut into units of a few passes
+ * over core groups of one size, or 64 rows; the first launch's waves take the pair units of all instances
+ * round-robin, the second's the single and diagonal units.  For many small instances
+ * this replaces a few kernels per instance by two launches that fill the GPU; all are capturable
  * in a hipGraph (no allocation, no sync).
  * An instance whose table has terms outside those classes (its residual table) needs that part
  * applied separately. */
@@ -450,19 +451,23 @@ typedef struct qmb_batch_item {
 typedef struct qmb_batch {
     int32_t n_items;
     int32_t dual;      /* 1: every item has in2/out2 */
-    int64_t total_units;
+    int64_t total_units;  /* at most; the indexes decide at each application */
     void* buffer;
     size_t bytes;
     void* items;       /* device table of the items */
-    int64_t* offsets;  /* device [3 * n_items + 1]: first unit of (type, item) */
+    int64_t* offsets;  /* device [3 * n_items + 1]: first unit of (type, item), written by each application of
+                          a large batch */
 } qmb_batch;
 
 int qmb_batch_workspace_size(int n_items, size_t* bytes);
-/* Copies the item table to the device; synchronises `stream` once (set-up, not per launch). */
+/* Copies the item table to the device; synchronises `stream` once (set-up, not per launch).  Nothing the
+ * tables and indexes hold is read: a plan may be made before they are finished, and stays valid when
+ * one is built again in the same workspace over as many rows with the same max_occupied (an application
+ * must be ordered after the builds, as any use of them). */
 int qmb_batch_plan(const qmb_batch_item* items, int n_items, void* buffer, size_t bytes, qmb_batch* out, void* stream);
-/* Two persistent launches of `waves` wavefronts each (0: 8192) over all units (the pair units, then
- * the single and diagonal units); mode 0 forward, 1 adjoint
- * (a Hermitian instance gives the same map in both).  A two-vector batch (dual) computes
+/* Two persistent launches of `waves` wavefronts each (0: 8192) over all units (the pair units, then the
+ * single and diagonal units), behind a one-block launch that numbers the units of a large batch; mode 0
+ * forward, 1 adjoint (a Hermitian instance gives the same map in both).  A two-vector batch (dual) computes
  * out = A in and out2 = A in2 (mode 0; A^H with mode 1) in the same pass, sharing every group walk
  * and coefficient read: for Hermitian instances that is the forward and the backward of a
  * training step in one pass. */

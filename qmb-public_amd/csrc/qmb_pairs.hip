@@ -48,20 +48,19 @@ inline unsigned blocks_for(int64_t n, int block = kBlock) {
     return static_cast<unsigned>(b < 1 ? 1 : b);
 }
 
-// Index of the calling wave among the grid's persistent waves, ordered so that each XCD holds a
-// contiguous eighth of [0, waves).  Workgroups go to the 8 XCDs round-robin by blockIdx.x, so with
+// Index of the calling wave among the persistent waves of the grid's first `blocks` blocks, ordered so that
+// each XCD holds a contiguous eighth of [0, waves).  Workgroups go to the 8 XCDs round-robin by blockIdx.x, so with
 // a grid that divides evenly, waves walking units w, w + waves, ... keep each XCD's L2 on the
 // coefficient rows of an eighth of every window of units instead of rows from the whole window.
 // Measured: the batch kernel gains (138.9 -> 134 ms on 64 molecular instances); the single-set
 // pair and single kernels lose (8.07 -> 8.46 ms at 1M configs), so they keep the plain order.
-__device__ __forceinline__ int64_t xcd_wave() {
+__device__ __forceinline__ int64_t xcd_wave(uint32_t blocks, int64_t in_block) {
     constexpr int kXcds = 8;
     constexpr int64_t kWavesPerBlock = kBlock / 64;
-    const int64_t in_block = threadIdx.x >> 6;
-    if (gridDim.x % kXcds != 0) {
+    if (blocks % kXcds != 0) {
         return static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + in_block;
     }
-    const int64_t waves = static_cast<int64_t>(gridDim.x) * kWavesPerBlock;
+    const int64_t waves = static_cast<int64_t>(blocks) * kWavesPerBlock;
     return static_cast<int64_t>(blockIdx.x % kXcds) * (waves / kXcds) + static_cast<int64_t>(blockIdx.x / kXcds) * kWavesPerBlock +
            in_block;
 }
@@ -2173,7 +2172,7 @@ __device__ __forceinline__ void single_rows(const SingleParams& p, int g, uint32
 
 // Rows [first, last) of one group of any size from mvals[s], lane = row.
 template <int W, bool ADJ, int NV, int CH>
-__device__ void single_group(const SingleParams& p, uint32_t s, uint32_t size, uint32_t first, uint32_t last, int lane, Stage<NV>& st) {
+__device__ __forceinline__ void single_group(const SingleParams& p, uint32_t s, uint32_t size, uint32_t first, uint32_t last, int lane, Stage<NV>& st) {
     const bool fermi = p.particle_cut == 1;
     const Entry head = binned_entry(p.mvals[s], fermi);
     Cfg<W> core = load_key<W>(p.ckeys, static_cast<int64_t>(head.row));
@@ -2741,10 +2740,13 @@ __global__ __launch_bounds__(kBlock) void diag_apply2_kernel(const uint64_t* __r
 }
 
 // --------------------------------------------------------------------- batched persistent launch --
-// Many instances (term tables + config sets) in one launch: the work of every instance is cut into
-// units -- 64 pair-core groups, 64 single-core groups, 64 diagonal rows -- numbered type-major
+// Many instances (term tables + config sets) in one pass: the work of every instance is cut into
+// units -- those of its core indexes' bins, and 64 diagonal rows -- numbered type-major
 // (all pair units, then singles, then diagonal, so the heaviest work is taken first), and
-// persistent waves take units round-robin until all are done.
+// persistent waves take units round-robin until all are done.  How many units an index makes up is
+// known when it is built, on the device, so each application numbers them: a plan, or a graph of
+// the launches, stays good when an index is built again in its place.  (Numbered by what the capacities
+// allow, the gaps left the waves unevenly loaded: 64 sets of 1000 rows 51 -> 134 us.)
 struct BatchItemDev {
     int32_t n_words, particle_cut, has_pairs, has_singles;
     int32_t n_bits, reserved;
@@ -2775,7 +2777,7 @@ struct BatchItemDev {
 constexpr int kBatchMaxItems = 4096;
 
 template <int W, bool ADJ, int NV>
-__device__ void diag_rows(const BatchItemDev& it, int64_t r0, int lane) {
+__device__ __forceinline__ void diag_rows(const BatchItemDev& it, int64_t r0, int lane) {
     const int64_t i = r0 + lane;
     if (i >= it.n) {
         return;
@@ -2797,7 +2799,7 @@ __device__ void diag_rows(const BatchItemDev& it, int64_t r0, int lane) {
 // PART 1: the pair units (type 0); PART 2: the single-excitation (type 1) and diagonal (type 2)
 // units.
 template <int W, bool ADJ, int NV, int PART>
-__device__ void batch_unit(const BatchItemDev& it, int type, int64_t local, int lane, Stage<NV>& stage) {
+__device__ __forceinline__ void batch_unit(const BatchItemDev& it, int type, int64_t local, int lane, Stage<NV>& stage) {
     if (PART == 1 && type == 0) {
         PairParams p{};
         p.coef = it.pcoef;
@@ -2851,40 +2853,154 @@ __device__ void batch_unit(const BatchItemDev& it, int type, int64_t local, int 
     }
 }
 
+// For batches whose waves do not number the units themselves: offsets[type * n_items + item] = first unit of the instance's units of the type, then their number.
+// One block; applications of one plan write the same.
+constexpr int kOffsetThreads = 1024;
+__global__ __launch_bounds__(kOffsetThreads) void batch_offsets_kernel(const BatchItemDev* __restrict__ items, int n_items,
+                                                                       int64_t* __restrict__ offsets) {
+    __shared__ int64_t s_wave[kOffsetThreads / 64];
+    constexpr int kSlots = 3 * kBatchMaxItems / kOffsetThreads;  // of a thread
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int slots = 3 * n_items;
+    const int per = (slots + kOffsetThreads - 1) / kOffsetThreads;
+    int64_t units[kSlots], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kSlots; ++k) {
+        const int slot = per * static_cast<int>(threadIdx.x) + k;
+        units[k] = 0;
+        if (k < per && slot < slots) {
+            const int type = slot / n_items;
+            const BatchItemDev& it = items[slot - type * n_items];
+            const CoreBins* bins = type == 0 ? it.pbins : it.sbins;
+            units[k] = type == 2 ? (it.n + 63) / 64 : (bins != nullptr ? bins->unit_start[kBins] : 0u);
+        }
+        sum += units[k];
+    }
+    int64_t incl = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int64_t o = __shfl_up(incl, d);
+        incl += lane >= d ? o : 0;
+    }
+    if (lane == 63) {
+        s_wave[wave] = incl;
+    }
+    __syncthreads();
+    int64_t run = incl - sum;
+    for (int w = 0; w < wave; ++w) {
+        run += s_wave[w];
+    }
+#pragma unroll
+    for (int k = 0; k < kSlots; ++k) {
+        const int slot = per * static_cast<int>(threadIdx.x) + k;
+        if (k < per && slot < slots) {
+            offsets[slot] = run;
+            run += units[k];
+            if (slot == slots - 1) {
+                offsets[slots] = run;
+            }
+        }
+    }
+}
+
 // One batch application is two persistent launches over the units, the pair units (PART 1), then the
 // single and diagonal units (PART 2): each kernel holds only its own unit code, so both keep the
 // packed groups within 128 VGPRs (4 waves per SIMD; 3 waves measured ~20% slower).  As one launch
 // over all unit types the kernel spilled at that limit and had to walk the 9..32-entry groups one
 // per wave (64 molecular instances, forward + backward: 115.0 ms against 108.2 ms split).
-template <bool ADJ, int NV, int PART>
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v, int lane) {
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = __shfl_up(v, d);
+        v += lane >= d ? o : 0u;
+    }
+    return v;
+}
+
+// OWN: every wave numbers the units itself, a lane an instance, and finds a unit's by a ballot, which
+// saves the launch of batch_offsets_kernel (3 us; a batch of 200 rows takes 17) but costs the pair units
+// of a large batch 2.7% (12 instances, 250,000 rows): for up to kOwnItems instances and kOwnUnits units,
+// a pass of some 30 us (16 x 500 rows 18.8 us, 22 with the launch; 64 x 1000 rows 56, 54 with it).
+constexpr int kOwnItems = 64;
+constexpr int64_t kOwnUnits = 1 << 15;
+
+template <bool ADJ, int NV, int PART, bool OWN>
 __global__ __launch_bounds__(kBlock, 4) void batch_kernel(const BatchItemDev* __restrict__ items, const int64_t* __restrict__ offsets,
-                                                       int n_items, int64_t total) {
-    const int lane = threadIdx.x & 63;
-    const int64_t wave = xcd_wave();
-    const int64_t nwaves = (static_cast<int64_t>(gridDim.x) * kBlock) >> 6;
+                                                       int n_items) {
     __shared__ Stage<NV> stages[kWavesPerBlock];
+    const int id = threadIdx.x & 63;
     Stage<NV>& stage = stages[threadIdx.x >> 6];
-    const int slots = 3 * n_items;
-    const int64_t first = PART == 2 ? offsets[n_items] : 0;
-    const int64_t last = PART == 1 ? offsets[n_items] : total;
-    for (int64_t u = first + wave; u < last; u += nwaves) {
-        // last slot whose first unit is <= u (offsets[slots] == total > u)
-        int lo = 0, hi = slots;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (offsets[mid] <= u) {
-                lo = mid;
+    // the part's units: pair units (PART 1), or `split` single units and then diagonal ones (PART 2)
+    uint32_t first_a = 0, first_b = 0, split = 0;
+    int64_t first = 0, total;
+    if constexpr (OWN) {
+        const bool in = id < n_items;
+        const BatchItemDev& it = items[in ? id : 0];
+        const CoreBins* bins = PART == 1 ? it.pbins : it.sbins;
+        const uint32_t a = in && bins != nullptr ? bins->unit_start[kBins] : 0u;
+        const uint32_t sum_a = wave_scan(a, id);
+        first_a = sum_a - a;
+        split = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(sum_a), 63));
+        total = split;
+        if (PART == 2) {
+            const uint32_t b = in ? static_cast<uint32_t>((it.n + 63) / 64) : 0u;
+            const uint32_t sum_b = wave_scan(b, id);
+            first_b = sum_b - b;
+            total += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(sum_b), 63));
+        }
+    } else {
+        first = PART == 2 ? offsets[n_items] : 0;
+        total = offsets[PART == 1 ? n_items : 3 * n_items] - first;
+    }
+    // as many blocks as there are units for: each XCD then gets an eighth of them
+    const uint32_t blocks = total >= static_cast<int64_t>(gridDim.x) * kWavesPerBlock
+                                ? gridDim.x
+                                : static_cast<uint32_t>((total + kWavesPerBlock - 1) / kWavesPerBlock);
+    if (blockIdx.x >= blocks) {
+        return;
+    }
+    const int64_t nwaves = static_cast<int64_t>(blocks) * kWavesPerBlock;
+    if constexpr (OWN) {
+        for (int64_t u = xcd_wave(blocks, __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6))); u < total; u += nwaves) {
+            const bool diagonal = PART == 2 && u >= split;
+            // the last instance whose first unit is <= v
+            const uint32_t v = static_cast<uint32_t>(u) - (diagonal ? split : 0u);
+            const uint32_t from = diagonal ? first_b : first_a;
+            const int item = 63 - __builtin_clzll(__ballot(from <= v && id < n_items));
+            const int64_t local = v - static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(from), item));
+            // made anew for each unit: what every group size derives from the lane would otherwise be computed
+            // ahead of the loop (it holds 128 registers and spills)
+            int lane = id;
+            asm volatile("" : "+v"(lane));
+            const int type = PART == 1 ? 0 : (diagonal ? 2 : 1);
+            const BatchItemDev& it = items[item];
+            if (PART == 1 || it.n_words == 1) {  // the pair units take any width
+                batch_unit<1, ADJ, NV, PART>(it, type, local, lane, stage);
             } else {
-                hi = mid;
+                batch_unit<2, ADJ, NV, PART>(it, type, local, lane, stage);
             }
         }
-        const int type = lo / n_items;
-        const BatchItemDev& it = items[lo - type * n_items];
-        const int64_t local = u - offsets[lo];
-        if (PART == 1 || it.n_words == 1) {  // the pair units take any width
-            batch_unit<1, ADJ, NV, PART>(it, type, local, lane, stage);
-        } else {
-            batch_unit<2, ADJ, NV, PART>(it, type, local, lane, stage);
+    } else {
+        const int slots = 3 * n_items;
+        const int64_t last = first + total;
+        for (int64_t u = first + xcd_wave(blocks, threadIdx.x >> 6); u < last; u += nwaves) {
+            // last slot whose first unit is <= u (offsets[slots] > u)
+            int lo = 0, hi = slots;
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (offsets[mid] <= u) {
+                    lo = mid;
+                } else {
+                    hi = mid;
+                }
+            }
+            const int type = lo / n_items;
+            const BatchItemDev& it = items[lo - type * n_items];
+            const int64_t local = u - offsets[lo];
+            if (PART == 1 || it.n_words == 1) {
+                batch_unit<1, ADJ, NV, PART>(it, type, local, id, stage);
+            } else {
+                batch_unit<2, ADJ, NV, PART>(it, type, local, id, stage);
+            }
         }
     }
 }
@@ -3607,6 +3723,10 @@ int batch_layout(Carver& cv, int n_items, qmb_batch* out) {
     return QMB_OK;
 }
 
+// Units that the bins of an index of this capacity can make up: none but a bin's last covers fewer than 32
+// entries (a group of 65 entries is two; a unit of the split bin is 16 slots of two entries).
+inline int64_t unit_bound(int64_t capacity) { return capacity > 0 ? capacity / 32 + kBins : 0; }
+
 size_t batch_bytes(int n_items) {
     Carver cv{nullptr, 0};
     return batch_layout(cv, n_items, nullptr) == QMB_OK ? cv.off : 0;
@@ -3622,8 +3742,6 @@ int batch_plan(const qmb_batch_item* items, int n_items, void* buffer, size_t by
     b.bytes = bytes;
     std::vector<BatchItemDev> dev(static_cast<size_t>(n_items));
     int dual = 0;
-    std::vector<int64_t> units(3 * static_cast<size_t>(n_items), 0);
-    std::vector<uint32_t> device_units(2 * static_cast<size_t>(n_items), 0u);  // units of the core indexes' bins
     for (int k = 0; k < n_items; ++k) {
         const qmb_batch_item& x = items[k];
         if (!x.pairs || !x.targets) {
@@ -3654,8 +3772,9 @@ int batch_plan(const qmb_batch_item* items, int n_items, void* buffer, size_t by
             d.n_pairs = x.pairs->n_pairs;
             d.pmvals = x.cores2->mvals;
             d.pglist = reinterpret_cast<const uint2*>(x.cores2->glist);
-            d.pbins = static_cast<const CoreBins*>(x.cores2->bins);
+            d.pbins = x.cores2->capacity > 0 ? static_cast<const CoreBins*>(x.cores2->bins) : nullptr;
             d.pcounts = x.cores2->counts;
+            b.total_units += unit_bound(x.cores2->capacity);
         }
         if (x.singles) {
             d.has_singles = 1;
@@ -3665,10 +3784,11 @@ int batch_plan(const qmb_batch_item* items, int n_items, void* buffer, size_t by
             d.skd_re = x.singles->real ? x.singles->kd_re : nullptr;
             d.smvals = x.cores1->mvals;
             d.sglist = reinterpret_cast<const uint2*>(x.cores1->glist);
-            d.sbins = static_cast<const CoreBins*>(x.cores1->bins);
+            d.sbins = x.cores1->capacity > 0 ? static_cast<const CoreBins*>(x.cores1->bins) : nullptr;
             d.scounts = x.cores1->counts;
+            b.total_units += unit_bound(x.cores1->capacity);
         }
-        units[2 * n_items + k] = (tg.n + 63) / 64;
+        b.total_units += (tg.n + 63) / 64;
         d.in = reinterpret_cast<const double2*>(x.in);
         d.out = reinterpret_cast<double2*>(x.out);
         d.in2 = reinterpret_cast<const double2*>(x.in2);
@@ -3680,28 +3800,9 @@ int batch_plan(const qmb_batch_item* items, int n_items, void* buffer, size_t by
         dual = two;
         dev[static_cast<size_t>(k)] = d;
     }
-    for (int k = 0; k < n_items; ++k) {
-        const BatchItemDev& d = dev[static_cast<size_t>(k)];
-        if (items[k].cores2->capacity > 0) {
-            QMB_HIP_TRY(hipMemcpyAsync(&device_units[k], &d.pbins->unit_start[kBins], sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-        }
-        if (items[k].singles && items[k].cores1->capacity > 0) {
-            QMB_HIP_TRY(hipMemcpyAsync(&device_units[n_items + k], &d.sbins->unit_start[kBins], sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-        }
-    }
-    QMB_HIP_TRY(hipStreamSynchronize(stream));
-    for (size_t q = 0; q < device_units.size(); ++q) {
-        units[q] = static_cast<int64_t>(device_units[q]);
-    }
-    std::vector<int64_t> offsets(units.size() + 1, 0);
-    for (size_t q = 0; q < units.size(); ++q) {
-        offsets[q + 1] = offsets[q] + units[q];
-    }
-    b.total_units = offsets.back();
     b.dual = dual;
     QMB_HIP_TRY(hipMemcpyAsync(b.items, dev.data(), dev.size() * sizeof(BatchItemDev), hipMemcpyHostToDevice, stream));
-    QMB_HIP_TRY(hipMemcpyAsync(b.offsets, offsets.data(), offsets.size() * sizeof(int64_t), hipMemcpyHostToDevice, stream));
-    // the host tables above go out of scope on return
+    // the host table above goes out of scope on return
     QMB_HIP_TRY(hipStreamSynchronize(stream));
     *out = b;
     return QMB_OK;
@@ -3724,23 +3825,28 @@ int apply_batch(const qmb_batch* batch, int mode, int waves, hipStream_t stream)
     blocks = blocks < need ? blocks : need;
     const auto* items = static_cast<const BatchItemDev*>(batch->items);
     const unsigned g = static_cast<unsigned>(blocks);
-    if (batch->dual) {
-        if (mode == 1) {
-            batch_kernel<true, 2, 1><<<g, kBlock, 0, stream>>>(items, batch->offsets, batch->n_items, batch->total_units);
-            batch_kernel<true, 2, 2><<<g, kBlock, 0, stream>>>(items, batch->offsets, batch->n_items, batch->total_units);
-        } else {
-            batch_kernel<false, 2, 1><<<g, kBlock, 0, stream>>>(items, batch->offsets, batch->n_items, batch->total_units);
-            batch_kernel<false, 2, 2><<<g, kBlock, 0, stream>>>(items, batch->offsets, batch->n_items, batch->total_units);
-        }
-    } else if (mode == 1) {
-        batch_kernel<true, 1, 1><<<g, kBlock, 0, stream>>>(items, batch->offsets, batch->n_items, batch->total_units);
-        batch_kernel<true, 1, 2><<<g, kBlock, 0, stream>>>(items, batch->offsets, batch->n_items, batch->total_units);
-    } else {
-        batch_kernel<false, 1, 1><<<g, kBlock, 0, stream>>>(items, batch->offsets, batch->n_items, batch->total_units);
-        batch_kernel<false, 1, 2><<<g, kBlock, 0, stream>>>(items, batch->offsets, batch->n_items, batch->total_units);
+    const bool own = batch->n_items <= kOwnItems && batch->total_units <= kOwnUnits;
+    if (!own) {
+        batch_offsets_kernel<<<1, kOffsetThreads, 0, stream>>>(items, batch->n_items, batch->offsets);
+        QMB_CHECK_LAUNCH();
     }
-    QMB_CHECK_LAUNCH();
-    return QMB_OK;
+    const auto both = [&](auto pair_units, auto other_units) -> int {
+        pair_units<<<g, kBlock, 0, stream>>>(items, batch->offsets, batch->n_items);
+        QMB_CHECK_LAUNCH();
+        other_units<<<g, kBlock, 0, stream>>>(items, batch->offsets, batch->n_items);
+        QMB_CHECK_LAUNCH();
+        return QMB_OK;
+    };
+    const auto go = [&](auto wave_numbers) -> int {
+        constexpr bool O = decltype(wave_numbers)::value;
+        if (batch->dual) {
+            return mode == 1 ? both(&batch_kernel<true, 2, 1, O>, &batch_kernel<true, 2, 2, O>)
+                             : both(&batch_kernel<false, 2, 1, O>, &batch_kernel<false, 2, 2, O>);
+        }
+        return mode == 1 ? both(&batch_kernel<true, 1, 1, O>, &batch_kernel<true, 1, 2, O>)
+                         : both(&batch_kernel<false, 1, 1, O>, &batch_kernel<false, 1, 2, O>);
+    };
+    return own ? go(std::true_type{}) : go(std::false_type{});
 }
 
 }  // namespace qmb

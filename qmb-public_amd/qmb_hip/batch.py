@@ -5,7 +5,7 @@ Each instance is a PreparedTerms (with the structured tables: pair and single ex
 diagonal records) and a PreparedTargets over its distinct config set.  The inputs and outputs of all
 instances are packed into two device buffers, so the plan (qmb_batch_plan) is built once and every
 launch (qmb_apply_batch) is two persistent kernels over all instances' work (the pair units, then the
-single and diagonal units); the whole step
+single and diagonal units), behind a one-block kernel that numbers the units of a large batch; the whole step
 can be captured in a hipGraph (torch.cuda.CUDAGraph) and replayed.  Instances whose tables keep
 terms outside the structured classes get those applied by one enumeration launch each after the
 batch.

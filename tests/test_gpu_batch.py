@@ -11,10 +11,13 @@ qmb_hip.batch.Batch):
     replays, reproduces the eager result on every replay;
   - a two-vector batch applies every instance to two vectors in one launch (forward and backward of
     a training step for Hermitian instances), equal to the per-instance results, graph replays too;
-  - the autotuner picks a wave count among its candidates without changing the result.
+  - the autotuner picks a wave count among its candidates without changing the result;
+  - a plan stays valid when the indexes it was made over are built again in their place.
 """
 
 from __future__ import annotations
+
+import ctypes
 
 import numpy as np
 import pytest
@@ -22,9 +25,11 @@ import torch
 
 from conftest import sorted_terms
 from oracle import oracle as orc
+from qmb_hip import _lib
 from qmb_hip import batch as qb
 from qmb_hip import prepared as pp
 from qmb_hip import synthetic as sy
+from qmb_hip.ops import _ptr, _stream
 
 pytestmark = pytest.mark.gpu
 
@@ -203,6 +208,58 @@ def test_batch_graph_replays_match_eager(cuda_device: torch.device) -> None:
         diff = (b.out - eager).abs().max().item()
         scale = eager.abs().max().item()
         assert diff <= 1e-12 * scale, (replay, diff)
+
+
+@pytest.mark.parametrize("two", [False, True], ids=["one-vector", "two-vector"])
+@pytest.mark.parametrize("count,instances_of", [(150, 2), (3000, 2), (150, 66)])
+def test_plan_outlives_a_rebuild_in_place(cuda_device: torch.device, count: int, instances_of: int, two: bool) -> None:
+    """A plan and a graph of its launch made over sets of scattered rows (hardly a group of two), then the
+    indexes built again in the same workspaces over rows with far more connections, and back: every
+    application is that of the rows the indexes hold.  150 rows: the one-block build; 3000: the general one;
+    66 instances: more than a wave numbers itself."""
+    n_orb, sets = 14, {}
+    s, k, c = sorted_terms(*sy.molecular_terms(n_orb, 91))
+    terms = pp.PreparedTerms(_dev(s, cuda_device), _dev(k, cuda_device), _dev(c, cuda_device), 4, 1)
+    for seed in range(92, 92 + instances_of):
+        sets[seed] = {"scattered": _dev(sy.sector_configs(n_orb, 5, 5, count, seed), cuda_device),
+                      "connected": _dev(sy.excitation_configs(n_orb, 5, 5, count, seed), cuda_device)}
+    instances = [(terms, pp.PreparedTargets(x["scattered"].clone(), 4, distinct=True)) for x in sets.values()]
+    b = qb.Batch(instances, two_vectors=two)
+    psis = [torch.from_numpy(sy.random_psi(count, 900 + j)).to(cuda_device) for j in range(2 * instances_of)]
+    b.set_inputs(psis[:instances_of], psis[instances_of:] if two else None)
+
+    def launch() -> None:
+        if two:
+            b.launch_both()
+        else:
+            b.launch(pp.MODE_FORWARD)
+
+    launch()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        launch()
+    lib = _lib.library()
+    for which in ("connected", "scattered", "connected"):
+        for x, (_, t) in zip(sets.values(), instances):
+            t.configs.copy_(x[which])
+            stream = _stream(cuda_device)
+            desc = _lib.QmbTargets()
+            _lib.check(lib.qmb_targets_build_keys(4, _ptr(t.configs), count, _ptr(t.buffer), t.buffer.numel(), ctypes.byref(desc), stream), "keys")
+            assert desc.keys == t.keys_desc.keys
+            for order in (2, 1):
+                buf, old = t._cores[order]  # pylint: disable=protected-access
+                cores = _lib.QmbCores()
+                _lib.check(lib.qmb_cores_build(ctypes.byref(desc), 10, order, _ptr(buf), buf.numel(), ctypes.byref(cores), stream), "cores")
+                assert (cores.mvals, cores.glist, cores.bins) == (old.mvals, old.glist, old.bins)
+        for run in (launch, graph.replay):
+            b.out.fill_(float("nan"))
+            run()
+            for j, x in enumerate(sets.values()):
+                fresh = pp.PreparedTargets(x[which], 4, distinct=True)
+                for second, vec in ((False, psis[j]), (True, psis[instances_of + j])) if two else ((False, psis[j]),):
+                    ref = _reference(terms, fresh, vec, pp.MODE_FORWARD)
+                    got = b.output(j, second).cpu().numpy()
+                    np.testing.assert_array_less(np.abs(got - ref), 1e-12 * _scale(ref, 10.0, vec) + 1e-300)
 
 
 def test_batch_autotune_keeps_result(cuda_device: torch.device) -> None:
