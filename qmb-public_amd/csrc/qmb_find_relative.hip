@@ -82,8 +82,9 @@ __device__ __forceinline__ double reach_of(uint64_t lo) {
 }
 
 // Rows and terms are ordered by the high word of the bits of |psi| and |coef| (20 bits of mantissa), so
-// a later one is at most this factor above an earlier one.  NaN orders first and drops nothing.
-constexpr double kOrderSlack = 1.0 + 2e-6;
+// a later one is at most a factor 1 + 2^-20 above an earlier one or, both denormal, 2^-1042 more: what
+// any from there on can have.  NaN orders first and drops nothing.
+__device__ __forceinline__ double at_most_from(double a) { return a * (1.0 + 2e-6) + 0x1p-1042; }
 
 __device__ __forceinline__ bool below_reach(double a, double b, double reach) { return a * b < reach; }
 
@@ -97,7 +98,7 @@ struct FrParams {
     const uint64_t* xfilter;
     uint64_t xfmask;
     const uint64_t* xcols;
-    const double* aw;  // |coef| per term, descending within each bucket (times kOrderSlack)
+    const double* aw;  // per term, |coef| at most from there on in its bucket (at_most_from)
     FrState* state;
     unsigned long long* hist;
     uint64_t* sel_c;   // [K][W] selected configs ("above" entries, then the kept candidates)
@@ -182,7 +183,7 @@ struct PrunedHooks : ActionHooks {
     const FrParams& p;
     double reach;
     __device__ explicit PrunedHooks(const FrParams& pp) : p(pp), reach(pp.state->reach) {}
-    __device__ __forceinline__ double tile_bound(int64_t i0) const { return hypot(p.psi[i0].x, p.psi[i0].y) * kOrderSlack; }
+    __device__ __forceinline__ double tile_bound(int64_t i0) const { return at_most_from(hypot(p.psi[i0].x, p.psi[i0].y)); }
     __device__ __forceinline__ bool drop(uint32_t t, double bound) const { return below_reach(p.aw[t], bound, reach); }
 };
 
@@ -461,7 +462,7 @@ __global__ void fr_term_gather_kernel(const uint32_t* __restrict__ order, const 
         const double2 c = coefs[o];
         out_recs[t] = recs[o];
         out_coefs[t] = c;
-        aw[t] = hypot(c.x, c.y) * kOrderSlack;
+        aw[t] = at_most_from(hypot(c.x, c.y));
     }
 }
 
@@ -519,7 +520,7 @@ __device__ int64_t fr_active(const double2* __restrict__ psi, int64_t n, double 
     int64_t lo = 0, hi = n;
     while (lo < hi) {
         const int64_t mid = (lo + hi) >> 1;
-        if (below_reach(amax, hypot(psi[mid].x, psi[mid].y) * kOrderSlack, reach)) {
+        if (below_reach(amax, at_most_from(hypot(psi[mid].x, psi[mid].y)), reach)) {
             hi = mid;
         } else {
             lo = mid + 1;
@@ -535,7 +536,7 @@ __device__ void fr_set_lo(FrState* st, uint64_t lo, const double2* __restrict__ 
 }
 
 __device__ __forceinline__ double fr_amax(const FrExponents* exps) {
-    return __longlong_as_double(static_cast<long long>(exps[1].most)) * kOrderSlack;
+    return at_most_from(__longlong_as_double(static_cast<long long>(exps[1].most)));
 }
 
 // The bounds of the first digit's pass: the products |psi| |coef| whose exponents sum to e or more number

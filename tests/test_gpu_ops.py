@@ -181,6 +181,35 @@ def test_find_relative_takes_exact_ties_by_config(cuda_device: torch.device, nam
         assert torch.equal(got, want), (got.shape, want.shape)
 
 
+@pytest.mark.parametrize("of", ["rows", "terms"])
+@pytest.mark.parametrize("name", ["molecular", "hubbard"])
+def test_find_relative_with_denormal_factors(cuda_device: torch.device, name: str, of: str) -> None:
+    """Rows (or coefficients) too small for the order the passes are cut by to tell them apart, zeros before
+    and between them, whose weights the other factor lifts to ordinary numbers: none may be cut off."""
+    rng = np.random.default_rng(81)
+    if name == "molecular":
+        s, k, c = sorted_terms(*sy.molecular_terms(8, 82))
+        cfg = sy.sector_configs(8, 3, 3, 500, 83)
+    else:
+        s, k, c = (x.numpy() for x in sy.terms_from_dict(sy.hubbard_dict(32, 1, 1.0, 4.0)))
+        cfg = sy.hubbard_chain_configs(32, 500, 84, n_seed_configs=64)
+    psi = rng.normal(size=len(cfg)) + 0j
+    c = np.stack([c[:, 0], np.zeros(len(c))], axis=1)
+    small = lambda n: np.where(np.arange(n) % 7 == 5, 1e-315 * 10.0 ** rng.uniform(-4, 0, size=n), 0.0)  # noqa: E731
+    if of == "rows":
+        psi, c = small(len(cfg)) * np.sign(psi.real) + 0j, c * 1e160
+    else:
+        psi, c = psi * 1e160, np.sign(c) * small(len(c))[:, None]
+    ns = ops.load(cfg.shape[1], 1)
+    host = [torch.from_numpy(np.ascontiguousarray(x)) for x in (cfg, psi.view(np.float64).reshape(-1, 2), s, k, c)]
+    for k_sel in (10, 1000, 100_000):
+        want = ns.find_relative(host[0], host[1], k_sel, host[2], host[3], host[4], host[0])
+        assert len(want) > 0
+        dev = [t.to(cuda_device) for t in host]
+        got = ns.find_relative(dev[0], dev[1], k_sel, dev[2], dev[3], dev[4], dev[0]).cpu()
+        assert torch.equal(got, want), (k_sel, got.shape, want.shape)
+
+
 DIAG_CASES = [
     ("molecular-20so", 1, lambda: sorted_terms(*sy.molecular_terms(10, 1001)), lambda: sy.sector_configs(10, 5, 5, 2000, 21)),
     ("random-ops", 1, lambda: tuple(x.numpy() for x in sy.random_terms(12, 500, 22)),
