@@ -140,7 +140,7 @@ __global__ void orig_records_kernel(const int16_t* __restrict__ site, const uint
 }
 
 // ------------------------------------------------------------------------------ targets ------
-// The key words, and *occupied raised to the most occupied sites of a row.  A grid-stride pass over at
+// The key words, and *occupied (unless null) raised to the most occupied sites of a row.  A grid-stride pass over at
 // most kKeysBlocks blocks with one atomic each: with a block per 256 rows every wave in flight raised
 // the same counter (250,000 rows: 30 us, of which 25 for that).
 constexpr unsigned kKeysBlocks = 1024;
@@ -173,6 +173,9 @@ __global__ __launch_bounds__(kBlock) void keys_kernel(const uint8_t* __restrict_
             occ += __popcll(w[k]);
         }
         most = occ > most ? occ : most;
+    }
+    if (occupied == nullptr) {
+        return;  // the whole grid
     }
     for (int d = 32; d > 0; d >>= 1) {
         const int o = __shfl_xor(most, d);
@@ -534,7 +537,6 @@ size_t sort_configs_scratch_bytes(int n_words, int64_t n) {
     cv.take<uint64_t>(N);            // word in
     cv.take<uint64_t>(N);            // word out
     cv.take<uint32_t>(N);            // perm in
-    cv.take<int64_t>(1);             // most occupied row (unused)
     cv.take_bytes(sort_bytes);
     return cv.off + 256;
 }
@@ -551,15 +553,13 @@ int sort_configs(int n_qubytes, const uint8_t* configs, int64_t n, uint64_t* key
     uint64_t* win = cv.take<uint64_t>(N);
     uint64_t* wout = cv.take<uint64_t>(N);
     uint32_t* pin = cv.take<uint32_t>(N);
-    int64_t* occupied = cv.take<int64_t>(1);
     size_t sort_bytes = 0;
     (void)rocprim::radix_sort_pairs(nullptr, sort_bytes, win, wout, pin, perm, static_cast<unsigned>(N));
     void* tmp = cv.take_bytes(sort_bytes);
     if (cv.off > scratch_bytes) {
         return set_error(QMB_ERR_WORKSPACE, "sort scratch too small: need %zu, have %zu", cv.off, scratch_bytes);
     }
-    QMB_TRY(launch_fill_u64(reinterpret_cast<uint64_t*>(occupied), 0ull, 1, stream));
-    QMB_TRY(keys_dispatch(W, configs, n, n_qubytes, raw, occupied, stream));
+    QMB_TRY(keys_dispatch(W, configs, n, n_qubytes, raw, nullptr, stream));
     iota_kernel<<<blocks_for(n), kBlock, 0, stream>>>(perm, n);
     QMB_CHECK_LAUNCH();
     // LSD over words: least significant word (last) first; each pass is a stable radix sort.
