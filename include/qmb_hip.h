@@ -350,7 +350,9 @@ int qmb_cores_build(const qmb_targets* targets, int32_t max_occupied, int32_t or
 
 /* Adds the pair-excitation part of mode 0 (forward, out = A in) or mode 1 (adjoint,
  * out = A^H in) on the set of `cores`/`targets` into out (float64 [n][2]).  A gather over the
- * core groups: one FP64 atomic per (config, group) sum, none per contribution. */
+ * core groups: one FP64 atomic per (config, group) sum, none per contribution.  Repeated calls agree
+ * to rounding (the waves' sums reach a row in the order they finish), and to the last bit for an
+ * index of capacity up to 512. */
 int qmb_apply_pairs(const qmb_pairs* pairs, const qmb_cores* cores, const qmb_targets* targets, const double* in, double* out,
                     int mode, void* stream);
 

@@ -1071,12 +1071,14 @@ __global__ __launch_bounds__(kBlock) void bin_scatter_kernel(const uint32_t* __r
 
 // A small set's whole core index in one block: emission, sort, flags, starts and bins, everything
 // between in LDS.  The general build is some twenty launches of a few microseconds each, whatever the
-// size.  The limit is the LDS: 17 bytes an entry and the sort's power of two.  Entries sort by (key,
+// size.  The limit is the LDS: 18 bytes an entry and the sort's power of two.  Entries sort by (key,
 // emission index k * n + row), the order the general build's stable sort gives.
 constexpr int kSmallCores = 8192;
 // Up to this many entries one wave takes all units, in order: the sums of so small a set then come out
 // the same in every call (whole units spread over waves add to a row in the order they finish), for
-// about the time that the kernel's launch and the call around it take anyway.
+// about the time that the kernel's launch and the call around it take anyway.  Larger ones are worth
+// more than the last bit: one wave over the 52 groups that three electrons in 52 sites make takes 235 ms,
+// all waves 0.4.
 constexpr int kTinyCores = 512;
 constexpr int kSmallThreads = 1024;
 
@@ -1092,6 +1094,7 @@ struct SmallLds {
     unsigned long long rank[kBins];
     uint32_t used, over, n_mixed;
 };
+static_assert(sizeof(SmallLds) + 3 * kBins * sizeof(uint32_t) <= 160 * 1024, "LDS, with bin_table's");
 constexpr uint32_t kSmallStay = 0xffffu;
 
 template <int W, int ORDER>
@@ -1391,7 +1394,7 @@ struct PairParams {
     const double2* in2;  // second input/output of a two-vector pass (NV = 2), else null
     double2* out2;
     const int64_t* table_counts;  // qmb_pairs.counts
-    int dense;                    // the bins above 32 entries are pair_dense_kernel's
+    int dense;                    // the bins above 64 entries are pair_dense_kernel's
 };
 
 // The lanes' entries as the rows of a group read them, in this wave's LDS: the amplitude with the
@@ -1752,7 +1755,7 @@ __global__ __launch_bounds__(kBlock) void pair_kernel(PairParams p) {
     }
 }
 
-// The groups above 32 entries of a real table, eight at a time as a dense product on the matrix unit.
+// The groups above 64 entries of a real table, eight at a time as a dense product on the matrix unit.
 // A panel is eight groups that follow each other in a bin; its slots are the U pair slots that any of
 // them has, and with S the table at these slots and B the [U][16] amplitudes (eight groups, real and imaginary
 // part, zero where a group has no such entry) the panel's contributions are S^T B (ADJ: S B).  The

@@ -68,7 +68,7 @@ FR_CASES = [
     ("ising-bose2", 2, lambda: tuple(x.numpy() for x in sy.terms_from_dict(sy.ising_dict(4, 2, x=0.8, zh=1.0, zv=0.4))),
      lambda: sy.sort_unique_configs(np.random.default_rng(6).integers(0, 256, size=(60, 1), dtype=np.uint8)), 40),
     ("k-exceeds-candidates", 1, lambda: sorted_terms(*sy.molecular_terms(4, 11)), lambda: sy.sector_configs(4, 2, 2, 5, 3), 100000),
-    # at least 4096 rows and K >= 256: the sampled threshold runs first (and is checked on the device)
+    # thousands of rows: most connections stay below the first digit's bound, or tie, or are all wanted
     ("molecular-20so-sampled", 1, lambda: sorted_terms(*sy.molecular_terms(10, 1001)), lambda: sy.sector_configs(10, 5, 5, 8192, 31),
      4000),
     ("hubbard-4x2-sampled-ties", 1, lambda: tuple(x.numpy() for x in sy.terms_from_dict(sy.hubbard_dict(4, 2, 1.0, 4.0))),

@@ -427,8 +427,9 @@ def test_groups_around_the_row_tiles(cuda_device: torch.device, order: int, size
 @pytest.mark.parametrize("size,shared,finite", [(80, True, True), (80, False, True), (129, True, True), (129, False, True), (80, True, False)])
 def test_panels_of_large_groups(cuda_device: torch.device, size: int, shared: bool, finite: bool) -> None:
     """An index of over 2^25 entries takes its groups above 64 entries in panels of eight: groups of `size`
-    site pairs beside two of 36 spectators, the same pairs in each (dense products) or random ones
-    (partly walked), and the groups that the spectators make; with an infinite coefficient no panel is dense."""
+    site pairs beside two of 36 spectators, the same pairs in each or random ones (dense products over a
+    small or a large union of slots), and the groups that the spectators make; with an infinite coefficient
+    no panel is dense."""
     nq, rng = 16, np.random.default_rng(size)
     grid = [(a, b) for a in range(0, 32, 2) for b in range(1, 32, 2)]
     combos = [(s, t) for s in range(32, 68) for t in range(32, s)]
@@ -464,3 +465,114 @@ def test_panels_of_large_groups(cuda_device: torch.device, size: int, shared: bo
     plain = pp.apply(terms, targets, cfg_t, gvec, pp.MODE_ADJOINT, symmetric=pp.SYMMETRIC_OFF, pairs=False).cpu().numpy()
     got = pp.apply(terms, targets, cfg_t, gvec, pp.MODE_ADJOINT, symmetric=pp.SYMMETRIC_OFF, pairs=True).cpu().numpy()
     assert np.abs(got - plain).max() <= bound * np.abs(g).max()
+
+
+def _panel_kinds(targets: pp.PreparedTargets, most: int = 400) -> dict[str, int]:
+    """What the panels of eight groups above 64 entries of the order-2 index are: dense (at least 20 pairs of
+    entries per 16 x 16 x 4 product of the slots they use), sparse, or wide (over 960 slots); the largest
+    group under "largest".  Up to `most` panels of a size range are looked at."""
+    desc, buf = targets.cores(2), targets._cores[2][0]  # pylint: disable=protected-access
+
+    def view(pointer: int, n: int, dtype: torch.dtype) -> np.ndarray:
+        off = int(pointer) - buf.data_ptr()
+        return buf[off:off + n * dtype.itemsize].view(dtype).cpu().numpy()
+
+    bins = view(desc.bins, 3 * 39 + 40, torch.int32).astype(np.int64)
+    groups, list_base = bins[:39], bins[78:117]
+    glist = view(desc.glist, 2 * (int(list_base[38]) + int(groups[38])), torch.int32).astype(np.int64).reshape(-1, 2) & 0xFFFFFFFF
+    slots = (view(desc.mvals, int(desc.capacity), torch.int64) >> 32) & 0xFFFF
+    kinds = {"dense": 0, "sparse": 0, "wide": 0, "largest": 0, "panels": 0}
+    for which, tiles in ((33, 2), (34, 2), (35, 3), (36, 4), (37, 5)):
+        panels = -(-int(groups[which]) // (8 * tiles))
+        kinds["panels"] += panels
+        for k in range(min(panels, most)):
+            lo = int(list_base[which]) + 8 * tiles * k
+            items = glist[lo:min(lo + 8 * tiles, int(list_base[which] + groups[which]))]
+            sizes = [(int(x), int(y) & 0xFFFF) for x, y in items if y >> 16 == 0]
+            used = len(np.unique(np.concatenate([slots[x:x + n] for x, n in sizes]))) if sizes else 0
+            pairs = sum(n * n for _, n in sizes)
+            kinds["wide" if used > 960 else ("dense" if pairs >= 80 * (-(-used // 16)) ** 2 else "sparse")] += 1
+            kinds["largest"] = max([kinds["largest"], *(n for _, n in sizes)])
+    return kinds
+
+
+def _hops_and_pairs(sites: int, n_terms: int, seed: int) -> tuple[np.ndarray, np.ndarray, np.ndarray]:
+    """A real non-Hermitian table of pair excitations, hops and diagonal terms on the first `sites` sites."""
+    rng = np.random.default_rng(seed)
+    site = rng.permuted(np.tile(np.arange(sites), (n_terms, 1)), axis=1)[:, :4].astype(np.int16)
+    kind = np.tile(np.array([1, 1, 0, 0], dtype=np.uint8), (n_terms, 1))
+    u = rng.random(n_terms)
+    kind[u < 0.2] = [1, 0, 2, 2]
+    kind[u < 0.1] = [1, 0, 2, 2]
+    site[u < 0.1, 1] = site[u < 0.1, 0]
+    site[u < 0.2, 2:] = 0
+    return site, kind, np.stack([rng.normal(size=n_terms), np.zeros(n_terms)], axis=1)
+
+
+@pytest.mark.parametrize("case", ["one-word", "one-word-hard-core", "sparse", "wide", "above-256"])
+def test_panels_with_two_vectors(cuda_device: torch.device, case: str) -> None:
+    """The panels with one vector and with two, forward and adjoint, where they are dense products and where
+    they are walked (too few pairs for the slots they use, or more slots than the LDS holds): one-word
+    configs, fermions and hard-core bosons, groups up to and above 256 entries."""
+    pc = 2 if case.endswith("hard-core") else 1
+    if case.startswith("one-word"):
+        s, k, c = sorted_terms(*sy.molecular_terms(26, 5))
+        c = c * np.where(np.random.default_rng(6).random(len(c)) < 0.5, 1.0, 0.5)[:, None]  # not Hermitian
+        cfg, nq = sy.excitation_configs(26, 7, 7, 400_000, 7), 7
+    else:
+        # `size` random pairs of opposite parity on the first `of` sites beside every two of the next `spectators`, `fixed` more occupied
+        of, size, spectators, fixed = {"sparse": (60, 90, 36, 32), "wide": (80, 400, 30, 18), "above-256": (36, 300, 50, 12)}[case]
+        rng, nq = np.random.default_rng(size), 16
+        grid = np.array([(a, b) for a in range(0, of, 2) for b in range(1, of, 2)])
+        combos = [(of + x, of + y) for y in range(spectators) for x in range(y)]
+        rows = np.zeros((len(combos) * size, 8 * nq), dtype=np.uint8)
+        for j, (x, y) in enumerate(combos):
+            part = rows[j * size:(j + 1) * size]
+            part[:, [x, y]] = 1
+            picked = grid[rng.permutation(len(grid))[:size]]
+            part[np.arange(size), picked[:, 0]] = 1
+            part[np.arange(size), picked[:, 1]] = 1
+        rows[:, of + spectators:of + spectators + fixed] = 1
+        cfg = sy.sort_unique_configs(np.packbits(rows, axis=1, bitorder="little"))
+        s, k, c = _hops_and_pairs(of + spectators, 8000, 9)
+    cfg_t = _dev(cfg, cuda_device)
+    terms = pp.PreparedTerms(_dev(s, cuda_device), _dev(k, cuda_device), _dev(c, cuda_device), nq, pc)
+    targets = pp.PreparedTargets(cfg_t, nq, distinct=True)
+    assert terms.pairs_desc.real == 1 and not terms.hermitian and terms.n_residual_terms == 0
+    assert targets.cores(2).capacity >= 1 << 25
+    kinds = _panel_kinds(targets)
+    assert kinds["panels"] >= 128
+    assert kinds[{"sparse": "sparse", "wide": "wide"}.get(case, "dense")] >= 8, kinds
+    if case in ("wide", "above-256"):
+        assert kinds["largest"] > 256
+    vecs = [torch.view_as_real(_dev(sy.random_psi(len(cfg), seed), cuda_device)).contiguous() for seed in (33, 34)]
+    for mode in (pp.MODE_FORWARD, pp.MODE_ADJOINT):
+        plain = [pp.apply(terms, targets, cfg_t, v, mode, symmetric=pp.SYMMETRIC_OFF, pairs=False) for v in vecs]
+        one = pp.apply(terms, targets, cfg_t, vecs[0], mode, symmetric=pp.SYMMETRIC_OFF, pairs=True)
+        both = pp.apply_dual(terms, targets, *vecs, mode)
+        for got, want, v in ((one, plain[0], vecs[0]), (both[0], plain[0], vecs[0]), (both[1], plain[1], vecs[1])):
+            # rows meet at most a few thousand of the terms: the rounding of their sums against the largest products
+            assert (got - want).abs().max().item() <= 1e-12 * np.abs(c).sum() * v.abs().max().item()
+
+
+@pytest.mark.parametrize("bits", [0, 4])
+@pytest.mark.parametrize("n_orb,electrons,n", [(4, 2, 36), (6, 2, 85), (10, 5, 11)])
+def test_small_indexes_repeat_to_the_last_bit(cuda_device: torch.device, n_orb: int, electrons: int, n: int, bits: int) -> None:
+    """An index of up to 512 entries (36 rows of 4 electrons: 216; 85: 510; 11 of 10: 495) is walked by one
+    wave in a fixed order: fresh indexes and repeated applications agree to the last bit, in both modes,
+    with the set's hash and with 4-bit hash columns (groups of many cores)."""
+    s, k, c = sorted_terms(*sy.molecular_terms(n_orb, 41))
+    cfg = sy.sector_configs(n_orb, electrons, electrons, n, 42)
+    cfg_t = _dev(cfg, cuda_device)
+    terms = pp.PreparedTerms(_dev(s, cuda_device), _dev(k, cuda_device), _dev(c, cuda_device), cfg.shape[1], 1)
+    vec = torch.view_as_real(_dev(sy.random_psi(n, 43), cuda_device)).contiguous()
+    first = {}
+    for _ in range(8):
+        targets = pp.PreparedTargets(cfg_t, cfg.shape[1], distinct=True)
+        if bits:
+            _build_cores_with_narrow_hash(targets, bits, 44)
+        assert targets.cores(2).capacity <= 512
+        for _again in range(3):
+            for mode in (pp.MODE_FORWARD, pp.MODE_ADJOINT):
+                got = pp.apply(terms, targets, cfg_t, vec, mode, symmetric=pp.SYMMETRIC_OFF, pairs=True).view(torch.int64)
+                assert torch.equal(got, first.setdefault(mode, got))
