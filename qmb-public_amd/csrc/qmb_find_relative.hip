@@ -28,6 +28,8 @@
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 
+#include <utility>
+
 #include "qmb_enum.hpp"
 
 namespace qmb {
@@ -502,14 +504,21 @@ struct FrExponents {
     unsigned long long most;
 };
 
-__global__ __launch_bounds__(256) void fr_exponents_kernel(const double2* __restrict__ v, int64_t n, FrExponents* __restrict__ exps) {
+// Of the rows (exps[0], the first row_blocks blocks) and of the terms (exps[1], the others).
+__global__ __launch_bounds__(256) void fr_exponents_kernel(const double2* __restrict__ psi, int64_t n_rows, unsigned row_blocks,
+                                                           const double2* __restrict__ coefs, int64_t n_terms, FrExponents* __restrict__ exps) {
     __shared__ uint32_t s_exp[2048];
     unsigned long long most = 0ull;
+    const bool rows = blockIdx.x < row_blocks;
+    const double2* v = rows ? psi : coefs;
+    const int64_t n = rows ? n_rows : n_terms;
+    const int64_t block = rows ? blockIdx.x : blockIdx.x - row_blocks, blocks = rows ? row_blocks : gridDim.x - row_blocks;
+    exps += rows ? 0 : 1;
     for (int b = threadIdx.x; b < 2048; b += 256) {
         s_exp[b] = 0u;
     }
     __syncthreads();
-    for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += gridDim.x * 256ll) {
+    for (int64_t i = block * 256 + threadIdx.x; i < n; i += blocks * 256) {
         const unsigned long long a = static_cast<unsigned long long>(__double_as_longlong(hypot(v[i].x, v[i].y)));
         atomicAdd(&s_exp[(a >> 52) & 0x7ffu], 1u);
         most = a > most ? a : most;
@@ -935,7 +944,7 @@ FrScratch fr_layout(Carver& cv, int W, int n_qubytes, int64_t n_i, int64_t k, in
     return s;
 }
 
-// Sorts perm (an index permutation over n entries) stably by config words ascending.
+// Sorts perm_a (an index permutation over n entries) stably by config words ascending; perm_b is free.
 template <int W>
 int sort_by_config(const uint64_t* words, int64_t n, FrScratch& s, hipStream_t stream) {
     for (int w = W - 1; w >= 0; --w) {
@@ -944,7 +953,7 @@ int sort_by_config(const uint64_t* words, int64_t n, FrScratch& s, hipStream_t s
         size_t need = s.tmp_bytes;
         QMB_HIP_TRY(rocprim::radix_sort_pairs(s.tmp, need, s.key_a, s.key_b, s.perm_a, s.perm_b, static_cast<unsigned>(n), 0, 64,
                                               stream));
-        QMB_HIP_TRY(hipMemcpyAsync(s.perm_a, s.perm_b, static_cast<size_t>(n) * sizeof(uint32_t), hipMemcpyDeviceToDevice, stream));
+        std::swap(s.perm_a, s.perm_b);
     }
     return QMB_OK;
 }
@@ -1023,9 +1032,9 @@ int find_relative_impl(const qmb_terms* terms, const qmb_targets* exclude, const
                                               static_cast<unsigned>(bits), stream));
         fr_term_gather_kernel<<<blocks_for(T), 256, 0, stream>>>(s.term_b, terms->recs, coefs, T, s.recs, s.coefs, s.aw);
         QMB_CHECK_LAUNCH();
-        fr_exponents_kernel<<<blocks_for(n_i) < 512u ? blocks_for(n_i) : 512u, 256, 0, stream>>>(psi, n_i, s.exps);
-        QMB_CHECK_LAUNCH();
-        fr_exponents_kernel<<<blocks_for(T) < 512u ? blocks_for(T) : 512u, 256, 0, stream>>>(coefs, T, s.exps + 1);
+        const unsigned row_blocks = blocks_for(n_i) < 512u ? blocks_for(n_i) : 512u;
+        const unsigned term_blocks = blocks_for(T) < 512u ? blocks_for(T) : 512u;
+        fr_exponents_kernel<<<row_blocks + term_blocks, 256, 0, stream>>>(psi, n_i, row_blocks, coefs, T, s.exps);
         QMB_CHECK_LAUNCH();
         fr_plan_kernel<<<1, 1024, 0, stream>>>(s.state, s.psi, n_i, s.exps, k);
         QMB_CHECK_LAUNCH();
