@@ -122,37 +122,35 @@ def read_traffic(workload: str, kernel: str) -> tuple[float | None, float | None
 def structured_model(pp: object, terms: object, targets: object, nq: int, n: int) -> dict[str, object]:
     """Bytes the structured application must move at least once (synchronises to size the core
     indexes).  Per kernel launch:
-      pair_kernel:   4 per group (its start) + per group of >= 2 entries its first entry's config
-                     words (8 W: every row of a group of one core has that core) + per entry of such a
-                     group: the entry (8, row and removed sites) and its row's amplitude (16); the
-                     coefficient table once (8 or 16 per entry of n_pairs^2); the output once (16 per
-                     row);
-      single_kernel: the same over the order-1 index, with the single-excitation tables (n_bits^2 +
-                     n_bits^3 entries) once;
+      pair_kernel (with pair_dense_kernel, which takes the groups above 64 entries of a large index): per
+                     entry of a group of >= 2 entries the binned entry (8, row, slot and sign) and its
+                     row's amplitude (16); the coefficient table once (8 or 16 per entry of n_pairs^2);
+                     the output once (16 per row);
+      single_kernel: the same over the order-1 index, and per group of >= 2 entries its first entry's
+                     config words (8 W), with the single-excitation tables (n_bits^2 + n_bits^3 entries)
+                     once;
       diag_apply:    per row its config words, amplitude and output (8 W + 32); the folded table once.
     Per core index build (packed entries): every entry emitted (8 written), sorted once (8 read + 8
-    written), split and flagged (8 read; 4 key + 8 value + 4 flag written; the config words of each
-    entry of a group of >= 2 entries read, 8 W), its flag read again for the starts (4), and 4 per
-    group start -- the sort's extra passes, the per-chunk head counts and the hash index are not
-    counted."""
+    written), split and flagged (8 read; 4 key + 8 value + 1 flag written; the config words of each
+    entry of a group of >= 2 entries read, 8 W), its flag read again for the starts (1); binned (its
+    value and flag read, 9; in a group of >= 2 entries the binned entry written, 8); and per group its
+    start written, counted and placed (12) -- the sort's extra passes, the counters and the hash index
+    are not counted."""
     words = (nq + 7) // 8
     out: dict[str, object] = {}
     coef_b = 8 if terms.pairs_desc.real else 16
     n_bits = 8 * nq
 
-    def walk(st: dict[str, int]) -> int:
-        return 4 * st["groups"] + 8 * words * st["multi_groups"] + 24 * st["multi_entries"]
-
     def build(st: dict[str, int]) -> int:
-        return 52 * st["entries"] + 8 * words * st["multi_entries"] + 4 * st["groups"]
+        return 55 * st["entries"] + (8 * words + 8) * st["multi_entries"] + 12 * st["groups"]
 
     st2 = pp.core_stats(targets, 2)
-    out["pair_kernel"] = dict(st2, bytes=walk(st2) + coef_b * terms.pairs_desc.n_pairs ** 2 + 16 * n)
+    out["pair_kernel"] = dict(st2, bytes=24 * st2["multi_entries"] + coef_b * terms.pairs_desc.n_pairs ** 2 + 16 * n)
     index_bytes = build(st2)
     if terms.singles_desc is not None:
         st1 = pp.core_stats(targets, 1)
         sb = 8 if terms.singles_desc.real else 16
-        out["single_kernel"] = dict(st1, bytes=walk(st1) + sb * (n_bits ** 2 + n_bits ** 3) + 16 * n)
+        out["single_kernel"] = dict(st1, bytes=24 * st1["multi_entries"] + 8 * words * st1["multi_groups"] + sb * (n_bits ** 2 + n_bits ** 3) + 16 * n)
         index_bytes += build(st1)
     out["diag_apply_kernel"] = {"bytes": n * (8 * words + 32) + 16 * (1 + n_bits + terms.pairs_desc.n_pairs)}
     out["core_index_build"] = {"bytes": index_bytes}
@@ -783,7 +781,7 @@ def run_vmc(args: argparse.Namespace, dev: object) -> int:
         "vmc": dict(parts, setup_ms=setup_ms, energies=energies, h_forward_ms=forward_ms, generate_unique_ms=sampler_ms,
                     h_elements_per_s=2 * m_hit / (parts["energy_forward_backward_ms"] * 1e-3)),
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBPS,
-                     "traffic": None, "kernel": "H forward (pair_kernel<W=2> + single_kernel<W=2> + diagonal)", "kernel_ms": forward_ms,
+                     "traffic": None, "kernel": "H forward (pair, single and diagonal kernels)", "kernel_ms": forward_ms,
                      "algorithmic_bytes": algo_bytes,
                      "model": "structured path, bytes moved at least once per application (pair, single and diagonal kernels)",
                      "model_parts": model,
@@ -1092,11 +1090,14 @@ def main() -> int:
         model = structured_model(pp, terms, targets, nq, n)
         kname = "pair_kernel"
         k_bytes, k_ms = model["pair_kernel"]["bytes"], parts["pair_kernel_ms"]
-        label = f"pair_kernel<{(nq + 7) // 8}, {'true' if pmode == pp.MODE_ADJOINT else 'false'}, 1>"
+        orientation, real = str(pmode == pp.MODE_ADJOINT).lower(), bool(terms.pairs_desc.real)
+        label = f"pair_kernel<{orientation}, {str(real).lower()}, 1>"
+        if real and targets.cores(2).capacity >= pp.DENSE_MIN_ENTRIES:
+            label = f"pair_dense_kernel<{orientation}, 1> + {label}"  # one timed call launches both
         app_bytes = sum(v["bytes"] for k, v in model.items() if k != "core_index_build")
         step_bytes = model["core_index_build"]["bytes"] + 2 * app_bytes
-        model_desc = ("structured path, bytes moved at least once per launch: group starts, one config per group of >= 2 "
-                      "entries, the entries of those groups with their rows' amplitudes, the coefficient table, the output")
+        model_desc = ("structured path, bytes moved at least once per launch: the binned entries of groups of >= 2 entries with "
+                      "their rows' amplitudes, the coefficient table, the output")
     elif use_hops:
         model = hop_model(terms, targets, nq, n)
         kname = "hop_kernel"

@@ -31,6 +31,8 @@ EXCLUDE_PAIRS = 1
 EXCLUDE_SINGLES = 2
 EXCLUDE_DIAGONAL = 4
 EXCLUDE_HOPS = 8
+# core index entries from which the groups above 64 entries of a real table go to pair_dense_kernel (kDenseMin)
+DENSE_MIN_ENTRIES = 1 << 25
 # The hop path tests the row pairs of each strings group; it is taken while those tests stay within
 # this many per (row, hop term) -- the enumeration's work per row is a few lookups per hop term.
 HOP_PAIRS_PER_TERM_ROW = 4

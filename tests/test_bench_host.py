@@ -40,13 +40,13 @@ def test_structured_model_terms(bench: types.ModuleType, nq: int, real: bool) ->
     coef = 8 if real else 16
     n_bits = 8 * nq
     out = bench.structured_model(pp, terms, None, nq, n)
-    # per launch: starts, one config per group of >= 2 entries, entry + amplitude per walked entry,
-    # the table once, the output once
-    assert out["pair_kernel"]["bytes"] == 4 * 355 + 8 * words * 125 + 24 * 680 + coef * n_pairs ** 2 + 16 * n
-    assert out["single_kernel"]["bytes"] == 4 * 93 + 8 * words * 20 + 24 * 66 + coef * (n_bits ** 2 + n_bits ** 3) + 16 * n
+    # per launch: entry + amplitude per entry of a group of >= 2, the table once, the output once; the single
+    # kernel one config per such group
+    assert out["pair_kernel"]["bytes"] == 24 * 680 + coef * n_pairs ** 2 + 16 * n
+    assert out["single_kernel"]["bytes"] == 8 * words * 20 + 24 * 66 + coef * (n_bits ** 2 + n_bits ** 3) + 16 * n
     assert out["diag_apply_kernel"]["bytes"] == n * (8 * words + 32) + 16 * (1 + n_bits + n_pairs)
-    # per build: 52 per entry, a config per entry of a group of >= 2, a start per group
-    assert out["core_index_build"]["bytes"] == sum(52 * s["entries"] + 8 * words * s["multi_entries"] + 4 * s["groups"]
+    # per build: 55 per entry, a config and a binned entry per entry of a group of >= 2, three passes over the starts
+    assert out["core_index_build"]["bytes"] == sum(55 * s["entries"] + (8 * words + 8) * s["multi_entries"] + 12 * s["groups"]
                                                    for s in st.values())
     assert out["pair_kernel"]["multi_groups"] == 125
 
