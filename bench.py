@@ -427,9 +427,9 @@ def run_batch(args: argparse.Namespace, dev: object) -> int:
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBPS,
                      "traffic": None, "kernel": "batch_kernel<adjoint, one vector> (one direction, all instances)", "kernel_ms": fwd_only,
                      "algorithmic_bytes": model_bytes,
-                     "model": "structured path, bytes moved at least once: group starts, one config per group of >= 2 entries, "
-                              "the entries of those groups with their rows' amplitudes, the coefficient tables, the outputs "
-                              "(summed over the instances)",
+                     "model": "structured path, bytes moved at least once: the binned entries of groups of >= 2 entries with "
+                              "their rows' amplitudes, a config per group of the single kernel, the coefficient tables, the "
+                              "outputs (summed over the instances)",
                      "lookup_model": {"what": "one key read per generated connection (the enumeration path's bound, not this path's)",
                                       "bytes": algo_bytes, "gbps_equivalent": algo_bytes / (fwd_only * 1e-3) / 1e9}},
         "batch": {"batched_graph_ms": graph_batch, "batched_eager_ms": eager_batch, "batched_two_launches_ms": two_launches,
