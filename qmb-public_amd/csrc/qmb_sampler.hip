@@ -269,6 +269,7 @@ constexpr int kFusedWaves = 16;
 constexpr int kFusedThreads = 64 * kFusedWaves;
 constexpr int kFusedTile = 16;     // rows whose outputs reach their lanes together
 constexpr int kFusedMaxTiles = 4;  // of a wave: a lane holds one row
+constexpr int64_t kFewRows = 12;   // a call of so few leaves rows of its one tile out, see site_rows
 
 __device__ __forceinline__ uint64_t wave_read64(uint64_t v, int lane) {
     const uint32_t lo = __builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(v)), lane);
@@ -334,9 +335,8 @@ __device__ __forceinline__ void stage_site(const SiteLds& s, const float* w1, in
     constexpr int H = 64 * HPL;
     constexpr int V = UnitVec<HPL>::V;
     for (int t = threadIdx.x; t < k_rows * H; t += blockDim.x) {
-        // consecutive LDS words: the other way round four lanes meet in a bank
-        const int u = t % (64 * V);
-        s.w1[t] = w1[t - u + u % V * 64 + u / V];
+        const int u = t % H;
+        s.w1[t - u + u / (64 * V) * (64 * V) + u % 64 * V + u / 64 % V] = w1[t];
     }
     for (int t = threadIdx.x; t < H; t += blockDim.x) {
         s.b1[t] = b1[t];
@@ -444,24 +444,27 @@ __device__ __forceinline__ void cut_bits(uint64_t& s0, uint64_t& s1, int n_bits)
 }
 
 // The outputs of a staged site network on the wave's rows (rows_here of them, lane = row, bits b0/b1).
-template <int HPL>
+// FEW: rows past rows_here do no work.  For calls of up to kFewRows rows, where the empty ones would be
+// much of the time (26 sites of width 512: one row 291 -> 163 us, four 341 -> 238; width 256: 181 -> 123,
+// 225 -> 160).  Larger calls compute the rows that a tile lacks as empty ones, beside waves that have whole
+// tiles: the tests cost 15 rows of width 64 5%, 1M rows of width 512 1%.
+template <int HPL, bool FEW>
 __device__ __forceinline__ void site_rows(const SiteLds& s, int n_out, int k_rows, int rows_here, uint64_t b0, uint64_t b1, int lane,
                                           float (&mine)[4]) {
     const SiteRegs<HPL> g = site_regs<HPL>(s, n_out, lane);
     const int from = 16 * ((lane & 15) >> 2) + 4 * (lane & 3);  // the lanes that receive a row's outputs
-    const auto tile = [&](auto whole, int t) {
-        constexpr bool kWhole = decltype(whole)::value;
+    for (int t = 0; kFusedTile * t < rows_here; ++t) {
         float out = 0.f;
         for (int q = 0; q < 4; ++q) {
-            const int r0 = kFusedTile * t + 4 * q;
-            if (!kWhole && r0 >= rows_here) {
+            if (FEW && kFusedTile * t + 4 * q >= rows_here) {
                 break;
             }
             float part[4][4];
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                if (kWhole || r0 + v < rows_here) {
-                    uint64_t s0 = wave_read64(b0, r0 + v), s1 = wave_read64(b1, r0 + v);
+                const int r = kFusedTile * t + 4 * q + v;
+                if (!FEW || r < rows_here) {
+                    uint64_t s0 = wave_read64(b0, r), s1 = wave_read64(b1, r);
                     cut_bits(s0, s1, k_rows);
                     site_row<HPL>(s, g, s0, s1, lane, part[v]);
                 } else {
@@ -469,29 +472,20 @@ __device__ __forceinline__ void site_rows(const SiteLds& s, int n_out, int k_row
                 }
             }
             const float sum = row_sums(part, lane);
-            const float s0 = __shfl(sum, lane & 15), s1 = __shfl(sum, 16 + (lane & 15));
-            const float s2 = __shfl(sum, 32 + (lane & 15)), s3 = __shfl(sum, 48 + (lane & 15));
-            out = lane >> 4 == q ? ((s0 + s1) + s2) + s3 : out;
+            const float r0 = __shfl(sum, lane & 15), r1 = __shfl(sum, 16 + (lane & 15));
+            const float r2 = __shfl(sum, 32 + (lane & 15)), r3 = __shfl(sum, 48 + (lane & 15));
+            out = lane >> 4 == q ? ((r0 + r1) + r2) + r3 : out;
         }
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             const float v = __shfl(out, from + c);
             mine[c] = lane >> 4 == t ? v + g.b2[c] : mine[c];
         }
-    };
-    // A tile that the rows do not fill does no work for those it lacks (one row through 26 sites of width
-    // 512: 290 -> 153 us); in its own copy, since the tests cost 1M rows 1%.
-    int t = 0;
-    for (; kFusedTile * (t + 1) <= rows_here; ++t) {
-        tile(std::true_type{}, t);
-    }
-    if (kFusedTile * t < rows_here) {
-        tile(std::false_type{}, t);
     }
 }
 
 // Forward of the whole network: log-amplitude (double) and phase per config.
-template <int HPL>
+template <int HPL, bool FEW>
 __global__ void __launch_bounds__(kFusedThreads)
     network_fused_kernel(int64_t n, int tiles, int n_sites, int spin_up, int spin_down, const uint8_t* __restrict__ configs, int n_qubytes,
                          const int64_t* __restrict__ ordering_reversed, const float* __restrict__ w1, const float* __restrict__ b1,
@@ -543,7 +537,7 @@ __global__ void __launch_bounds__(kFusedThreads)
         }
         __syncthreads();
         float mine[4] = {0.f, 0.f, 0.f, 0.f};
-        site_rows<HPL>(s, n_out, k_rows, rows_here, b0, b1w, lane, mine);
+        site_rows<HPL, FEW>(s, n_out, k_rows, rows_here, b0, b1w, lane, mine);
         if (!valid) {
             continue;
         }
@@ -569,7 +563,7 @@ __global__ void __launch_bounds__(kFusedThreads)
 
 // One sampling step at `site` with the site network fused in: children log-probabilities and
 // Gumbel-perturbed values, as children_kernel computes them from given logits.
-template <int HPL>
+template <int HPL, bool FEW>
 __global__ void __launch_bounds__(kFusedThreads)
     sampler_fused_kernel(int64_t n, int tiles, int site, int n_sites, int spin_up, int spin_down, const uint64_t* __restrict__ prefix, int words,
                          const float* __restrict__ w1, const float* __restrict__ b1, const float* __restrict__ w2,
@@ -594,7 +588,7 @@ __global__ void __launch_bounds__(kFusedThreads)
                     w2 + static_cast<size_t>(site) * 4 * H, b2 + 4 * site, 4);
     __syncthreads();
     float mine[4] = {0.f, 0.f, 0.f, 0.f};
-    site_rows<HPL>(s, 4, 2 * site, rows_here, b0, b1w, lane, mine);
+    site_rows<HPL, FEW>(s, 4, 2 * site, rows_here, b0, b1w, lane, mine);
     if (!valid) {
         return;
     }
@@ -713,10 +707,10 @@ int network_forward_fused(int64_t n, int n_sites, int hidden, int spin_up, int s
     const unsigned grid = fused_grid(n, &tiles);
     return by_hidden(hidden, [&](auto hc) -> int {
         constexpr int HPL = decltype(hc)::value;
-        QMB_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&network_fused_kernel<HPL>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        static_cast<int>(lds)));
-        network_fused_kernel<HPL><<<grid, kFusedThreads, lds, stream>>>(n, tiles, n_sites, spin_up, spin_down, configs, n_qubytes, ordering_reversed,
-                                                                       w1, b1, w2, b2, wp1, bp1, wp2, bp2, amplitude, phase);
+        const auto kernel = n <= kFewRows ? &network_fused_kernel<HPL, true> : &network_fused_kernel<HPL, false>;
+        QMB_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+        kernel<<<grid, kFusedThreads, lds, stream>>>(n, tiles, n_sites, spin_up, spin_down, configs, n_qubytes, ordering_reversed, w1, b1, w2,
+                                                     b2, wp1, bp1, wp2, bp2, amplitude, phase);
         QMB_CHECK_LAUNCH();
         return QMB_OK;
     });
@@ -744,11 +738,11 @@ int sampler_step_fused(int64_t n, int site, int n_sites, int hidden, int spin_up
     const unsigned grid = fused_grid(n, &tiles);
     return by_hidden(hidden, [&](auto hc) -> int {
         constexpr int HPL = decltype(hc)::value;
-        QMB_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&sampler_fused_kernel<HPL>), hipFuncAttributeMaxDynamicSharedMemorySize,
+        const auto kernel = n <= kFewRows ? &sampler_fused_kernel<HPL, true> : &sampler_fused_kernel<HPL, false>;
+        QMB_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                         static_cast<int>(fused_lds_bytes(2 * n_sites, hidden))));
-        sampler_fused_kernel<HPL><<<grid, kFusedThreads, lds, stream>>>(n, tiles, site, n_sites, spin_up, spin_down, prefix, words, w1, b1, w2, b2,
-                                                                       unperturbed, perturbed, uniform, seed, child_unperturbed,
-                                                                       child_perturbed);
+        kernel<<<grid, kFusedThreads, lds, stream>>>(n, tiles, site, n_sites, spin_up, spin_down, prefix, words, w1, b1, w2, b2, unperturbed,
+                                                     perturbed, uniform, seed, child_unperturbed, child_perturbed);
         QMB_CHECK_LAUNCH();
         return QMB_OK;
     });

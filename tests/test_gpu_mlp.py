@@ -283,3 +283,28 @@ def test_fused_rows_are_independent_of_the_launch(cuda_device: torch.device, sit
         assert torch.equal(got[unset], want[unset])
         if sites > 1:
             assert bool(unset.any())
+
+
+@pytest.mark.parametrize("sites,hidden", [(1, 64), (7, 128), (26, 256), (26, 512), (37, 512)])
+def test_few_fused_rows_are_those_of_a_larger_call(cuda_device: torch.device, sites: int, hidden: int) -> None:
+    """Calls of 1 to 17 rows (up to 12 leave the rows that a tile lacks out) give each row the bits that it
+    has among 300, and so does a unique draw, which begins with one row and grows."""
+    up, down = (sites + 1) // 2, sites // 2
+    net = _net(sites, up, down, (hidden,), 1, torch.float32, cuda_device, seed=hidden + sites)
+    rng = np.random.default_rng(sites)
+    bits = np.zeros((300, sites, 2), dtype=np.uint8)
+    for spin, count in ((0, up), (1, down)):
+        bits[:, :, spin] = rng.random((300, sites)).argsort(axis=1).argsort(axis=1) < count
+    x = torch.from_numpy(np.packbits(bits.reshape(300, 2 * sites), axis=1, bitorder="little")).to(cuda_device)
+    with torch.no_grad():
+        for p in net.parameters():
+            p.mul_(0.3)
+        assert net._fused_ok()  # pylint: disable=protected-access
+        want = torch.view_as_real(net(x)).view(torch.int64)
+        for rows in range(1, 18):
+            for lo in (0, 283 - rows):
+                got = torch.view_as_real(net(x[lo:lo + rows])).view(torch.int64)
+                assert torch.equal(got, want[lo:lo + rows]), (rows, lo)
+        drawn = [net.generate_unique(n, seed=3)[0] for n in (1, 5, 12, 13, 40)]
+        again = [net.generate_unique(n, seed=3)[0] for n in (1, 5, 12, 13, 40)]
+        assert all(torch.equal(a, b) for a, b in zip(drawn, again))
