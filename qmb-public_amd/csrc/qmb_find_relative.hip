@@ -114,12 +114,15 @@ struct FrParams {
     int direct;
 };
 
-// |sign * coef * psi|^2 with every product and sum rounded separately (no contraction), so the
-// bits match a plain IEEE evaluation of the reference expression (qmb/_hamiltonian_cpu.cpp:388-392).
+// |sign * coef * psi|^2 with every product and sum rounded separately, so the bits match a plain IEEE
+// evaluation of the reference expression (qmb/_hamiltonian_cpu.cpp:388-392) and are the same in every
+// kernel: the passes compare the weights that others counted for equality.  (__dmul_rn and __dadd_rn are
+// ordinary operators here, which the compiler fuses, each kernel in its own way, unless told not to.)
 __device__ __forceinline__ uint64_t weight_bits(const double2 cf, const double2 v) {
-    const double re = __dsub_rn(__dmul_rn(cf.x, v.x), __dmul_rn(cf.y, v.y));
-    const double im = __dadd_rn(__dmul_rn(cf.x, v.y), __dmul_rn(cf.y, v.x));
-    const double w = __dadd_rn(__dmul_rn(re, re), __dmul_rn(im, im));
+#pragma clang fp contract(off)
+    const double re = cf.x * v.x - cf.y * v.y;
+    const double im = cf.x * v.y + cf.y * v.x;
+    const double w = re * re + im * im;
     return static_cast<uint64_t>(__double_as_longlong(w));
 }
 

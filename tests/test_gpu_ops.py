@@ -181,6 +181,28 @@ def test_find_relative_takes_exact_ties_by_config(cuda_device: torch.device, nam
         assert torch.equal(got, want), (got.shape, want.shape)
 
 
+@pytest.mark.parametrize("sites,n_terms", [(20, 3000), (20, 6000), (70, 3000), (70, 6000)])
+def test_find_relative_weighs_without_contraction(cuda_device: torch.device, sites: int, n_terms: int) -> None:
+    """Complex coefficients of a few sizes: |coef psi_i|^2 of a row then takes values that are equal but for
+    the rounding of their products, and the choice among them depends on the last bit of every weight: each
+    product and sum is rounded by itself, as the host operator's.  Both enumerations, one and two words."""
+    rng = np.random.default_rng(sites + n_terms)
+    s, k, c = (x.numpy() for x in sy.random_terms(sites, n_terms, 85))
+    c = np.round(c * 2) / 2
+    nq = (sites + 7) // 8
+    bits = np.zeros((2000, 8 * nq), dtype=np.uint8)
+    bits[:, :sites] = rng.random((2000, sites)) < 0.5
+    cfg = sy.sort_unique_configs(np.packbits(bits, axis=1, bitorder="little"))
+    psi = np.repeat(rng.normal(size=40) + 1j * rng.normal(size=40), 50)[: len(cfg)]
+    ns = ops.load(nq, 1)
+    host = [torch.from_numpy(np.ascontiguousarray(x)) for x in (cfg, psi.view(np.float64).reshape(-1, 2), s, k, c)]
+    dev = [t.to(cuda_device) for t in host]
+    for k_sel in (10, 300, 3000, 30_000):
+        want = ns.find_relative(host[0], host[1], k_sel, host[2], host[3], host[4], host[0])
+        got = ns.find_relative(dev[0], dev[1], k_sel, dev[2], dev[3], dev[4], dev[0]).cpu()
+        assert torch.equal(got, want), (k_sel, got.shape, want.shape)
+
+
 @pytest.mark.parametrize("of", ["rows", "terms"])
 @pytest.mark.parametrize("name", ["molecular", "hubbard"])
 def test_find_relative_with_denormal_factors(cuda_device: torch.device, name: str, of: str) -> None:
